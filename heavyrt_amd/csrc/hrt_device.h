@@ -29,6 +29,9 @@ constexpr uint32_t kEmptyLeaf = 0x80000000u;  // PackOffsetAndSize(0, 0): a leaf
 // Deepest possible BLAS path: the Karras tree over unique 30-bit codes has at
 // most 30 internal levels, so at most 30 deferred children are ever pending.
 constexpr int kStackDepth = 32;
+// The walks of walk2.h keep one entry below those (kInvalid, which ends the
+// walk when it is popped) and may store a node that does not count above them.
+constexpr int kWalkDepth = kStackDepth + 2;
 
 __host__ __device__ inline uint32_t pack_leaf(uint32_t start, uint32_t count) {
   return kLeafBit | ((count << 24) & kSizeMask) | (start & kStartMask);
@@ -49,6 +52,17 @@ struct __attribute__((aligned(64))) NodePair {
   float4 lmax;  // xyz = left child box max,  w = unused (0)
   float4 rmin;  // xyz = right child box min, w = bits of right child ref
   float4 rmax;  // xyz = right child box max, w = unused (0)
+};
+
+// Two levels of the BVH2 below one internal node, 128 bytes, for the
+// nearest-hit walks (walk2.h): the boxes and references of its four
+// grandchildren, 32 bytes each ({lo.xyz, reference}, {hi.xyz, child}), where
+// `child` is the reference of the child the grandchild belongs to (the walk
+// defers a farther child as such).  A child that is a leaf takes its first
+// slot, with the second one a copy whose reference is kInvalid.  Node k's is
+// at index k.
+struct __attribute__((aligned(128))) WideNode {
+  float4 g[8];
 };
 
 // Triangle in leaf order, 48 bytes: vertex A, the edges B-A and C-A as the
@@ -88,6 +102,18 @@ struct ShortStack {
     if (top < kLds) return lds[top * kStride];
     return spill[size_t(top - kLds) * spill_stride];
   }
+  // The walks of walk2.h: peek reads entry top - 1 (top > 0) ahead of need as
+  // far as it lies in the LDS part, and pop_peeked gives the entry itself; put
+  // sets entry `top` to v when `keep` (without it the slot, which holds
+  // nothing, may be written or not).  None of them moves top.
+  __device__ inline uint32_t peek(int top) const { return lds[(top <= kLds ? top - 1 : 0) * kStride]; }
+  __device__ inline uint32_t pop_peeked(int top, uint32_t peeked) const {
+    return top <= kLds ? peeked : spill[size_t(top - 1 - kLds) * spill_stride];
+  }
+  __device__ inline void put(int top, uint32_t v, bool keep) const {
+    if (top < kLds) lds[top * kStride] = v;
+    else if (keep) spill[size_t(top - kLds) * spill_stride] = v;
+  }
   // Pushes c3 if p3, then c2 if p2, then c1 if p1.  With room for three more
   // entries in the LDS part, each value is stored at the top slot whether or
   // not it is pushed (a slot at or above top holds nothing), so there is no
@@ -107,6 +133,15 @@ struct ShortStack {
       if (p1) push(top, c1);
     }
   }
+};
+// The stack of a walk that cannot get deeper than its LDS part.
+template <int kStride>
+struct LdsStack {
+  lds_u32* lds;
+  __device__ explicit LdsStack(uint32_t* lds_generic) : lds((lds_u32*)(lds_generic)) {}
+  __device__ inline uint32_t peek(int top) const { return lds[(top - 1) * kStride]; }
+  __device__ inline uint32_t pop_peeked(int, uint32_t peeked) const { return peeked; }
+  __device__ inline void put(int top, uint32_t v, bool) const { lds[top * kStride] = v; }
 };
 constexpr int kShortStack = 16;  // LDS entries per lane in the persistent kernels
 

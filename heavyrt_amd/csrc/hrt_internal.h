@@ -66,6 +66,11 @@ struct Blas {
   uint32_t nquads = 0;
   Quad32* quads32 = nullptr;
   Quad16* quads16 = nullptr;
+  // two levels per internal node for nearest-hit walks (made on demand by
+  // blas_build_wide); the word after the last node is not zero where a walk on
+  // them could differ from one on the pairs
+  WideNode* wide = nullptr;
+  bool wide_made = false;  // blas_build_wide has run on the tree as it is now
   // parity hooks (kept only when requested)
   uint32_t* codes_in = nullptr;    // Morton code per input triangle
   uint32_t* codes_sorted = nullptr;
@@ -116,6 +121,22 @@ hipError_t blas_ploc(Blas& b, hipStream_t stream, bool* replaced);
 // Collapses the built BVH2 into FP32 and FP16 BVH4 nodes (idempotent);
 // synchronises the stream.
 hipError_t blas_build_bvh4(Blas& b, hipStream_t stream);
+// The WideNodes of b as the walks read them: null without them, `differ` the
+// word that sends a walk to the pairs.
+struct WalkNodes {
+  const WideNode* wide;
+  const NodePair* pairs;
+  const uint32_t* differ;
+};
+inline uint32_t internal_nodes(const Blas& b) { return b.leaves > 1 ? b.leaves - 1 : 1; }
+inline WalkNodes walk_nodes(const Blas& b) {
+  const WideNode* w = b.wide_made ? b.wide : nullptr;
+  return WalkNodes{w, b.pairs, w ? reinterpret_cast<const uint32_t*>(w + internal_nodes(b)) : nullptr};
+}
+// Makes b.wide from the node pairs (idempotent; after a refit again, in the
+// same memory).  Without memory for it b.wide stays null, which is no error.
+// Asynchronous on `stream`.
+hipError_t blas_build_wide(Blas& b, hipStream_t stream);
 // Leaf-order triangles with absolute vertices for the watertight test
 // (idempotent).  Asynchronous on `stream`.
 hipError_t blas_build_wt_tris(Blas& b, hipStream_t stream);

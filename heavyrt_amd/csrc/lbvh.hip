@@ -507,6 +507,43 @@ __global__ __launch_bounds__(kBlock) void k_collapse4(const NodePair* __restrict
   q16[q] = h;
 }
 
+// One WideNode per internal node (a one-leaf tree's pair 0 counts as one):
+// three pairs in, 128 B out.  *differ is set when a child box is not the union
+// of its own children's boxes, or one of those is inverted (a leaf of NaN
+// vertices): the walk takes a child's distances from its children's.
+__global__ __launch_bounds__(kBlock) void k_wide_nodes(const NodePair* __restrict__ pairs, uint32_t n,
+                                                       WideNode* __restrict__ out, uint32_t* __restrict__ differ) {
+  const uint32_t k = blockIdx.x * kBlock + threadIdx.x;
+  if (k >= n) return;
+  Child g[4];
+  uint32_t ref[2];
+  bool exact = true;
+  for (int side = 0; side < 2; side++) {
+    const Child c = pair_child(pairs, k, side);
+    Child &g0 = g[2 * side], &g1 = g[2 * side + 1];
+    ref[side] = c.ref;
+    if (c.ref & kLeafBit) {
+      g0 = g1 = c;
+      g1.ref = kInvalid;
+      continue;
+    }
+    g0 = pair_child(pairs, c.ref, 0);
+    g1 = pair_child(pairs, c.ref, 1);
+    exact = exact && g0.lo.x <= g0.hi.x && g0.lo.y <= g0.hi.y && g0.lo.z <= g0.hi.z && g1.lo.x <= g1.hi.x &&
+            g1.lo.y <= g1.hi.y && g1.lo.z <= g1.hi.z && c.lo.x == fminf(g0.lo.x, g1.lo.x) &&
+            c.lo.y == fminf(g0.lo.y, g1.lo.y) && c.lo.z == fminf(g0.lo.z, g1.lo.z) &&
+            c.hi.x == fmaxf(g0.hi.x, g1.hi.x) && c.hi.y == fmaxf(g0.hi.y, g1.hi.y) &&
+            c.hi.z == fmaxf(g0.hi.z, g1.hi.z);
+  }
+  if (!exact) *differ = 1u;
+  WideNode w;
+  for (int i = 0; i < 4; i++) {
+    w.g[2 * i] = make_float4(g[i].lo.x, g[i].lo.y, g[i].lo.z, __uint_as_float(g[i].ref));
+    w.g[2 * i + 1] = make_float4(g[i].hi.x, g[i].hi.y, g[i].hi.z, __uint_as_float(ref[i >> 1]));
+  }
+  out[k] = w;
+}
+
 // Leaf-order triangle j with its absolute vertices for the watertight test:
 // {A, original id}, {B, 0}, {C, 0} (the vertices exactly as stored, so
 // triangles that share a vertex see the same values).
@@ -562,7 +599,7 @@ void blas_free(Blas& b) {
     delete b.any_tree;
     b.any_tree = nullptr;
   }
-  void* ptrs[] = {b.leaf_run,   b.parent_leaf, b.node_range, b.meta,       b.tris_wt,
+  void* ptrs[] = {b.leaf_run,   b.parent_leaf, b.node_range, b.meta,       b.tris_wt, b.wide,
                   b.verts,      b.idx,        b.pairs,      b.tris,      b.perm,   b.parent,
                   b.quads32,    b.quads16,    b.codes_in,   b.codes_sorted, b.ids_sorted,
                   b.run_start,  b.ucodes,     b.karras_lr};
@@ -723,6 +760,7 @@ hipError_t blas_refit(Blas& b, hipStream_t s) {
   std::memcpy(b.box, hbox, sizeof(b.box));
   // boxes changed: the BVH4 nodes, the watertight records and the any-hit
   // tree are made again on the next commit
+  b.wide_made = false;
   if (b.tris_wt) (void)hipFree(b.tris_wt);
   b.tris_wt = nullptr;
   if (b.quads32) (void)hipFree(b.quads32);
@@ -766,6 +804,22 @@ hipError_t tlas_build(Blas& t, const InstDev* by_id, InstDev* leaf_order, hipStr
   return lbvh_build(t, src, N, s, [&](const uint32_t* ids_sorted) {
     k_inst_order<<<blocks_for(N), kBlock, 0, s>>>(by_id, ids_sorted, N, leaf_order, t.perm);
   });
+}
+
+hipError_t blas_build_wide(Blas& b, hipStream_t s) {
+  if (b.wide_made) return hipSuccess;
+  const uint32_t n = internal_nodes(b);
+  if (!b.wide && hipMalloc(&b.wide, sizeof(WideNode) * (size_t(n) + 1)) != hipSuccess) {
+    (void)hipGetLastError();  // no memory: the walks stay on the pairs
+    b.wide = nullptr;
+    return hipSuccess;
+  }
+  uint32_t* differ = reinterpret_cast<uint32_t*>(b.wide + n);
+  k_fill<<<1, kBlock, 0, s>>>(differ, sizeof(WideNode) / 4, 0u);
+  k_wide_nodes<<<blocks_for(n), kBlock, 0, s>>>(b.pairs, n, b.wide, differ);
+  HRT_CHECK(hipGetLastError());
+  b.wide_made = true;
+  return hipSuccess;
 }
 
 hipError_t blas_build_wt_tris(Blas& b, hipStream_t s) {

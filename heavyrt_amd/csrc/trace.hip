@@ -10,8 +10,9 @@
 // tFar = -w that stops at its first hit (BVH4HalfRT.cpp:260-262, 82).
 //
 // Layout: NodePair (64 B, both children of one internal node) and TriPre
-// (48 B, A / B-A / C-A / original id), both in HBM; the per-lane stack of
-// deferred children lives in LDS, 32 entries, interleaved by lane.
+// (48 B, A / B-A / C-A / original id), both in HBM, and WideNode (128 B, two
+// levels) for the four-lane walk; the stack of deferred children lives in LDS,
+// interleaved by lane or ray (walk2.h).
 //
 // Execution: a persistent wave64 kernel.  Each wave keeps 64 rays in flight;
 // when enough lanes have finished, the wave counts its idle lanes with one
@@ -33,6 +34,7 @@
 #include <vector>
 
 #include "hrt_internal.h"
+#include "walk2.h"
 
 namespace hrt {
 namespace {
@@ -44,8 +46,8 @@ constexpr int kRefillAt = 16;  // refill when at least this many lanes are idle
 constexpr uint32_t kClaim = 128;  // ray indices a wave claims from the queue at once
 // One-ray-per-lane kernel: stack entries per lane in LDS.  With 16 (16 KB
 // per 256-thread block) LDS allows 8 waves per SIMD and deeper entries, up to
-// kStackDepth, go to a per-lane global spill area; with kStackDepth nothing
-// spills but LDS allows 5 waves per SIMD.  The launcher takes the full LDS
+// kWalkDepth, go to a per-lane global spill area; with kWalkDepth nothing
+// spills but LDS allows 4 waves per SIMD.  The launcher takes the full LDS
 // stack when its whole grid is resident at once (a small batch gains nothing
 // from more waves and would pay for the spills), the short one otherwise.
 constexpr int kSimpleLds = 16;
@@ -61,8 +63,8 @@ struct HitOutFull {  // CRT_Hit (CrossRT.h:20-27)
 
 __global__ void k_reset_counter(uint32_t* c) { *c = 0u; }
 
-// Reference-order reference kernel (one ray per lane, no refill).  Kept for
-// the counting variant used to report the reference's traversal counters.
+// The reference's order, one ray per lane (no refill): nearest hits, and the
+// counting variant, whose counters are the reference's.
 template <bool kForceAny, bool kStats, int kLds, class Tri = MtTest>
 __global__ __launch_bounds__(256) void k_trace_simple(const NodePair* __restrict__ pairs,
                                                       const TriPre* __restrict__ tris,
@@ -72,7 +74,10 @@ __global__ __launch_bounds__(256) void k_trace_simple(const NodePair* __restrict
   __shared__ uint32_t stack_mem[kLds * 256];
   const uint64_t i = uint64_t(blockIdx.x) * 256 + threadIdx.x;
   if (i >= n) return;
-  const ShortStack<kLds, 256> stk{stack_mem + threadIdx.x, spill + i, gridDim.x * 256u};
+  std::conditional_t<kLds == kWalkDepth, LdsStack<256>, ShortStack<kLds, 256>> stk = [&] {
+    if constexpr (kLds == kWalkDepth) return LdsStack<256>(stack_mem + threadIdx.x);
+    else return ShortStack<kLds, 256>{stack_mem + threadIdx.x, spill + i, gridDim.x * 256u};
+  }();
   const Ray r = rays[i];
   const float3 o = make_float3(r.pos_near.x, r.pos_near.y, r.pos_near.z);
   const float3 d = make_float3(r.dir_far.x, r.dir_far.y, r.dir_far.z);
@@ -87,39 +92,19 @@ __global__ __launch_bounds__(256) void k_trace_simple(const NodePair* __restrict
   h.u = 0.0f;
   h.v = 0.0f;
   uint32_t npairs = 0, ntests = 0;
-  int top = 0;
+  int top = 1;
   uint32_t cur = 0;
-  while (true) {
-    bool pop;
-    if ((cur & kLeafBit) == 0) {
-      const float4* pp = reinterpret_cast<const float4*>(pairs + cur);
-      const float4 lmin = pp[0], lmax = pp[1], rmin = pp[2], rmax = pp[3];
-      if (kStats) npairs++;
-      const float2 t0 = tt.box(o, inv, lmin.x, lmin.y, lmin.z, lmax.x, lmax.y, lmax.z);
-      const float2 t1 = tt.box(o, inv, rmin.x, rmin.y, rmin.z, rmax.x, rmax.y, rmax.z);
-      const bool h0 = (t0.x <= t0.y) && (t0.y >= tnear) && (t0.x <= h.t);
-      const bool h1 = (t1.x <= t1.y) && (t1.y >= tnear) && (t1.x <= h.t);
-      const uint32_t c0 = __float_as_uint(lmin.w), c1 = __float_as_uint(rmin.w);
-      pop = !h0 && !h1;
-      cur = h0 ? c0 : c1;
-      if (h0 && h1) {
-        const bool left_first = t0.x <= t1.x;
-        cur = left_first ? c0 : c1;
-        stk.push(top, left_first ? c1 : c0);
-      }
-    } else {
-      pop = true;
-      if (cur != kInvalid) {
-        const uint32_t s = leaf_start(cur), c = leaf_count(cur);
-        if (kStats) ntests += c;
-        for (uint32_t k = s; k < s + c; k++) tri_test(tt, o, d, tnear, tris[k], h);
-        if (any && h.prim != kInvalid) break;
-      }
+  stk.put(0, kInvalid, true);
+  while (cur != kInvalid) {
+    if (kStats) {
+      npairs += (cur & kLeafBit) == 0;
+      ntests += (cur & kLeafBit) != 0 && leaf_count(cur) != 0;
     }
-    if (pop) {
-      if (top == 0) break;
-      cur = stk.pop(top);
-    }
+    const bool leaf_done = walk_step(pairs, tris, tt, o, d, inv, tnear, h.t, stk, top, cur,
+                                     [&h](float t, float u, float v, uint32_t prim) {
+                                       if (t < h.t) h = HitRec{t, prim, u, v};
+                                     });
+    if (any && leaf_done && h.prim != kInvalid) break;
   }
   if (kStats) {
     stats[2 * i + 0] = npairs;
@@ -128,6 +113,56 @@ __global__ __launch_bounds__(256) void k_trace_simple(const NodePair* __restrict
   if (kForceAny) {
     static_cast<uint8_t*>(out)[i] = (h.prim != kInvalid) ? 1 : 0;
   } else if (format == kHitCompact) {
+    static_cast<uint2*>(out)[i] = make_uint2(__float_as_uint(h.t), h.prim);
+  } else {
+    const bool hit = h.prim != kInvalid;
+    float4* o4 = reinterpret_cast<float4*>(static_cast<HitOutFull*>(out) + i);
+    o4[0] = make_float4(h.t, __uint_as_float(h.prim), __uint_as_float(hit ? ids.x : kInvalid),
+                        __uint_as_float(hit ? ids.y : kInvalid));
+    o4[1] = make_float4(h.u, h.v, 0.0f, 0.0f);
+  }
+}
+
+// Nearest hits in the reference's order, four lanes per ray (walk_quad_step),
+// kQuadRays rays per workgroup.  On a tree whose WideNodes may not be walked
+// the four lanes walk its pairs alike.
+constexpr uint32_t kQuadRays = 64;
+template <class Tri>
+__global__ __launch_bounds__(256) void k_trace_quad(WalkNodes nodes, const TriPre* __restrict__ tris,
+                                                    const Ray* __restrict__ rays, uint64_t n, void* out, int format,
+                                                    uint2 ids) {
+  __shared__ uint32_t stack_mem[kWalkDepth * kQuadRays];
+  const uint32_t l = threadIdx.x & 3u, q = threadIdx.x >> 2;
+  const uint64_t i = uint64_t(blockIdx.x) * kQuadRays + q;
+  if (i >= n) return;
+  const LdsStack<int(kQuadRays)> stk(stack_mem + q);
+  const Ray r = rays[i];
+  const float3 o = make_float3(r.pos_near.x, r.pos_near.y, r.pos_near.z);
+  const float3 d = make_float3(r.dir_far.x, r.dir_far.y, r.dir_far.z);
+  const float tnear = r.pos_near.w;
+  const bool any = r.dir_far.w <= 0.0f;
+  const float3 inv = safe_inverse(d);
+  const Tri tt(o, d);
+  HitRec h{any ? -r.dir_far.w : r.dir_far.w, kInvalid, 0.0f, 0.0f};
+  int top = 1;
+  uint32_t cur = 0;
+  stk.put(0, kInvalid, true);
+  if (*nodes.differ == 0u) {
+    while (cur != kInvalid) {
+      const bool leaf_done = walk_quad_step(nodes.wide, tris, tt, l, o, d, inv, tnear, stk, top, cur, h);
+      if (any && leaf_done && h.prim != kInvalid) break;
+    }
+  } else {
+    while (cur != kInvalid) {
+      const bool leaf_done = walk_step(nodes.pairs, tris, tt, o, d, inv, tnear, h.t, stk, top, cur,
+                                       [&h](float t, float u, float v, uint32_t prim) {
+                                         if (t < h.t) h = HitRec{t, prim, u, v};
+                                       });
+      if (any && leaf_done && h.prim != kInvalid) break;
+    }
+  }
+  if (l != 0) return;
+  if (format == kHitCompact) {
     static_cast<uint2*>(out)[i] = make_uint2(__float_as_uint(h.t), h.prim);
   } else {
     const bool hit = h.prim != kInvalid;
@@ -333,15 +368,30 @@ hipError_t launch_simple(const Blas& b, const TraceArgs& a, uint32_t blocks, uin
 template <class Tri>
 hipError_t trace_blas_with(const Blas& b, const TraceArgs& a, hipStream_t stream) {
   if (a.anyhit && !a.stats) return launch_persistent<true, true, Tri>(b, a, stream);
+  // Four lanes per ray while that fills at most half of the chip's waves
+  // (65,536 rays): the launch then lasts as long as its longest walks, which
+  // are shorter this way.  us a call on soup (400,000 triangles), hills with
+  // boxes (500,000) and sphere (80,000), random rays / camera, four lanes and
+  // one: 1,000 rays 121 and 150 / 83 and 103, 74 and 98; 65,000 rays 202 and
+  // 229 / 107 and 145, 93 and 113; 130,000 rays (every wave resident) 315 and
+  // 264 / 113 and 169, 87 and 92; 262,000 rays 471 and 387 / 168 and 200.
+  const WalkNodes nodes = walk_nodes(b);
+  const uint64_t quads = (a.n + kQuadRays - 1) / kQuadRays;
+  if (nodes.wide && !a.stats && 2 * quads <= resident_grid(reinterpret_cast<const void*>(&k_trace_quad<Tri>), 256)) {
+    const uint32_t blocks = uint32_t(quads);
+    k_trace_quad<Tri><<<blocks, 256, 0, stream>>>(nodes, tri_records<Tri>(b), a.rays, a.n, a.out, a.format,
+                                                  make_uint2(a.inst_id, a.geom_id));
+    return hipGetLastError();
+  }
   // One ray per lane: the counting variant (the reference's order) and
   // nearest hits (rays that arrive in screen order stay coherent within a
   // wave, which the refilling kernel gives up).
   const uint32_t blocks = uint32_t((a.n + 255) / 256);
-  if (blocks <= resident_grid(reinterpret_cast<const void*>(&k_trace_simple<false, false, kStackDepth, Tri>), 256))
-    return launch_simple<kStackDepth, Tri>(b, a, blocks, nullptr, stream);
+  if (blocks <= resident_grid(reinterpret_cast<const void*>(&k_trace_simple<false, false, kWalkDepth, Tri>), 256))
+    return launch_simple<kWalkDepth, Tri>(b, a, blocks, nullptr, stream);
   uint32_t* spill = nullptr;
   hipError_t e = hipMallocAsync(reinterpret_cast<void**>(&spill),
-                                sizeof(uint32_t) * size_t(blocks) * 256 * (kStackDepth - kSimpleLds), stream);
+                                sizeof(uint32_t) * size_t(blocks) * 256 * (kWalkDepth - kSimpleLds), stream);
   if (e != hipSuccess) return e;
   e = launch_simple<kSimpleLds, Tri>(b, a, blocks, spill, stream);
   const hipError_t f = hipFreeAsync(spill, stream);

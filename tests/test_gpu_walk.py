@@ -1,0 +1,92 @@
+"""The two forms of the BVH2 nearest-hit walk (four lanes per ray for small launches, one for large ones): bit for
+bit the oracle's hits, and the counting variant's, at the sizes where the form or the last workgroup changes."""
+import numpy as np
+import pytest
+
+import heavyrt_amd as H
+from gpu_util import make_scene, say, trace
+from heavyrt_amd import workloads as W
+from oracle import oracle as O
+from test_gpu_parity import rays_for
+
+pytestmark = pytest.mark.gpu
+
+
+def stacked(n=100, copies=2):
+    """A small soup with n nested triangles in one Morton cell (one leaf), and every triangle twice (equal t)."""
+    v, f = W.soup(500, stream=W.STREAM_TEST)
+    tri = np.array([[0.0, 0.0, 0.0], [1.0, 0.0, 0.2], [0.0, 1.0, 0.1]]) - np.array([1.0, 1.0, 0.3]) / 3.0
+    k = np.arange(1, n + 1)[:, None, None]
+    nest = (np.array([0.5, 0.5, 0.5]) + 1e-3 * tri[None] * k + np.array([0, 0, 1e-6]) * k).reshape(-1, 3)
+    v = np.concatenate([v, nest.astype(np.float32)])
+    f = np.concatenate([f, 1500 + np.arange(3 * n, dtype=np.uint32).reshape(-1, 3)])
+    return v, np.concatenate([f] * copies)
+
+
+MESHES = {
+    "one_triangle": lambda: (np.array([[0, 0, 0], [1, 0, 0], [0, 1, 0]], np.float32), np.array([[0, 1, 2]], np.uint32)),
+    "two_leaves": lambda: W.soup(2, stream=W.STREAM_TEST),
+    "three_leaves": lambda: W.soup(3, stream=W.STREAM_TEST),
+    "stacked": lambda: stacked(50),
+    "soup_20k": lambda: W.soup(20_000, stream=W.STREAM_TEST),
+}
+
+
+def same(a, b):
+    for k in ("t", "prim", "u", "v"):
+        np.testing.assert_array_equal(a[k].view(np.uint32), b[k].view(np.uint32))
+
+
+@pytest.mark.parametrize("mesh", sorted(MESHES))
+@pytest.mark.parametrize("n", [1, 3, 63, 65, 5000])
+def test_small_launches_match_the_oracle(gpu_ctx, mesh, n):
+    v, f = MESHES[mesh]()
+    say(f"walk {mesh} {n}")
+    s = make_scene(gpu_ctx, v, f, keep=False)
+    rays = rays_for(v, n, 8100)
+    rays[1::3, 7] = -2.0 * W.scene_diagonal(v)  # any-hit queries among them
+    rays[2::7, 4:7] = [0.0, 0.0, -1.0]          # axis-parallel directions
+    g = trace(s, rays, "full")
+    t, prim = O.OracleBVH(v, f).trace(rays)[:2]
+    np.testing.assert_array_equal(g["t"].view(np.uint32), t.view(np.uint32))
+    np.testing.assert_array_equal(g["prim"], prim)
+    same(g, trace(s, rays, "full", stats=True))  # counted on the node pairs
+    s.close()
+
+
+@pytest.mark.parametrize("test", [H.TRI_MT, H.TRI_WATERTIGHT], ids=["mt", "wt"])
+def test_forms_agree_across_sizes(gpu_ctx, test):
+    v, f = W.merge(W.icosphere(4), W.ground_quad())
+    s = H.Scene(gpu_ctx)
+    s.add_instance(s.add_triangles(v, f))
+    s.set_triangle_test(test)
+    s.commit()
+    rays = rays_for(v, 140_000, 8200)
+    whole = trace(s, rays, "full")  # a ray per lane
+    for n in (1, 64, 32_768, 65_535, 65_536, 65_537, 131_073):
+        say(f"walk size {n}")
+        part = trace(s, rays[:n], "full")
+        for k in ("t", "prim", "u", "v"):
+            np.testing.assert_array_equal(part[k].view(np.uint32), whole[k][:n].view(np.uint32))
+    s.close()
+
+
+def test_nan_vertices_walk_the_pairs(gpu_ctx):
+    """A leaf without finite corners has an inverted box, which a union of boxes drops: such trees keep their pairs."""
+    v, f = W.soup(3000, stream=W.STREAM_TEST)
+    v = v.copy()
+    v[f[::97].reshape(-1)] = np.nan
+    s = make_scene(gpu_ctx, v, f, keep=False)
+    rays = rays_for(np.nan_to_num(v), 4000, 8300)
+    same(trace(s, rays, "full"), trace(s, rays, "full", stats=True))
+    s.close()
+
+
+def test_refit_moves_the_walked_boxes(gpu_ctx):
+    v, f = W.soup(20_000, stream=W.STREAM_TEST)
+    s = make_scene(gpu_ctx, v, f, keep=False)
+    s.update_triangles(0, (v * np.float32(1.5) + np.float32(0.25)).astype(np.float32), quality=3)
+    s.commit()
+    rays = rays_for(v * 1.5 + 0.25, 4000, 8400)
+    same(trace(s, rays, "full"), trace(s, rays, "full", stats=True))
+    s.close()
