@@ -395,24 +395,6 @@ __device__ inline bool mt_test(float3 o, float3 d, float tnear, const TriPre& tr
   return false;
 }
 
-// Same test with the (t, primId) rule of the BVH4 path: an equal-distance
-// triangle wins when its original id is smaller, so the nearest hit does not
-// depend on the order nodes are visited in.  t == tFar with no hit yet stays
-// outside the open interval.
-__device__ inline bool mt_test_lex(float3 o, float3 d, float tnear, const TriPre& tri, HitRec& h) {
-  float t, u, v;
-  const uint32_t prim = __float_as_uint(tri.a.w);
-  if (mt_eval(o, d, tnear, tri, t, u, v) &&
-      (t < h.t || (t == h.t && h.prim != kInvalid && prim < h.prim))) {
-    h.t = t;
-    h.prim = prim;
-    h.u = u;
-    h.v = v;
-    return true;
-  }
-  return false;
-}
-
 // ---------------------------------------------------------------------------
 // Triangle-test policies.  The traversal kernels take one as a template
 // parameter; a lane makes its ray's policy object once (per refill) and tests
@@ -539,25 +521,6 @@ __device__ inline bool tri_test_lex(const Tri& k, float3 o, float3 d, float tnea
     h.prim = prim;
     h.u = u;
     h.v = v;
-    return true;
-  }
-  return false;
-}
-
-// Two-level rule: inside one instance the first strictly closer hit wins, as
-// in mt_test; a hit at the same distance in an instance with a smaller id
-// replaces one from a larger id, so across instances the answer does not
-// depend on the order the top-level tree is walked in.
-__device__ inline bool mt_test_inst(float3 o, float3 d, float tnear, const TriPre& tri, uint32_t inst, HitRec& h,
-                                    uint32_t& h_inst) {
-  float t, u, v;
-  if (mt_eval(o, d, tnear, tri, t, u, v) &&
-      (t < h.t || (t == h.t && h.prim != kInvalid && inst < h_inst))) {
-    h.t = t;
-    h.prim = __float_as_uint(tri.a.w);
-    h.u = u;
-    h.v = v;
-    h_inst = inst;
     return true;
   }
   return false;

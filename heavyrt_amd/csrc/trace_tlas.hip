@@ -20,16 +20,19 @@
 // order (80 B each: inverse rows, the object's pairs and triangles, ids).
 //
 // Execution: a persistent wave64 kernel with ballot-based refill, one node
-// pair or one leaf per lane per step, and a per-lane stack of 64 entries: 16
-// in LDS, the rest in a per-lane global spill area.  64 covers the deepest
-// possible walk: at most 30 pending entries in the top-level tree plus 30 in
-// one object's tree (Karras trees over unique 30-bit codes have at most 30
-// internal levels).
+// pair, one triangle or one instance per lane per step (walk2.h), and a
+// per-lane stack of kTwoLevelDepth entries: 16 in LDS, the rest in a per-lane
+// global spill area.  That covers the deepest possible walk: the pending
+// entries of the top-level tree and of one object's tree (at most kStackDepth
+// each), the entry that ends the walk and the one that ends an object's.
+// Bound by waits for fetches: 480,000 camera rays over 2,001 instances took
+// 495 us with a pair and then a whole leaf per step, 426 with one fetch.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 
 #include "hrt_internal.h"
+#include "walk2.h"
 
 namespace hrt {
 namespace {
@@ -38,33 +41,12 @@ constexpr int kWave = 64;
 constexpr int kBlock = kWave;
 constexpr int kRefillAt = 16;
 constexpr uint32_t kClaim = 128;  // ray indices a wave claims from the queue at once
-constexpr int kTwoLevelDepth = 64;
+constexpr int kTwoLevelDepth = 2 * kStackDepth + 3;
+// Stack entry under an object's walk: the instance is done when it is popped.
+// (No leaf has this value: its triangles would lie past the 24-bit range.)
+constexpr uint32_t kInstanceDone = kInvalid - 1u;
 
 __global__ void k_reset_counter(uint32_t* c) { *c = 0u; }
-
-// One step of the near-first pair test shared by both levels: returns the next
-// node to visit, pushes the deferred child, or reports that both missed.
-__device__ inline bool pair_step(const NodePair* __restrict__ P, uint32_t& cur, float3 o, float3 inv, float tnear,
-                                 float tmax, const ShortStack<kShortStack, kBlock>& stk, int& top) {
-  const float4* pp = reinterpret_cast<const float4*>(P + cur);
-  const float4 lmin = pp[0], lmax = pp[1], rmin = pp[2], rmax = pp[3];
-  const float2 t0 = slab(o, inv, lmin.x, lmin.y, lmin.z, lmax.x, lmax.y, lmax.z);
-  const float2 t1 = slab(o, inv, rmin.x, rmin.y, rmin.z, rmax.x, rmax.y, rmax.z);
-  const bool h0 = (t0.x <= t0.y) && (t0.y >= tnear) && (t0.x <= tmax);
-  const bool h1 = (t1.x <= t1.y) && (t1.y >= tnear) && (t1.x <= tmax);
-  const uint32_t c0 = __float_as_uint(lmin.w), c1 = __float_as_uint(rmin.w);
-  if (h0 && h1) {
-    const bool left_first = t0.x <= t1.x;
-    cur = left_first ? c0 : c1;
-    stk.push(top, left_first ? c1 : c0);
-    return true;
-  }
-  if (h0 || h1) {
-    cur = h0 ? c0 : c1;
-    return true;
-  }
-  return false;
-}
 
 template <bool kForceAny, bool kStats>
 __global__ __launch_bounds__(kBlock) void k_trace_two_level(const NodePair* __restrict__ tlas,
@@ -92,7 +74,7 @@ __global__ __launch_bounds__(kBlock) void k_trace_two_level(const NodePair* __re
   const NodePair* P = tlas;  // tree being walked
   const TriPre* T = nullptr;
   bool in_blas = false;
-  int top = 0, inst_top = 0;
+  int top = 0;
   uint32_t k = 0, kend = 0;  // instances of the current top-level leaf
   uint32_t cur_inst = 0, cur_geom = 0;
   uint32_t cur = kInvalid;
@@ -110,24 +92,11 @@ __global__ __launch_bounds__(kBlock) void k_trace_two_level(const NodePair* __re
     cur_inst = I->inst;
     cur_geom = I->geom;
     in_blas = true;
-    inst_top = top;
+    stk.put(top, kInstanceDone, true);
+    top++;
     cur = 0;
   };
-  // the current subtree is done: next instance of the leaf, or pop
-  auto next = [&]() {
-    if (in_blas && top == inst_top) {
-      if (++k < kend) {
-        enter(k);
-        return;
-      }
-      in_blas = false;
-      P = tlas;
-      o = wo;
-      d = wd;
-      inv = winv;
-    }
-    cur = (top > 0) ? stk.pop(top) : kInvalid;
-  };
+  auto pop = [&]() { cur = stk.pop(top); };
 
   while (true) {
     const uint64_t idle = __ballot(!active);
@@ -152,8 +121,8 @@ __global__ __launch_bounds__(kBlock) void k_trace_two_level(const NodePair* __re
           h_inst = h_geom = kInvalid;
           P = tlas;
           in_blas = false;
-          top = 0;
-          inst_top = 0;
+          stk.put(0, kInvalid, true);
+          top = 1;
           k = kend = 0;
           cur = 0;
           npairs = ntests = 0;
@@ -166,15 +135,22 @@ __global__ __launch_bounds__(kBlock) void k_trace_two_level(const NodePair* __re
     while (true) {
       bool done = false;
       if (active) {
-        if ((cur & kLeafBit) == 0) {
-          if (kStats) npairs++;
-          if (!pair_step(P, cur, o, inv, tnear, h.t, stk, top)) next();
-        } else if (in_blas) {
-          const uint32_t s = leaf_start(cur), c = leaf_count(cur);
-          if (kStats) ntests += c;
-          for (uint32_t j = s; j < s + c; j++)
-            if (mt_test_inst(o, d, tnear, T[j], cur_inst, h, h_inst)) h_geom = cur_geom;
-          next();
+        bool leaf_done = false;
+        if (in_blas || (cur & kLeafBit) == 0) {
+          if (kStats) {
+            npairs += (cur & kLeafBit) == 0;
+            ntests += (cur & kLeafBit) != 0 && leaf_count(cur) != 0;
+          }
+          // inside one instance the first strictly closer hit wins; at equal
+          // t an instance with a smaller id replaces one with a larger id
+          leaf_done = walk_step(P, T, MtTest(), o, d, inv, tnear, h.t, stk, top, cur,
+                                [&](float t, float u, float v, uint32_t prim) {
+                                  if (t < h.t || (t == h.t && h.prim != kInvalid && cur_inst < h_inst)) {
+                                    h = HitRec{t, prim, u, v};
+                                    h_inst = cur_inst;
+                                    h_geom = cur_geom;
+                                  }
+                                });
         } else {
           const uint32_t s = leaf_start(cur), c = leaf_count(cur);
           if (c > 0) {
@@ -182,10 +158,22 @@ __global__ __launch_bounds__(kBlock) void k_trace_two_level(const NodePair* __re
             kend = s + c;
             enter(k);
           } else {
-            next();
+            pop();
           }
         }
-        done = (cur == kInvalid) || (any && h.prim != kInvalid);
+        if (cur == kInstanceDone) {  // the next instance of the leaf, or on with the top-level tree
+          if (++k < kend) {
+            enter(k);
+          } else {
+            in_blas = false;
+            P = tlas;
+            o = wo;
+            d = wd;
+            inv = winv;
+            pop();
+          }
+        }
+        done = (cur == kInvalid) || (any && leaf_done && h.prim != kInvalid);
       }
       if (done) {
         const bool hit = h.prim != kInvalid;
@@ -235,20 +223,11 @@ __global__ __launch_bounds__(256) void k_misses(const Ray* __restrict__ rays, ui
   }
 }
 
-int resident_grid(const void* kernel) {
-  int dev = 0, cus = 0, per_cu = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return 1024;
-  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) cus = 256;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kBlock, 0) != hipSuccess || per_cu <= 0)
-    per_cu = 8;
-  return cus * per_cu;
-}
-
 template <bool kAny, bool kStats>
 hipError_t launch(const Blas& tlas, const InstDev* inst, const TraceArgs& a, hipStream_t stream) {
   const void* kfn = reinterpret_cast<const void*>(&k_trace_two_level<kAny, kStats>);
   const uint64_t want = (a.n + kBlock - 1) / kBlock;
-  const int grid = int(std::min<uint64_t>(want, uint64_t(resident_grid(kfn))));
+  const int grid = int(std::min<uint64_t>(want, uint64_t(resident_grid(kfn, kBlock))));
   const size_t spill_words = size_t(grid) * kBlock * (kTwoLevelDepth - kShortStack);
   uint32_t* buf = nullptr;
   hipError_t e = hipMallocAsync(reinterpret_cast<void**>(&buf), sizeof(uint32_t) * (64 + spill_words), stream);
