@@ -22,6 +22,7 @@
 
 #include "ao.h"
 #include "hrt_internal.h"
+#include "quad.h"
 
 namespace hrt {
 namespace {
@@ -401,9 +402,168 @@ __global__ __launch_bounds__(kBlock4, 8) void k_trace4_any_persistent(const void
   }
 }
 
+// --- Four lanes per ray (quad.h) ---------------------------------------------
+// A launch that leaves the chip idle lasts as long as its longest walk, a chain
+// of one node fetch and its arithmetic per step.  With a child per lane a step
+// is a fetch of 16 bytes a lane (FP16; the four lanes read the 64-byte node
+// together) and about 55 VALU instructions instead of 130, and a leaf's first
+// four triangles are tested at once.  The walk is the one-lane kernels' own:
+// the same boxes, order and rules, so the same hits.
+constexpr uint32_t kQuadRays4 = 64;  // rays per workgroup of 256
+
+// Box distances and reference of child l of node q.
+template <bool kFp16, bool kFused, class Tri>
+__device__ inline float2 child_box(const void* __restrict__ quads, uint32_t q, uint32_t l, float3 o, float3 inv,
+                                   float3 oi, bool fz, const Tri& tt, uint32_t& ref) {
+  if (kFp16) {
+    const uint4 w = static_cast<const Quad16*>(quads)[q].c[l];
+    ref = w.w;
+    if (kFused && !Tri::kRobustBoxes && fz) return slab_fused(oi, inv, w, near_far_selectors(inv));
+    return tt.box(o, inv, h2f_lo(w.x), h2f_hi(w.x), h2f_lo(w.y), h2f_hi(w.y), h2f_lo(w.z), h2f_hi(w.z));
+  }
+  const float* f = reinterpret_cast<const float*>(static_cast<const Quad32*>(quads) + q) + l;
+  ref = __float_as_uint(f[24]);
+  return tt.box(o, inv, f[0], f[8], f[16], f[4], f[12], f[20]);
+}
+
+// Nearest hits, k_trace4_simple's walk.  Its five-comparator network runs over
+// the lanes (the same exchanges, so the same order on equal entries); then
+// lane k holds the k-th child, and the lanes store what is deferred at once.
+template <bool kFp16, class Tri>
+__global__ __launch_bounds__(256) void k_trace4_quad(const void* __restrict__ quads, const TriPre* __restrict__ tris,
+                                                     const Ray* __restrict__ rays, uint64_t n, void* out, int format,
+                                                     uint2 ids) {
+  // kStackDepth4 deferred children and, below them, kInvalid, which ends the walk
+  __shared__ uint32_t stack_mem[(kStackDepth4 + 1) * kQuadRays4];
+  const uint32_t l = threadIdx.x & 3u, slot = threadIdx.x >> 2;
+  const uint64_t i = uint64_t(blockIdx.x) * kQuadRays4 + slot;
+  if (i >= n) return;
+  lds_u32* stack = (lds_u32*)(stack_mem + slot);
+  const Ray r = rays[i];
+  const float3 o = make_float3(r.pos_near.x, r.pos_near.y, r.pos_near.z);
+  const float3 d = make_float3(r.dir_far.x, r.dir_far.y, r.dir_far.z);
+  const float tnear = r.pos_near.w;
+  const bool any = r.dir_far.w <= 0.0f;
+  const float3 inv = safe_inverse(d);
+  const Tri tt(o, d);
+  HitRec h{any ? -r.dir_far.w : r.dir_far.w, kInvalid, 0.0f, 0.0f};
+  uint32_t top = 1, cur = 0;
+  stack[0] = kInvalid;
+  while (cur != kInvalid) {
+    const uint32_t popped = stack[(top - 1) * kQuadRays4];
+    if (int32_t(cur) >= 0) {
+      uint32_t ch;
+      const float2 bt = child_box<kFp16, false>(quads, cur, l, o, inv, o, false, tt, ch);
+      float tm = child_hit(bt, ch, tnear, h.t) ? bt.x : kMaxFloat;
+      // (0,1) (2,3), then (0,2) (1,3), then (1,2): the lower lane takes the
+      // other's child when that one is strictly nearer
+      auto exchange = [&](float to, uint32_t co, bool lower, bool in) {
+        const bool take = in & (lower ? to < tm : tm < to);
+        tm = take ? to : tm;
+        ch = take ? co : ch;
+      };
+      exchange(quad_x1(tm), quad_x1(ch), (l & 1u) == 0u, true);
+      exchange(quad_x2(tm), quad_x2(ch), (l & 2u) == 0u, true);
+      exchange(quad_read<quad_perm(0, 2, 1, 3)>(tm), quad_read<quad_perm(0, 2, 1, 3)>(ch), l == 1u,
+               l == 1u || l == 2u);
+      const uint32_t hits = quad_or(tm < kMaxFloat ? 1u << l : 0u);  // 0, 1, 3, 7 or 15
+      const uint32_t nh = __popc(hits);
+      if (l > 0u && l < nh) stack[(top + nh - 1u - l) * kQuadRays4] = ch;
+      cur = nh ? quad_read<quad_perm(0, 0, 0, 0)>(ch) : popped;
+      top += nh - 1u;
+      continue;
+    }
+    const uint32_t s = leaf_start(cur), c = leaf_count(cur);
+    bool hit;
+    if (any)  // the leaf's first triangle that is hit
+      hit = quad_triangles<true>(tris, l, s, c, tt, o, d, tnear, h,
+                                 [](float t, uint32_t, const HitRec& h0) { return t < h0.t; });
+    else
+      hit = quad_triangles<false, true>(tris, l, s, c, tt, o, d, tnear, h, [](float t, uint32_t p, const HitRec& h0) {
+        return t < h0.t || (t == h0.t && h0.prim != kInvalid && p < h0.prim);
+      });
+    if (any && hit) break;
+    const bool last = c <= 4u;
+    cur = last ? popped : cur - (4u << 24) + 4u;
+    top -= uint32_t(last);
+  }
+  if (l == 0u) write_hit<false>(out, i, format, ids, h);
+}
+
+// Any-hit answers, the children in stored order as in the persistent kernel.
+template <bool kFp16, class Src, class Tri>
+__global__ __launch_bounds__(256) void k_trace4_any_quad(const void* __restrict__ quads,
+                                                         const TriPre* __restrict__ tris, Src src, uint64_t n,
+                                                         uint8_t* __restrict__ out) {
+  __shared__ uint32_t stack_mem[(kStackDepth4 + 1) * kQuadRays4];
+  const uint32_t l = threadIdx.x & 3u, slot = threadIdx.x >> 2;
+  const uint64_t at = uint64_t(blockIdx.x) * kQuadRays4 + slot;
+  if (at >= n) return;
+  lds_u32* stack = (lds_u32*)(stack_mem + slot);
+  const uint64_t i = src.index(at);
+  const Ray r = src.ray(i);
+  const float3 o = make_float3(r.pos_near.x, r.pos_near.y, r.pos_near.z);
+  const float3 d = make_float3(r.dir_far.x, r.dir_far.y, r.dir_far.z);
+  const float tnear = r.pos_near.w;
+  const float3 inv = safe_inverse(d);
+  const float3 oi = neg_o_inv(o, inv);
+  const bool fz = fused_ok(oi);
+  const Tri tt(o, d);
+  HitRec h{fabsf(r.dir_far.w), kInvalid, 0.0f, 0.0f};
+  uint32_t top = 1, cur = h.t > tnear ? 0u : kInvalid;
+  bool hit = false;
+  stack[0] = kInvalid;
+  while (cur != kInvalid) {
+    const uint32_t popped = stack[(top - 1) * kQuadRays4];
+    if (int32_t(cur) >= 0) {
+      uint32_t ch;
+      const float2 bt = child_box<kFp16, kFp16>(quads, cur, l, o, inv, oi, fz, tt, ch);
+      const bool in = child_hit(bt, ch, tnear, h.t);
+      const uint32_t hits = quad_or(in ? 1u << l : 0u);
+      const uint32_t nh = __popc(hits), below = __popc(hits & ((1u << l) - 1u));
+      if (in && below > 0u) stack[(top + nh - 1u - below) * kQuadRays4] = ch;
+      // references are never 0: the root is nobody's child, a leaf has kLeafBit
+      const uint32_t next = quad_or(in && below == 0u ? ch : 0u);
+      cur = nh ? next : popped;
+      top += nh - 1u;
+      continue;
+    }
+    const uint32_t s = leaf_start(cur), c = leaf_count(cur);
+    bool mine = false;
+    if (l < c) mine = tri_hit_before(tt, o, d, tnear, tris[s + l], h.t);
+    hit = quad_or(mine ? 1u : 0u) != 0u;
+    if (hit) break;
+    const bool last = c <= 4u;
+    cur = last ? popped : cur - (4u << 24) + 4u;
+    top -= uint32_t(last);
+  }
+  if (l == 0u) out[i] = hit ? 1 : 0;
+}
+
+// Whether a launch of n rays takes four lanes per ray: up to `share` times the
+// rays resident at once (131,072).  us a call, one lane and four, on the FP16
+// nodes of the clustered tree of soup (400,000 triangles), hills with boxes
+// (500,000) and sphere (80,000):
+//   nearest hits, random rays, share 1/2: 1,000 rays 207/175, 84/60, 93/75;
+//     65,000 rays 294/207, 141/97, 139/95; 262,000 rays 415/473, 222/197,
+//     183/158.
+//   any-hit, bounced rays, share 4 (the persistent kernel's last rays cost it
+//     about 100 us at any size): 1,000 rays 172/72, 116/49, 91/43; 65,000 rays
+//     270/128, 185/82, 128/54; 524,000 rays 437/431, 321/236, 270/165;
+//     1,048,000 rays 597/758, 403/421, 321/280.
+inline bool takes_quads(const void* kernel, uint64_t n, double share) {
+  return double((n + kQuadRays4 - 1) / kQuadRays4) <= share * resident_grid(kernel, 256);
+}
+constexpr double kQuadShareNearest = 0.5, kQuadShareAny = 4.0;
+
 template <bool kFp16, class Src, class Tri>
 hipError_t launch_any4(const Blas& b, Src src, uint64_t n, uint8_t* out, hipStream_t stream,
                        uint32_t* workspace = nullptr, size_t workspace_words = 0) {
+  if (takes_quads(reinterpret_cast<const void*>(&k_trace4_any_quad<kFp16, Src, Tri>), n, kQuadShareAny)) {
+    k_trace4_any_quad<kFp16, Src, Tri><<<uint32_t((n + kQuadRays4 - 1) / kQuadRays4), 256, 0, stream>>>(
+        kFp16 ? static_cast<const void*>(b.quads16) : b.quads32, tri_records<Tri>(b), src, n, out);
+    return hipGetLastError();
+  }
   const void* kfn = reinterpret_cast<const void*>(&k_trace4_any_persistent<kFp16, Src, Tri>);
   const uint64_t want = (n + kBlock4 - 1) / kBlock4;
   constexpr size_t kLaneWords = kStackDepth4 - kShortStack;
@@ -477,6 +637,13 @@ __global__ void k_order_or_null(const uint32_t* __restrict__ err, const uint32_t
 template <bool kFp16, class Tri>
 hipError_t launch_simple4(const Blas& b, const TraceArgs& a, const uint32_t* const* order_slot,
                           hipStream_t stream) {
+  if (!a.anyhit && !a.stats && takes_quads(reinterpret_cast<const void*>(&k_trace4_quad<kFp16, Tri>), a.n,
+                                             kQuadShareNearest)) {
+    k_trace4_quad<kFp16, Tri><<<uint32_t((a.n + kQuadRays4 - 1) / kQuadRays4), 256, 0, stream>>>(
+        kFp16 ? static_cast<const void*>(b.quads16) : b.quads32, tri_records<Tri>(b), a.rays, a.n, a.out, a.format,
+        make_uint2(a.inst_id, a.geom_id));
+    return hipGetLastError();
+  }
   const uint32_t blocks = uint32_t((a.n + kBlock4 - 1) / kBlock4);
   const void* q = kFp16 ? static_cast<const void*>(b.quads16) : static_cast<const void*>(b.quads32);
   // stack entries beyond the LDS part, per lane (none while LDS holds them all)
@@ -590,6 +757,11 @@ hipError_t serve_any4(bool fp16, const uint32_t* off, const ServeSeg* segs, uint
 
 void warm_any_hit_launchers() {
   warm_bvh2_any_hit_launchers();
+  const void* quad[] = {reinterpret_cast<const void*>(&k_trace4_any_quad<true, StoredRays, MtTest>),
+                        reinterpret_cast<const void*>(&k_trace4_any_quad<false, StoredRays, MtTest>),
+                        reinterpret_cast<const void*>(&k_trace4_any_quad<true, StoredRays, WtTest>),
+                        reinterpret_cast<const void*>(&k_trace4_any_quad<false, StoredRays, WtTest>)};
+  for (const void* f : quad) (void)resident_grid(f, 256);
   const void* k[] = {reinterpret_cast<const void*>(&k_trace4_any_persistent<true, StoredRays, MtTest>),
                      reinterpret_cast<const void*>(&k_trace4_any_persistent<false, StoredRays, MtTest>),
                      reinterpret_cast<const void*>(&k_trace4_any_persistent<true, StoredRays, WtTest>),

@@ -27,18 +27,12 @@
 #include <hip/hip_runtime.h>
 
 #include "hrt_device.h"
+#include "quad.h"
 
 namespace hrt {
 
-typedef float walk_f4 __attribute__((ext_vector_type(4)));
-
 __device__ inline bool walk_hit(float t0, float t1, float tnear, float tmax) {
   return bool(int(t0 <= t1) & int(t1 >= tnear) & int(t0 <= tmax));  // no branches
-}
-
-__device__ inline TriPre walk_triangle(walk_f4 q0, walk_f4 q1, walk_f4 q2) {
-  return TriPre{make_float4(q0.x, q0.y, q0.z, q0.w), make_float4(q1.x, q1.y, q1.z, 0.0f),
-                make_float4(q2.x, q2.y, q2.z, 0.0f)};
 }
 
 // One step of a lane at `cur` (not kInvalid): the pair's or the triangle's
@@ -93,21 +87,6 @@ __device__ inline bool walk_step(const NodePair* __restrict__ P, const TriPre* _
   return leaf && pop;
 }
 
-// The value of the lane one and two places on in this lane's group of four
-// (lane ^ 1, lane ^ 2).
-__device__ inline uint32_t quad_x1(uint32_t v) {
-  return uint32_t(__builtin_amdgcn_update_dpp(0, int(v), 0xB1, 0xF, 0xF, true));
-}
-__device__ inline uint32_t quad_x2(uint32_t v) {
-  return uint32_t(__builtin_amdgcn_update_dpp(0, int(v), 0x4E, 0xF, 0xF, true));
-}
-__device__ inline float quad_x1(float v) { return __uint_as_float(quad_x1(__float_as_uint(v))); }
-__device__ inline float quad_x2(float v) { return __uint_as_float(quad_x2(__float_as_uint(v))); }
-__device__ inline uint32_t quad_or(uint32_t v) {
-  v |= quad_x1(v);
-  return v | quad_x2(v);
-}
-
 // Entry and exit of the union of this lane's box and lane ^ 1's, from their
 // distances per axis.  In asm because the compiler quiets (v_max x, x) every
 // operand that comes through DPP or asm, 14 instructions more; a DPP source
@@ -134,10 +113,8 @@ __device__ inline void quad_union(float nx, float ny, float nz, float fx, float 
 // exactly, because rounding is monotonic; k_wide_nodes finds the trees where a
 // stored child box is not the union of its children's, and they are walked on
 // their pairs.  Both levels use the same hit distance, as the reference's two
-// steps do, since no triangle lies between them.  A lane's candidate triangles
-// are taken in leaf order: the nearest of the four, the first on equal t, and
-// only if it is nearer than the hit so far.  Returns true when the ray has
-// just finished a leaf.
+// steps do, since no triangle lies between them.  Returns true when the ray
+// has just finished a leaf.
 template <class Tri, class Stack>
 __device__ inline bool walk_quad_step(const WideNode* __restrict__ W, const TriPre* __restrict__ T, const Tri& tt,
                                       uint32_t l, float3 o, float3 d, float3 inv, float tnear, const Stack& stk,
@@ -193,28 +170,8 @@ __device__ inline bool walk_quad_step(const WideNode* __restrict__ W, const TriP
     return false;
   }
   const uint32_t count = leaf_count(cur);
-  float t = 0.0f, u = 0.0f, v = 0.0f;
-  uint32_t prim = kInvalid;
-  if (l < count) {
-    const walk_f4* p = reinterpret_cast<const walk_f4*>(T + leaf_start(cur) + l);
-    walk_f4 q0 = p[0], q1 = p[1], q2 = p[2];
-    asm volatile("" : "+v"(q0), "+v"(q1), "+v"(q2));
-    if (tt.eval(o, d, tnear, walk_triangle(q0, q1, q2), t, u, v) && t < h.t) prim = __float_as_uint(q0.w);
-  }
-  const float kInf = __builtin_inff();
-  const float tc = prim != kInvalid ? t : kInf;
-  float m = fminf(tc, quad_x1(tc));
-  m = fminf(m, quad_x2(m));
-  // the lowest lane whose t is the least
-  uint32_t w = prim != kInvalid && tc == m ? 1u << l : 0u;
-  w = quad_or(w);
-  if (w != 0u) {
-    const bool mine = (w & (0u - w)) == (1u << l);
-    h.t = __uint_as_float(quad_or(mine ? __float_as_uint(t) : 0u));  // not m: +0 and -0 are equal
-    h.prim = quad_or(mine ? prim : 0u);
-    h.u = __uint_as_float(quad_or(mine ? __float_as_uint(u) : 0u));
-    h.v = __uint_as_float(quad_or(mine ? __float_as_uint(v) : 0u));
-  }
+  quad_triangles(T, l, leaf_start(cur), count, tt, o, d, tnear, h,
+                 [](float t, uint32_t, const HitRec& h0) { return t < h0.t; });
   const bool last = count <= 4u;
   cur = last ? popped : cur - (4u << 24) + 4u;
   top -= int(last);

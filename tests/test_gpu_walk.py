@@ -71,6 +71,27 @@ def test_forms_agree_across_sizes(gpu_ctx, test):
     s.close()
 
 
+@pytest.mark.parametrize("layout", [H.LAYOUT_BVH4, H.LAYOUT_PLOC_FP16], ids=["bvh4", "ploc_fp16"])
+@pytest.mark.parametrize("test", [H.TRI_MT, H.TRI_WATERTIGHT], ids=["mt", "wt"])
+def test_bvh4_forms_agree_across_sizes(gpu_ctx, layout, test):
+    v, f = W.merge(stacked(50), W.icosphere(3))
+    s = H.Scene(gpu_ctx)
+    s.add_instance(s.add_triangles(v, f))
+    s.set_triangle_test(test)
+    s.commit(layout=layout)
+    rays = rays_for(v, 600_000, 8500)
+    rays[1::5, 7] = -0.7 * W.scene_diagonal(v)  # any-hit queries among the nearest ones
+    whole, hit = trace(s, rays[:200_000], "full"), trace(s, rays, "any")["hit"]  # a ray per lane
+    say(f"bvh4 walk layout {layout}: {int(hit.sum())} of {hit.size} hit")
+    for n in (1, 17, 64, 4097, 65_536, 65_537, 131_073):
+        part = trace(s, rays[:n], "full")
+        for k in ("t", "prim", "u", "v"):
+            np.testing.assert_array_equal(part[k].view(np.uint32), whole[k][:n].view(np.uint32))
+    for n in (1, 63, 65_537, 524_288, 524_289):
+        np.testing.assert_array_equal(trace(s, rays[:n], "any")["hit"], hit[:n])
+    s.close()
+
+
 def test_nan_vertices_walk_the_pairs(gpu_ctx):
     """A leaf without finite corners has an inverted box, which a union of boxes drops: such trees keep their pairs."""
     v, f = W.soup(3000, stream=W.STREAM_TEST)
