@@ -901,6 +901,15 @@ hrt_status hrt_eye_render(hrt_scene* s, const float projInvColMajor16[16], const
   hipStream_t hs = stream ? static_cast<hipStream_t>(stream) : s->ctx->stream;
   hipError_t e = hipSetDevice(s->ctx->device);
   if (e != hipSuccess) return fail_hip(e, "hipSetDevice");
+  const bool on_bvh2 = s->layout == HRT_LAYOUT_BVH2 || s->layout == HRT_LAYOUT_AUTO || s->layout == HRT_LAYOUT_AUTO_FP16;
+  if (!s->two_level && on_bvh2 && n <= 0x7FFFFFFFull) {
+    const hrt::Blas* b = nullptr;
+    uint32_t inst = 0;
+    if ((st = select_blas(s, &b, &inst)) != HRT_OK) return st;
+    e = hrt::eye_frame(*b, s->committed_tri_test == HRT_TRI_WATERTIGHT, cam, width, height, pal, outColor, hs);
+    return e == hipSuccess ? HRT_OK : fail_hip(e, "eye render");
+  }
+  // other trees: rays to HBM, traced as a batch, coloured from the hits
   void* buf = nullptr;
   if ((e = hipMallocAsync(&buf, 40 * n, hs)) != hipSuccess) return fail_hip(e, "eye render buffers");
   float* rays = static_cast<float*>(buf);

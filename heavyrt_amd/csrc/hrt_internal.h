@@ -272,6 +272,9 @@ hipError_t eye_make_rays(const EyeCamera& cam, uint32_t width, uint32_t height, 
 // as the rays were made.
 hipError_t eye_colors(const void* hits_compact, uint32_t width, uint32_t height, const EyePalette& pal,
                       uint32_t* out_color, hipStream_t stream, bool stripes = false);
+// The whole frame in one launch on b's BVH2: rays, nearest hits and colours.
+hipError_t eye_frame(const Blas& b, bool watertight, const EyeCamera& cam, uint32_t width, uint32_t height,
+                     const EyePalette& pal, uint32_t* out_color, hipStream_t stream);
 // The 02_rtao frame's colours from compact primary hits (superblock order)
 // and one occlusion byte per AO ray (spp per pixel).
 hipError_t ao_colors(const void* hits_compact, const uint8_t* occluded, uint32_t width, uint32_t height,

@@ -33,6 +33,7 @@
 #include <mutex>
 #include <vector>
 
+#include "eye.h"
 #include "hrt_internal.h"
 #include "walk2.h"
 
@@ -63,14 +64,54 @@ struct HitOutFull {  // CRT_Hit (CrossRT.h:20-27)
 
 __global__ void k_reset_counter(uint32_t* c) { *c = 0u; }
 
+// Where a nearest-hit kernel's rays come from and its hits go.
+//   RayBatch   rays and hit records of a batch in HBM
+//   EyeFrame   a frame of hrt_eye_render: rays made in registers, the pixel's
+//              colour written (0 on a miss, else palette[primId % size]).  One
+//              launch instead of rays, trace and colours with 40 bytes a pixel
+//              through a buffer allocated per frame: 512x512 frames of sphere,
+//              hills with boxes and soup (100,000 triangles) 134, 253 and 308
+//              us before the one-fetch walk, 87, 150 and 246 now; 64x64 109,
+//              160 and 200, now 57, 86 and 105.
+struct RayBatch {
+  const Ray* __restrict__ rays;
+  void* __restrict__ out;
+  int format;
+  uint2 ids;
+  __device__ Ray ray(uint64_t i) const { return rays[i]; }
+  __device__ void put(uint64_t i, const HitRec& h) const {
+    if (format == kHitCompact) {
+      static_cast<uint2*>(out)[i] = make_uint2(__float_as_uint(h.t), h.prim);
+      return;
+    }
+    const bool hit = h.prim != kInvalid;
+    float4* o4 = reinterpret_cast<float4*>(static_cast<HitOutFull*>(out) + i);
+    o4[0] = make_float4(h.t, __uint_as_float(h.prim), __uint_as_float(hit ? ids.x : kInvalid),
+                        __uint_as_float(hit ? ids.y : kInvalid));
+    o4[1] = make_float4(h.u, h.v, 0.0f, 0.0f);
+  }
+};
+
+struct EyeFrame {
+  EyeCamera cam;
+  EyePalette pal;
+  uint32_t width, height;
+  uint32_t* __restrict__ color;
+  uint32_t group;  // rays per workgroup of the kernel
+  __device__ uint2 pixel(uint32_t i) const { return xcd_stripe_pixel(i, width, height, group); }
+  __device__ Ray ray(uint64_t i) const { return eye_ray(cam, pixel(uint32_t(i)), width, height); }
+  __device__ void put(uint64_t i, const HitRec& h) const {
+    const uint2 px = pixel(uint32_t(i));
+    color[px.y * width + px.x] = h.prim == kInvalid ? 0u : pal.c[h.prim % pal.n];
+  }
+};
+
 // The reference's order, one ray per lane (no refill): nearest hits, and the
 // counting variant, whose counters are the reference's.
-template <bool kForceAny, bool kStats, int kLds, class Tri = MtTest>
+template <bool kForceAny, bool kStats, int kLds, class Tri, class Io>
 __global__ __launch_bounds__(256) void k_trace_simple(const NodePair* __restrict__ pairs,
-                                                      const TriPre* __restrict__ tris,
-                                                      const Ray* __restrict__ rays, uint64_t n, void* out,
-                                                      int format, uint2 ids, uint32_t* __restrict__ stats,
-                                                      uint32_t* __restrict__ spill) {
+                                                      const TriPre* __restrict__ tris, Io io, uint64_t n,
+                                                      uint32_t* __restrict__ stats, uint32_t* __restrict__ spill) {
   __shared__ uint32_t stack_mem[kLds * 256];
   const uint64_t i = uint64_t(blockIdx.x) * 256 + threadIdx.x;
   if (i >= n) return;
@@ -78,7 +119,7 @@ __global__ __launch_bounds__(256) void k_trace_simple(const NodePair* __restrict
     if constexpr (kLds == kWalkDepth) return LdsStack<256>(stack_mem + threadIdx.x);
     else return ShortStack<kLds, 256>{stack_mem + threadIdx.x, spill + i, gridDim.x * 256u};
   }();
-  const Ray r = rays[i];
+  const Ray r = io.ray(i);
   const float3 o = make_float3(r.pos_near.x, r.pos_near.y, r.pos_near.z);
   const float3 d = make_float3(r.dir_far.x, r.dir_far.y, r.dir_far.z);
   const float tnear = r.pos_near.w;
@@ -110,33 +151,23 @@ __global__ __launch_bounds__(256) void k_trace_simple(const NodePair* __restrict
     stats[2 * i + 0] = npairs;
     stats[2 * i + 1] = ntests;
   }
-  if (kForceAny) {
-    static_cast<uint8_t*>(out)[i] = (h.prim != kInvalid) ? 1 : 0;
-  } else if (format == kHitCompact) {
-    static_cast<uint2*>(out)[i] = make_uint2(__float_as_uint(h.t), h.prim);
-  } else {
-    const bool hit = h.prim != kInvalid;
-    float4* o4 = reinterpret_cast<float4*>(static_cast<HitOutFull*>(out) + i);
-    o4[0] = make_float4(h.t, __uint_as_float(h.prim), __uint_as_float(hit ? ids.x : kInvalid),
-                        __uint_as_float(hit ? ids.y : kInvalid));
-    o4[1] = make_float4(h.u, h.v, 0.0f, 0.0f);
-  }
+  if constexpr (kForceAny) static_cast<uint8_t*>(io.out)[i] = (h.prim != kInvalid) ? 1 : 0;
+  else io.put(i, h);
 }
 
 // Nearest hits in the reference's order, four lanes per ray (walk_quad_step),
 // kQuadRays rays per workgroup.  On a tree whose WideNodes may not be walked
 // the four lanes walk its pairs alike.
 constexpr uint32_t kQuadRays = 64;
-template <class Tri>
-__global__ __launch_bounds__(256) void k_trace_quad(WalkNodes nodes, const TriPre* __restrict__ tris,
-                                                    const Ray* __restrict__ rays, uint64_t n, void* out, int format,
-                                                    uint2 ids) {
+template <class Tri, class Io>
+__global__ __launch_bounds__(256) void k_trace_quad(WalkNodes nodes, const TriPre* __restrict__ tris, Io io,
+                                                    uint64_t n) {
   __shared__ uint32_t stack_mem[kWalkDepth * kQuadRays];
   const uint32_t l = threadIdx.x & 3u, q = threadIdx.x >> 2;
   const uint64_t i = uint64_t(blockIdx.x) * kQuadRays + q;
   if (i >= n) return;
   const LdsStack<int(kQuadRays)> stk(stack_mem + q);
-  const Ray r = rays[i];
+  const Ray r = io.ray(i);
   const float3 o = make_float3(r.pos_near.x, r.pos_near.y, r.pos_near.z);
   const float3 d = make_float3(r.dir_far.x, r.dir_far.y, r.dir_far.z);
   const float tnear = r.pos_near.w;
@@ -161,16 +192,7 @@ __global__ __launch_bounds__(256) void k_trace_quad(WalkNodes nodes, const TriPr
       if (any && leaf_done && h.prim != kInvalid) break;
     }
   }
-  if (l != 0) return;
-  if (format == kHitCompact) {
-    static_cast<uint2*>(out)[i] = make_uint2(__float_as_uint(h.t), h.prim);
-  } else {
-    const bool hit = h.prim != kInvalid;
-    float4* o4 = reinterpret_cast<float4*>(static_cast<HitOutFull*>(out) + i);
-    o4[0] = make_float4(h.t, __uint_as_float(h.prim), __uint_as_float(hit ? ids.x : kInvalid),
-                        __uint_as_float(hit ? ids.y : kInvalid));
-    o4[1] = make_float4(h.u, h.v, 0.0f, 0.0f);
-  }
+  if (l == 0) io.put(i, h);
 }
 
 // Persistent wave64 traversal with ballot-based refill.
@@ -349,53 +371,55 @@ hipError_t launch_persistent(const Blas& b, const TraceArgs& a, hipStream_t stre
   return e != hipSuccess ? e : f;
 }
 
-template <int kLds, class Tri>
-hipError_t launch_simple(const Blas& b, const TraceArgs& a, uint32_t blocks, uint32_t* spill, hipStream_t stream) {
-  const uint2 ids = make_uint2(a.inst_id, a.geom_id);
+// Nearest hits of n rays in the reference's order.  Four lanes per ray while
+// that fills at most half of the chip's waves (65,536 rays): the launch then lasts as long as its longest walks, which are shorter this
+// way.  us a call on soup (400,000 triangles), hills with boxes (500,000) and
+// sphere (80,000), random rays / camera, four lanes and one: 1,000 rays 121
+// and 150 / 83 and 103, 74 and 98; 65,000 rays 202 and 229 / 107 and 145, 93
+// and 113; 130,000 rays (every wave resident) 315 and 264 / 113 and 169, 87
+// and 92; 262,000 rays 471 and 387 / 168 and 200.
+template <class Tri, class Io>
+hipError_t trace_nearest(const Blas& b, const Io& io, uint64_t n, hipStream_t stream) {
   const TriPre* tris = tri_records<Tri>(b);
-  if (a.stats && a.anyhit)
-    k_trace_simple<true, true, kLds, Tri><<<blocks, 256, 0, stream>>>(b.pairs, tris, a.rays, a.n, a.out, a.format,
-                                                                       ids, a.stats, spill);
-  else if (a.stats)
-    k_trace_simple<false, true, kLds, Tri><<<blocks, 256, 0, stream>>>(b.pairs, tris, a.rays, a.n, a.out, a.format,
-                                                                        ids, a.stats, spill);
-  else
-    k_trace_simple<false, false, kLds, Tri><<<blocks, 256, 0, stream>>>(b.pairs, tris, a.rays, a.n, a.out,
-                                                                         a.format, ids, nullptr, spill);
-  return hipGetLastError();
+  const WalkNodes nodes = walk_nodes(b);
+  const uint64_t quads = (n + kQuadRays - 1) / kQuadRays;
+  if (nodes.wide && 2 * quads <= resident_grid(reinterpret_cast<const void*>(&k_trace_quad<Tri, Io>), 256)) {
+    Io qio = io;
+    if constexpr (std::is_same<Io, EyeFrame>::value) qio.group = kQuadRays;
+    k_trace_quad<Tri, Io><<<uint32_t(quads), 256, 0, stream>>>(nodes, tris, qio, n);
+    return hipGetLastError();
+  }
+  // One ray per lane (rays that arrive in screen order stay coherent within a
+  // wave, which a refilling kernel gives up).
+  const uint32_t blocks = uint32_t((n + 255) / 256);
+  if (blocks <= resident_grid(reinterpret_cast<const void*>(&k_trace_simple<false, false, kWalkDepth, Tri, Io>), 256)) {
+    k_trace_simple<false, false, kWalkDepth, Tri, Io><<<blocks, 256, 0, stream>>>(b.pairs, tris, io, n, nullptr,
+                                                                                  nullptr);
+    return hipGetLastError();
+  }
+  uint32_t* spill = nullptr;
+  hipError_t e = hipMallocAsync(reinterpret_cast<void**>(&spill),
+                                sizeof(uint32_t) * size_t(blocks) * 256 * (kWalkDepth - kSimpleLds), stream);
+  if (e != hipSuccess) return e;
+  k_trace_simple<false, false, kSimpleLds, Tri, Io><<<blocks, 256, 0, stream>>>(b.pairs, tris, io, n, nullptr, spill);
+  e = hipGetLastError();
+  const hipError_t f = hipFreeAsync(spill, stream);
+  return e != hipSuccess ? e : f;
 }
 
 template <class Tri>
 hipError_t trace_blas_with(const Blas& b, const TraceArgs& a, hipStream_t stream) {
   if (a.anyhit && !a.stats) return launch_persistent<true, true, Tri>(b, a, stream);
-  // Four lanes per ray while that fills at most half of the chip's waves
-  // (65,536 rays): the launch then lasts as long as its longest walks, which
-  // are shorter this way.  us a call on soup (400,000 triangles), hills with
-  // boxes (500,000) and sphere (80,000), random rays / camera, four lanes and
-  // one: 1,000 rays 121 and 150 / 83 and 103, 74 and 98; 65,000 rays 202 and
-  // 229 / 107 and 145, 93 and 113; 130,000 rays (every wave resident) 315 and
-  // 264 / 113 and 169, 87 and 92; 262,000 rays 471 and 387 / 168 and 200.
-  const WalkNodes nodes = walk_nodes(b);
-  const uint64_t quads = (a.n + kQuadRays - 1) / kQuadRays;
-  if (nodes.wide && !a.stats && 2 * quads <= resident_grid(reinterpret_cast<const void*>(&k_trace_quad<Tri>), 256)) {
-    const uint32_t blocks = uint32_t(quads);
-    k_trace_quad<Tri><<<blocks, 256, 0, stream>>>(nodes, tri_records<Tri>(b), a.rays, a.n, a.out, a.format,
-                                                  make_uint2(a.inst_id, a.geom_id));
-    return hipGetLastError();
-  }
-  // One ray per lane: the counting variant (the reference's order) and
-  // nearest hits (rays that arrive in screen order stay coherent within a
-  // wave, which the refilling kernel gives up).
+  const RayBatch io{a.rays, a.out, a.format, make_uint2(a.inst_id, a.geom_id)};
+  if (!a.stats) return trace_nearest<Tri>(b, io, a.n, stream);
+  // the counting variant, on the pairs
+  const TriPre* tris = tri_records<Tri>(b);
   const uint32_t blocks = uint32_t((a.n + 255) / 256);
-  if (blocks <= resident_grid(reinterpret_cast<const void*>(&k_trace_simple<false, false, kWalkDepth, Tri>), 256))
-    return launch_simple<kWalkDepth, Tri>(b, a, blocks, nullptr, stream);
-  uint32_t* spill = nullptr;
-  hipError_t e = hipMallocAsync(reinterpret_cast<void**>(&spill),
-                                sizeof(uint32_t) * size_t(blocks) * 256 * (kWalkDepth - kSimpleLds), stream);
-  if (e != hipSuccess) return e;
-  e = launch_simple<kSimpleLds, Tri>(b, a, blocks, spill, stream);
-  const hipError_t f = hipFreeAsync(spill, stream);
-  return e != hipSuccess ? e : f;
+  if (a.anyhit)
+    k_trace_simple<true, true, kWalkDepth, Tri><<<blocks, 256, 0, stream>>>(b.pairs, tris, io, a.n, a.stats, nullptr);
+  else
+    k_trace_simple<false, true, kWalkDepth, Tri><<<blocks, 256, 0, stream>>>(b.pairs, tris, io, a.n, a.stats, nullptr);
+  return hipGetLastError();
 }
 
 }  // namespace
@@ -429,6 +453,15 @@ uint32_t resident_grid(const void* kernel, int block) {
   std::lock_guard<std::mutex> lock(mu);
   cache.push_back(Entry{dev, kernel, block, grid});
   return grid;
+}
+
+hipError_t eye_frame(const Blas& b, bool watertight, const EyeCamera& cam, uint32_t width, uint32_t height,
+                     const EyePalette& pal, uint32_t* out_color, hipStream_t stream) {
+  const uint64_t n = uint64_t(width) * height;
+  if (n == 0) return hipSuccess;
+  if (watertight && !b.tris_wt) return hipErrorInvalidValue;
+  const EyeFrame io{cam, pal, width, height, out_color, 256u};
+  return watertight ? trace_nearest<WtTest>(b, io, n, stream) : trace_nearest<MtTest>(b, io, n, stream);
 }
 
 hipError_t trace_blas(const Blas& b, const TraceArgs& a, hipStream_t stream) {

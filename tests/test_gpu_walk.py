@@ -111,3 +111,30 @@ def test_refit_moves_the_walked_boxes(gpu_ctx):
     rays = rays_for(v * 1.5 + 0.25, 4000, 8400)
     same(trace(s, rays, "full"), trace(s, rays, "full", stats=True))
     s.close()
+
+
+@pytest.mark.parametrize("test", [H.TRI_MT, H.TRI_WATERTIGHT], ids=["mt", "wt"])
+@pytest.mark.parametrize("w,h", [(16, 8), (256, 256), (264, 256), (1032, 520)])
+def test_frame_in_one_launch_equals_its_parts(gpu_ctx, test, w, h):
+    import torch
+
+    v, f = W.eye_scene()
+    s = H.Scene(gpu_ctx)
+    s.add_instance(s.add_triangles(v, f))
+    s.set_triangle_test(test)
+    s.commit()
+    say(f"eye frame {w}x{h}")
+    cam, stream = W.eye_camera(w, h), torch.cuda.current_stream().cuda_stream
+    rays = torch.zeros((w * h, 8), dtype=torch.float32, device="cuda")
+    xy = torch.zeros(w * h, dtype=torch.int32, device="cuda")
+    image = torch.zeros((h, w), dtype=torch.int32, device="cuda")
+    gpu_ctx.eye_make_rays(*cam, w, h, rays, xy, stream=stream)
+    s.eye_render(*cam, w, h, W.EYE_PALETTE, image, stream=stream)
+    torch.cuda.synchronize()
+    prim = trace(s, rays.cpu().numpy(), "compact")["prim"]
+    px = xy.cpu().numpy().view(np.uint32)
+    want = np.zeros((h, w), np.uint32)
+    hit = prim != 0xFFFFFFFF
+    want[(px >> 16)[hit], (px & 0xFFFF)[hit]] = W.EYE_PALETTE[prim[hit] % W.EYE_PALETTE.size]
+    np.testing.assert_array_equal(image.cpu().numpy().view(np.uint32), want)
+    s.close()
