@@ -145,16 +145,7 @@ struct LdsStack {
 };
 constexpr int kShortStack = 16;  // LDS entries per lane in the persistent kernels
 
-// The logical block a workgroup works on, so that each XCD's L2 serves one
-// contiguous stretch of the rays.  The dispatcher hands workgroups to the
-// eight XCDs in turn (workgroup b to XCD b mod 8); XCD x gets the x-th
-// eighth of the logical blocks, in order.  A permutation of [0, n).
-constexpr uint32_t kXcds = 8;
-__device__ inline uint32_t xcd_block(uint32_t b, uint32_t n) {
-  const uint32_t per = n / kXcds, rem = n % kXcds;
-  const uint32_t x = b % kXcds, i = b / kXcds;
-  return x * per + (x < rem ? x : rem) + i;
-}
+constexpr uint32_t kXcds = 8;  // workgroup b runs on XCD b mod kXcds
 
 // Set bits of m in the lanes below this one (v_mbcnt_lo / v_mbcnt_hi).
 __device__ inline uint32_t lanes_below(uint64_t m) {

@@ -34,13 +34,17 @@ constexpr int kRefillAt4 = 40;
 // to global memory).  Deep, incoherent nearest-hit walks push often and
 // measured slower with spills, so BVH4 keeps its whole stack in LDS.
 constexpr int kSimpleLds4 = 48;
-// Nearest-hit batches of at least this many rays are sorted into coherent
-// waves before they are traced.  On 4,194,304 incoherent rays in a
-// 4,194,304-triangle soup the FP16 walk fetches 6 % fewer bytes from beyond
-// the L2 and takes 21.8 instead of 24.0 ms; a refilling persistent kernel
-// (wave-local ray pool, speculative while-while) was no faster there (24.8
-// ms unsorted, 23.3 sorted): the walk waits on memory, not on idle lanes.
+// Nearest-hit batches of at least this many rays on a tree (nodes and
+// triangles) of at least this many bytes are sorted into coherent waves before
+// they are traced.  A tree well inside the 256 MB MALL gains nothing that pays
+// for the sort: ms a call on FP16 nodes of the clustered tree, in the rays' own
+// order and sorted, random rays / camera rays: 1,048,576 rays in a
+// 1,000,000-triangle soup (70 MB) 1.55 and 1.52 / 0.82 and 1.06, over
+// 1,000,000 triangles of hills 0.64 and 0.81 / 0.29 and 0.63; 4,194,304 rays in
+// a 4,194,304-triangle soup (290 MB) 13.2 and 9.4 / 4.6 and 5.5, in a
+// 2,000,000-triangle soup (140 MB) 7.9 and 6.5 / 3.2 and 4.1.
 constexpr uint64_t kSortRaysMin4 = 1u << 20;
+constexpr uint64_t kSortTreeMin4 = 128u << 20;
 // The speculative any-hit kernels leave the node loop for the leaf phase once
 // this many lanes or fewer still look for a leaf (0 would wait for the last).
 constexpr uint32_t kLeafPhaseAt = 4;
@@ -151,28 +155,12 @@ __device__ inline void write_hit(void* out, uint64_t i, int format, uint2 ids, c
   }
 }
 
-// One ray per lane, the reference's order step by step (also the counting
-// variant: quads visited, triangles in visited leaves).
-template <bool kForceAny, bool kFp16, bool kStats, class Tri = MtTest>
-__global__ __launch_bounds__(kBlock4) void k_trace4_simple(const void* __restrict__ quads,
-                                                           const TriPre* __restrict__ tris,
-                                                           const Ray* __restrict__ rays, uint64_t n, void* out,
-                                                           int format, uint2 ids, uint32_t* __restrict__ stats,
-                                                           uint32_t* __restrict__ spill,
-                                                           const uint32_t* const* __restrict__ order_slot) {
-  __shared__ uint32_t stack_mem[kSimpleLds4 * kBlock4];
-  const uint32_t* __restrict__ order = order_slot ? *order_slot : nullptr;
-  // a sorted batch: each XCD takes one contiguous eighth of the sorted order,
-  // so its L2 serves rays of similar direction and origin (5 % faster on 4 M
-  // incoherent rays); rays in their own order keep the dispatch order, whose
-  // interleaving balances the XCDs over uneven screen regions
-  const uint64_t lane_id =
-      uint64_t(order ? xcd_block(blockIdx.x, gridDim.x) : blockIdx.x) * kBlock4 + threadIdx.x;
-  if (lane_id >= n) return;
-  // thread k traces ray order[k] when the batch was sorted into coherent waves
-  const uint64_t i = order ? uint64_t(order[lane_id]) : lane_id;
-  if (i >= n) return;
-  const ShortStack<kSimpleLds4, kBlock4> stk{stack_mem + threadIdx.x, spill + lane_id, gridDim.x * kBlock4};
+// The walk of ray i on one lane, the reference's order step by step (also the
+// counting variant: quads visited, triangles in visited leaves).
+template <bool kForceAny, bool kFp16, bool kStats, class Tri, class Stack>
+__device__ inline void trace4_one(const void* __restrict__ quads, const TriPre* __restrict__ tris,
+                                  const Ray* __restrict__ rays, uint64_t i, void* out, int format, uint2 ids,
+                                  uint32_t* __restrict__ stats, const Stack& stk) {
   const Ray r = rays[i];
   const float3 o = make_float3(r.pos_near.x, r.pos_near.y, r.pos_near.z);
   const float3 d = make_float3(r.dir_far.x, r.dir_far.y, r.dir_far.z);
@@ -220,6 +208,54 @@ __global__ __launch_bounds__(kBlock4) void k_trace4_simple(const void* __restric
     stats[2 * i + 1] = ntests;
   }
   write_hit<kForceAny>(out, i, format, ids, h);
+}
+
+// One ray per lane, in the rays' own order.
+template <bool kForceAny, bool kFp16, bool kStats, class Tri = MtTest>
+__global__ __launch_bounds__(kBlock4) void k_trace4_simple(const void* __restrict__ quads,
+                                                           const TriPre* __restrict__ tris,
+                                                           const Ray* __restrict__ rays, uint64_t n, void* out,
+                                                           int format, uint2 ids, uint32_t* __restrict__ stats,
+                                                           uint32_t* __restrict__ spill) {
+  __shared__ uint32_t stack_mem[kSimpleLds4 * kBlock4];
+  const uint64_t i = uint64_t(blockIdx.x) * kBlock4 + threadIdx.x;
+  if (i >= n) return;
+  const ShortStack<kSimpleLds4, kBlock4> stk{stack_mem + threadIdx.x, spill + i, gridDim.x * kBlock4};
+  trace4_one<kForceAny, kFp16, kStats, Tri>(quads, tris, rays, i, out, format, ids, stats, stk);
+}
+
+// Nearest hits of a sorted batch: lane k of a wave's 64 traces ray order[k] (k
+// itself when the order slot is null: the sort failed).  Bound by bytes from
+// beyond the L2, so each XCD works through one contiguous eighth of the order
+// and its L2 serves rays of nearby origins and similar directions; a wave takes
+// the next 64 rays of its XCD's eighth, then of the others', since the eighths
+// take unequal time (camera rays: a region of the screen each).
+template <bool kFp16, class Tri>
+__global__ __launch_bounds__(kBlock4) void k_trace4_sorted(const void* __restrict__ quads,
+                                                           const TriPre* __restrict__ tris,
+                                                           const Ray* __restrict__ rays, uint64_t n, void* out,
+                                                           int format, uint2 ids, uint32_t* __restrict__ spill,
+                                                           const uint32_t* const* __restrict__ order_slot,
+                                                           uint32_t* __restrict__ queue) {
+  __shared__ uint32_t stack_mem[kSimpleLds4 * kBlock4];
+  const uint32_t* __restrict__ order = *order_slot;
+  const ShortStack<kSimpleLds4, kBlock4> stk{stack_mem + threadIdx.x, spill + blockIdx.x * kBlock4 + threadIdx.x,
+                                             gridDim.x * kBlock4};
+  for (uint32_t tried = 0; tried < kXcds;) {
+    const uint32_t p = (blockIdx.x + tried) % kXcds;
+    const uint64_t lo = n * p / kXcds, hi = n * (p + 1) / kXcds;
+    uint32_t b = 0;
+    if (threadIdx.x == 0) b = atomicAdd(queue + p * kXcdQueueStride, uint32_t(kBlock4));
+    const uint64_t base = lo + uint64_t(__shfl(b, 0));
+    if (base >= hi) {
+      tried++;
+      continue;
+    }
+    const uint64_t k = base + threadIdx.x;
+    if (k < hi)
+      trace4_one<false, kFp16, false, Tri>(quads, tris, rays, order ? uint64_t(order[k]) : k, out, format, ids,
+                                           nullptr, stk);
+  }
 }
 
 // Persistent speculative any-hit over BVH4 nodes with ballot-based refill
@@ -586,12 +622,17 @@ hipError_t launch_any4(const Blas& b, Src src, uint64_t n, uint8_t* out, hipStre
   return e != hipSuccess ? e : f;
 }
 
-// Sort key of a ray for coherent waves: 7 bits of direction (the cube face of
+// Sort key of a ray for coherent waves: 12 bits of a Morton code of the origin
+// on a 16^3 grid over the scene box, then 7 bits of direction (the cube face of
 // the largest |d| component, 6 faces, times a 4x4 grid of the other two
-// components divided by it) above a 24-bit Morton code of the origin on a
-// 256^3 grid over the scene box (clamped).  Rays with similar directions and
-// nearby origins then share waves, so their node and triangle fetches hit the
-// same cache lines.  A NaN component lands in cell 0.
+// components divided by it), then the 12 further bits of the origin on a 256^3
+// grid (clamped).  The rays in flight on an XCD then start close to each other,
+// and those of a wave go the same way.  Direction bits in front make every wave
+// more alike but spread the rays in flight over the whole scene: 4,194,304
+// random rays in a 4,194,304-triangle soup take 12.0 ms with all 24 origin bits
+// below the direction, 10.1 with 15, 9.4 with 12, 9.9 with 9, 10.0 with none.
+// A NaN component lands in cell 0.
+constexpr uint32_t kKeyFineBits = 12;
 __device__ inline uint32_t spread8(uint32_t x) {
   x = (x | (x << 8)) & 0x0000F00Fu;
   x = (x | (x << 4)) & 0x000C30C3u;
@@ -624,19 +665,23 @@ __global__ __launch_bounds__(256) void k_ray_keys(const Ray* __restrict__ rays, 
   const uint32_t cx = uint32_t(fminf(fmaxf((r.pos_near.x - lo.x) * scale.x, 0.0f), 255.0f));
   const uint32_t cy = uint32_t(fminf(fmaxf((r.pos_near.y - lo.y) * scale.y, 0.0f), 255.0f));
   const uint32_t cz = uint32_t(fminf(fmaxf((r.pos_near.z - lo.z) * scale.z, 0.0f), 255.0f));
-  keys[i] = ((face * 16u + cp * 4u + cq) << 24) | spread8(cx) | (spread8(cy) << 1) | (spread8(cz) << 2);
+  const uint32_t dir = face * 16u + cp * 4u + cq, org = spread8(cx) | (spread8(cy) << 1) | (spread8(cz) << 2);
+  keys[i] = ((org >> kKeyFineBits) << (kKeyFineBits + 7)) | (dir << kKeyFineBits) |
+            (org & ((1u << kKeyFineBits) - 1u));
   ids[i] = i;
 }
 
 // The order the trace kernel reads: the sorted one, or none (unsorted) when
 // the sort failed (its look-back gave up: *err != 0) and left it incomplete.
-__global__ void k_order_or_null(const uint32_t* __restrict__ err, const uint32_t* order, const uint32_t** slot) {
-  *slot = (*err == 0u) ? order : nullptr;
+// Also clears the trace's ray queues.
+__global__ void k_order_or_null(const uint32_t* __restrict__ err, const uint32_t* order, const uint32_t** slot,
+                                uint32_t* __restrict__ queue) {
+  queue[threadIdx.x] = 0u;
+  if (threadIdx.x == 0) *slot = (*err == 0u) ? order : nullptr;
 }
 
 template <bool kFp16, class Tri>
-hipError_t launch_simple4(const Blas& b, const TraceArgs& a, const uint32_t* const* order_slot,
-                          hipStream_t stream) {
+hipError_t launch_simple4(const Blas& b, const TraceArgs& a, hipStream_t stream) {
   if (!a.anyhit && !a.stats && takes_quads(reinterpret_cast<const void*>(&k_trace4_quad<kFp16, Tri>), a.n,
                                              kQuadShareNearest)) {
     k_trace4_quad<kFp16, Tri><<<uint32_t((a.n + kQuadRays4 - 1) / kQuadRays4), 256, 0, stream>>>(
@@ -659,41 +704,47 @@ hipError_t launch_simple4(const Blas& b, const TraceArgs& a, const uint32_t* con
   if (a.anyhit) {
     if (a.stats)
       k_trace4_simple<true, kFp16, true, Tri><<<blocks, kBlock4, 0, stream>>>(q, tris, a.rays, a.n, a.out, a.format,
-                                                                             ids, a.stats, spill, nullptr);
+                                                                             ids, a.stats, spill);
     else
       k_trace4_simple<true, kFp16, false, Tri><<<blocks, kBlock4, 0, stream>>>(q, tris, a.rays, a.n, a.out, a.format,
-                                                                              ids, nullptr, spill, nullptr);
+                                                                              ids, nullptr, spill);
   } else {
     if (a.stats)
       k_trace4_simple<false, kFp16, true, Tri><<<blocks, kBlock4, 0, stream>>>(q, tris, a.rays, a.n, a.out, a.format,
-                                                                              ids, a.stats, spill, nullptr);
+                                                                              ids, a.stats, spill);
     else
       k_trace4_simple<false, kFp16, false, Tri><<<blocks, kBlock4, 0, stream>>>(q, tris, a.rays, a.n, a.out,
-                                                                               a.format, ids, nullptr, spill, order_slot);
+                                                                               a.format, ids, nullptr, spill);
   }
   e = hipGetLastError();
   const hipError_t f = spill ? hipFreeAsync(spill, stream) : hipSuccess;
   return e != hipSuccess ? e : f;
 }
 
-// Nearest hits of a large batch: the rays are sorted into coherent waves
-// first (k_ray_keys, then the onesweep radix sort of the engine's builder),
-// and each thread traces the ray the order gives it; the answers land at the
-// rays' own indices, so the output is what an unsorted trace writes.
+// Nearest hits of a large batch on a large tree: the rays are sorted into
+// coherent waves first (k_ray_keys, then the onesweep radix sort of the
+// engine's builder), and each lane traces the ray the order gives it; the
+// answers land at the rays' own indices, so the output is what an unsorted
+// trace writes.
 template <bool kFp16, class Tri>
 hipError_t launch_nearest4_sorted(const Blas& b, const TraceArgs& a, hipStream_t stream) {
   const uint64_t n = a.n;
   const size_t sort_words = radix_sort_scratch_words(n, 4);
-  // keys, ids (twice), radix scratch, the error word and the order slot
-  const size_t words = 4 * n + sort_words + 64;
+  const uint32_t grid = uint32_t(std::min<uint64_t>(
+      resident_grid(reinterpret_cast<const void*>(&k_trace4_sorted<kFp16, Tri>), kBlock4), (n + kBlock4 - 1) / kBlock4));
+  // the order slot and the error word, the queues, keys and ids (twice), radix
+  // scratch and the stack entries beyond the LDS part of every lane
+  const size_t spill_words = size_t(grid) * kBlock4 * (kStackDepth4 - kSimpleLds4);
+  const size_t words = 64 + kXcdQueueWords + 4 * n + sort_words + spill_words;
   uint32_t* base = nullptr;
   hipError_t e = hipMallocAsync(reinterpret_cast<void**>(&base), sizeof(uint32_t) * words, stream);
   if (e != hipSuccess) return e;
   // base[0..1]: the order slot (8-byte aligned), base[2]: the sort's error word
   const uint32_t** slot = reinterpret_cast<const uint32_t**>(base);
   uint32_t* err = base + 2;
-  uint32_t *ka = base + 64, *va = ka + n, *kb = ka + 2 * n, *vb = ka + 3 * n;
-  uint32_t* scratch = ka + 4 * n;
+  uint32_t* queue = base + 64;
+  uint32_t *ka = queue + kXcdQueueWords, *va = ka + n, *kb = ka + 2 * n, *vb = ka + 3 * n;
+  uint32_t *scratch = ka + 4 * n, *spill = scratch + sort_words;
   const float3 lo = make_float3(b.box[0], b.box[1], b.box[2]);
   const float ex = b.box[4] - b.box[0], ey = b.box[5] - b.box[1], ez = b.box[6] - b.box[2];
   const float3 scale = make_float3(ex > 0.f ? 256.f / ex : 0.f, ey > 0.f ? 256.f / ey : 0.f, ez > 0.f ? 256.f / ez : 0.f);
@@ -705,10 +756,12 @@ hipError_t launch_nearest4_sorted(const Blas& b, const TraceArgs& a, hipStream_t
   if (e == hipSuccess) e = radix_sort(ka, va, kb, vb, n, 0, 4, scratch, err, stream);
   const uint32_t* order = va;  // four passes: the sorted pairs end in (ka, va)
   if (e == hipSuccess) {
-    k_order_or_null<<<1, 1, 0, stream>>>(err, order, slot);
+    k_order_or_null<<<1, kXcdQueueWords, 0, stream>>>(err, order, slot, queue);
+    k_trace4_sorted<kFp16, Tri><<<grid, kBlock4, 0, stream>>>(
+        kFp16 ? static_cast<const void*>(b.quads16) : b.quads32, tri_records<Tri>(b), a.rays, n, a.out, a.format,
+        make_uint2(a.inst_id, a.geom_id), spill, slot, queue);
     e = hipGetLastError();
   }
-  if (e == hipSuccess) e = launch_simple4<kFp16, Tri>(b, a, slot, stream);
   const hipError_t f = hipFreeAsync(base, stream);
   return e != hipSuccess ? e : f;
 }
@@ -721,9 +774,10 @@ hipError_t trace_blas4_with(const Blas& b, const TraceArgs& a, bool fp16, hipStr
     return fp16 ? launch_any4<true, StoredRays, Tri>(b, src, a.n, out, stream, a.workspace, a.workspace_words)
                 : launch_any4<false, StoredRays, Tri>(b, src, a.n, out, stream, a.workspace, a.workspace_words);
   }
-  if (!a.stats && !a.anyhit && a.n >= kSortRaysMin4)
+  const uint64_t tree = b.nquads * (fp16 ? sizeof(Quad16) : sizeof(Quad32)) + b.ntris * uint64_t(sizeof(TriPre));
+  if (!a.stats && !a.anyhit && a.n >= kSortRaysMin4 && tree >= kSortTreeMin4)
     return fp16 ? launch_nearest4_sorted<true, Tri>(b, a, stream) : launch_nearest4_sorted<false, Tri>(b, a, stream);
-  return fp16 ? launch_simple4<true, Tri>(b, a, nullptr, stream) : launch_simple4<false, Tri>(b, a, nullptr, stream);
+  return fp16 ? launch_simple4<true, Tri>(b, a, stream) : launch_simple4<false, Tri>(b, a, stream);
 }
 
 }  // namespace

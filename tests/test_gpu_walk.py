@@ -138,3 +138,27 @@ def test_frame_in_one_launch_equals_its_parts(gpu_ctx, test, w, h):
     want[(px >> 16)[hit], (px & 0xFFFF)[hit]] = W.EYE_PALETTE[prim[hit] % W.EYE_PALETTE.size]
     np.testing.assert_array_equal(image.cpu().numpy().view(np.uint32), want)
     s.close()
+
+
+@pytest.mark.parametrize("layout", [H.LAYOUT_BVH4, H.LAYOUT_BVH4_FP16], ids=["fp32", "fp16"])
+def test_sorted_batch_equals_its_parts(gpu_ctx, layout):
+    """2^20 rays or more on a tree of 128 MB or more are traced in sorted order, under either triangle test."""
+    rng = np.random.default_rng(7)
+    n = 2_200_000
+    v = (rng.random((n, 1, 3)) + 0.02 * (rng.random((n, 3, 3)) - 0.5)).reshape(-1, 3).astype(np.float32)
+    f = np.arange(3 * n, dtype=np.uint32).reshape(-1, 3)
+    s = H.Scene(gpu_ctx)
+    s.add_instance(s.add_triangles(v, f))
+    rays = W.incoherent_rays((1 << 20) + 3, stream=W.STREAM_TEST)
+    rays[5::1001, 7] = -0.5
+    rays[6::1003, 4] = np.nan
+    for test in (H.TRI_MT, H.TRI_WATERTIGHT):
+        s.set_triangle_test(test)
+        s.commit(layout=layout)
+        say(f"sorted batch layout {layout} test {test}")
+        whole = trace(s, rays, "full")
+        for lo, hi in ((0, 1000), (600_000, (1 << 20) + 3)):
+            part = trace(s, rays[lo:hi], "full")
+            for k in ("t", "prim", "u", "v"):
+                np.testing.assert_array_equal(part[k].view(np.uint32), whole[k][lo:hi].view(np.uint32))
+    s.close()
