@@ -158,8 +158,8 @@ __device__ inline bool walk_quad_step(const WideNode* __restrict__ W, const TriP
     const bool first = hg & !((og < eg) | ((og == eg) & ((l & 1u) != 0u)));
     // references are never 0: the root is nobody's child, a leaf has kLeafBit
     const uint32_t next = quad_or(first ? ref : 0u);
-    const uint32_t far_grand = quad_or(hg & !first ? ref : 0u);
-    uint32_t far_child = hc & !nearer ? child : 0u;
+    const uint32_t far_grand = quad_or((hg & !first) ? ref : 0u);
+    uint32_t far_child = (hc & !nearer) ? child : 0u;
     far_child |= quad_x2(far_child);
     const bool on = next != 0u, deferred = far_child != 0u, deferred2 = far_grand != 0u;
     cur = on ? next : (deferred ? far_child : popped);

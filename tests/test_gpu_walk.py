@@ -7,6 +7,7 @@ import heavyrt_amd as H
 from gpu_util import make_scene, say, trace
 from heavyrt_amd import workloads as W
 from oracle import oracle as O
+from test_gpu_bvh4 import oracle_any_tree
 from test_gpu_parity import rays_for
 
 pytestmark = pytest.mark.gpu
@@ -161,4 +162,19 @@ def test_sorted_batch_equals_its_parts(gpu_ctx, layout):
             part = trace(s, rays[lo:hi], "full")
             for k in ("t", "prim", "u", "v"):
                 np.testing.assert_array_equal(part[k].view(np.uint32), whole[k][lo:hi].view(np.uint32))
+    s.close()
+
+
+@pytest.mark.parametrize("ntris", [3, 255, 4096, 4097, 5000, 70_000])
+def test_clustered_hierarchy_at_round_edges(gpu_ctx, ntris):
+    """The clustering's two forms (a workgroup up to 4,096 clusters, tiles of 256 above) build the oracle's nodes."""
+    v, f = W.soup(ntris, stream=W.STREAM_TEST + 1)
+    s = H.Scene(gpu_ctx, keep_build_arrays=True)
+    s.add_instance(s.add_triangles(v, f))
+    s.commit(layout=H.LAYOUT_PLOC)
+    say(f"clustering {ntris}")
+    ob, clustered = oracle_any_tree(v, f)
+    sizes = s.dump(0, H.DUMP_ANY_TREE | H.DUMP_SIZES)
+    assert (int(sizes[1]), int(sizes[5])) == (ob.leaves, int(clustered))
+    np.testing.assert_array_equal(s.dump(0, H.DUMP_ANY_TREE | H.DUMP_LR_NODES), ob.lr_nodes())
     s.close()
