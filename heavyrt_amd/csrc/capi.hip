@@ -603,11 +603,16 @@ hrt_status hrt_commit(hrt_scene* s, int quality, int layout) {
       }
     }
   }
-  // nearest hits on the BVH2 trees walk two levels a fetch
+  // nearest hits on the BVH2 trees walk two levels a fetch; the records are
+  // whole before this returns, as a trace may follow on any stream
   if (!single || layout == HRT_LAYOUT_BVH2 || layout == HRT_LAYOUT_AUTO || layout == HRT_LAYOUT_AUTO_FP16) {
-    for (const Instance& in : s->instances)
-      if ((e = hrt::blas_build_wide(s->geoms[in.geom], s->ctx->stream)) != hipSuccess)
-        return fail_hip(e, "nearest-hit nodes");
+    bool made = false;
+    for (const Instance& in : s->instances) {
+      hrt::Blas& b = s->geoms[in.geom];
+      made |= !b.wide_made;
+      if ((e = hrt::blas_build_wide(b, s->ctx->stream)) != hipSuccess) return fail_hip(e, "nearest-hit nodes");
+    }
+    if (made && (e = hipStreamSynchronize(s->ctx->stream)) != hipSuccess) return fail_hip(e, "nearest-hit nodes");
   }
   if (wt) {
     hrt::Blas& b = s->geoms[s->instances[0].geom];

@@ -178,3 +178,26 @@ def test_clustered_hierarchy_at_round_edges(gpu_ctx, ntris):
     assert (int(sizes[1]), int(sizes[5])) == (ob.leaves, int(clustered))
     np.testing.assert_array_equal(s.dump(0, H.DUMP_ANY_TREE | H.DUMP_LR_NODES), ob.lr_nodes())
     s.close()
+
+
+@pytest.mark.parametrize("layout", [H.LAYOUT_BVH2, H.LAYOUT_AUTO_FP16], ids=["bvh2", "auto_fp16"])
+def test_commit_is_whole_for_a_trace_on_another_stream(gpu_ctx, layout):
+    """The rays wait on the device and the stream is idle: the trace starts as soon as the commit has returned."""
+    import torch
+    v, f = W.soup(400_000, stream=W.STREAM_TEST)
+    rays = torch.from_numpy(rays_for(v, 4000, 8500)).cuda()
+    out = [torch.zeros((4000, 8), dtype=torch.int32, device="cuda") for _ in range(2)]
+    other = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    s = H.Scene(gpu_ctx)
+    s.add_instance(s.add_triangles(v, f))
+    for scale in (1.0, 1.25):
+        if scale != 1.0:
+            s.update_triangles(0, (v * np.float32(scale)).astype(np.float32), quality=3)
+        s.commit(layout=layout)
+        s.trace_nearest(rays, 4000, out[0], H.HIT_FULL, stream=other.cuda_stream)
+        torch.cuda.synchronize()
+        s.trace_nearest(rays, 4000, out[1], H.HIT_FULL, stream=other.cuda_stream)
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(out[0].cpu().numpy(), out[1].cpu().numpy())
+    s.close()
