@@ -108,19 +108,6 @@ void instance_box(const float* gbox8, const float* m, float* out8) {
   }
 }
 
-// Float4 copy of caller vertices with w = 1 (BVH2CommonRT_host.cpp:79-84).
-std::vector<float> repack_vertices(const float* vpos, size_t nVert, size_t vStrideBytes) {
-  const size_t stride = vStrideBytes / 4;
-  std::vector<float> v4(4 * nVert);
-  for (size_t i = 0; i < nVert; i++) {
-    v4[4 * i + 0] = vpos[i * stride + 0];
-    v4[4 * i + 1] = vpos[i * stride + 1];
-    v4[4 * i + 2] = vpos[i * stride + 2];
-    v4[4 * i + 3] = 1.0f;
-  }
-  return v4;
-}
-
 bool is_identity(const float* m) {
   for (int c = 0; c < 4; c++)
     for (int r = 0; r < 4; r++)
@@ -132,6 +119,7 @@ bool is_identity(const float* m) {
 
 struct hrt_scene {
   hrt_ctx* ctx = nullptr;
+  std::shared_ptr<hrt::DevCache> mem;  // the context's
   std::vector<hrt::Blas> geoms;
   std::vector<Instance> instances;
   bool committed = false;
@@ -187,7 +175,10 @@ void free_tlas(hrt_scene* s) {
     (void)hipStreamSynchronize(s->ctx->stream);
   }
   hrt::blas_free(s->tlas);
-  if (s->inst_dev) (void)hipFree(s->inst_dev);
+  if (s->inst_dev) {
+    s->mem->wait();
+    s->mem->free(s->inst_dev);
+  }
   s->inst_dev = nullptr;
   s->two_level = false;
 }
@@ -210,8 +201,8 @@ hrt_status build_tlas(hrt_scene* s) {
     r.inst = uint32_t(i);
   }
   hipStream_t hs = s->ctx->stream;
-  hipError_t e = hrt::blas_alloc(s->tlas, uint32_t(2 * n), uint32_t(n), s->keep_debug);
-  if (e == hipSuccess) e = hipMalloc(&s->inst_dev, 2 * n * sizeof(hrt::InstDev));
+  hipError_t e = hrt::blas_alloc(s->tlas, s->mem.get(), uint32_t(2 * n), uint32_t(n), s->keep_debug);
+  if (e == hipSuccess) e = s->mem->alloc(&s->inst_dev, 2 * n * sizeof(hrt::InstDev));
   if (e == hipSuccess) e = hipMemcpyAsync(s->tlas.verts, boxes.data(), 4 * boxes.size(), hipMemcpyHostToDevice, hs);
   if (e == hipSuccess)
     e = hipMemcpyAsync(s->inst_dev, recs.data(), n * sizeof(hrt::InstDev), hipMemcpyHostToDevice, hs);
@@ -226,6 +217,32 @@ hrt_status build_tlas(hrt_scene* s) {
   }
   s->two_level = true;
   return HRT_OK;
+}
+
+// Caller vertices as float4 with w = 1 (BVH2CommonRT_host.cpp:79-84) in `out`.
+// Records of at most kRawStride bytes go up as they are and are expanded on the
+// device (13 MB of packed ones: 0.4 ms; the float4 copy on the host that went
+// up before cost 0.9 ms more, and 11 at 50 MB); wider ones are packed on the
+// host first.  *raw is device scratch that the
+// caller gives back once the stream has been waited for.
+constexpr size_t kRawStride = 32;
+hipError_t upload_vertices(hrt_ctx* ctx, const float* vpos, size_t nVert, size_t vStrideBytes, float4* out,
+                           void** raw) {
+  std::vector<float> packed;
+  if (vStrideBytes > kRawStride) {
+    packed.resize(3 * nVert);
+    for (size_t i = 0; i < nVert; i++) std::memcpy(&packed[3 * i], vpos + i * (vStrideBytes / 4), 12);
+    vpos = packed.data();
+    vStrideBytes = 12;
+  }
+  const size_t bytes = (nVert - 1) * vStrideBytes + 12;  // the last record may end after its position
+  hipError_t e = ctx->mem->alloc(raw, bytes);
+  if (e == hipSuccess) e = hipMemcpyAsync(*raw, vpos, bytes, hipMemcpyHostToDevice, ctx->stream);
+  if (e == hipSuccess && !packed.empty()) e = hipStreamSynchronize(ctx->stream);  // `packed` ends here
+  if (e == hipSuccess)
+    e = hrt::expand_vertices(static_cast<const float*>(*raw), uint32_t(vStrideBytes / 4), uint32_t(nVert), out,
+                             ctx->stream);
+  return e;
 }
 
 hrt_status select_blas(hrt_scene* s, const hrt::Blas** out, uint32_t* inst) {
@@ -344,6 +361,12 @@ hrt_status hrt_init(int device, hrt_ctx** out) {
   hrt_ctx* c = new (std::nothrow) hrt_ctx();
   if (!c) return fail(HRT_ERR_OUT_OF_MEMORY, "host allocation failed");
   c->device = device;
+  try {
+    c->mem = std::make_shared<hrt::DevCache>(device);
+  } catch (const std::bad_alloc&) {
+    delete c;
+    return fail(HRT_ERR_OUT_OF_MEMORY, "host allocation failed");
+  }
   if ((e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking)) != hipSuccess) {
     delete c;
     return fail_hip(e, "hipStreamCreate");
@@ -375,6 +398,7 @@ hrt_status hrt_scene_create(hrt_ctx* ctx, hrt_scene** out) {
   hrt_scene* s = new (std::nothrow) hrt_scene();
   if (!s) return fail(HRT_ERR_OUT_OF_MEMORY, "host allocation failed");
   s->ctx = ctx;
+  s->mem = ctx->mem;
   *out = s;
   return HRT_OK;
 }
@@ -433,24 +457,44 @@ hrt_status hrt_add_triangles(hrt_scene* s, const float* vpos, size_t nVert, size
   if (ntris == 0) return fail(HRT_ERR_INVALID_ARG, "need at least one triangle");
   if (ntris > 0x00FFFFFFu) return fail(HRT_ERR_INVALID_ARG, "more than 16777215 triangles in one geometry (24-bit leaf start)");
   if (nVert == 0 || nVert > 0xFFFFFFFFull) return fail(HRT_ERR_INVALID_ARG, "bad vertex count");
-  for (size_t i = 0; i < 3 * ntris; i++)
-    if (idx[i] >= nVert) return fail(HRT_ERR_INVALID_ARG, "index out of range");
-
-  const std::vector<float> v4 = repack_vertices(vpos, nVert, vStrideBytes);
+  // Indices are checked before anything follows them: on the host while that
+  // is cheaper than a pass over the uploaded ones and a wait (about 20 us).
+  const bool check_here = ntris < 16384;
+  if (check_here) {
+    for (size_t i = 0; i < 3 * ntris; i++)
+      if (idx[i] >= nVert) return fail(HRT_ERR_INVALID_ARG, "index out of range");
+  }
   hipError_t e = hipSetDevice(s->ctx->device);
   if (e != hipSuccess) return fail_hip(e, "hipSetDevice");
   hrt::Blas b;
-  if ((e = hrt::blas_alloc(b, uint32_t(nVert), uint32_t(ntris), s->keep_debug)) != hipSuccess) {
+  if ((e = hrt::blas_alloc(b, s->mem.get(), uint32_t(nVert), uint32_t(ntris), s->keep_debug)) != hipSuccess) {
     hrt::blas_free(b);
     return fail_hip(e, "AddGeom_Triangles3f allocation");
   }
   hipStream_t hs = s->ctx->stream;
-  e = hipMemcpyAsync(b.verts, v4.data(), 16 * nVert, hipMemcpyHostToDevice, hs);
-  if (e == hipSuccess) e = hipMemcpyAsync(b.idx, idx, 12 * ntris, hipMemcpyHostToDevice, hs);
-  if (e == hipSuccess) e = hrt::blas_build(b, hs);
+  void* raw = nullptr;
+  bool in_range = true;
+  e = hipMemcpyAsync(b.idx, idx, 12 * ntris, hipMemcpyHostToDevice, hs);
+  if (e == hipSuccess) e = upload_vertices(s->ctx, vpos, nVert, vStrideBytes, b.verts, &raw);
+  if (e == hipSuccess && !check_here) {
+    hrt::Readback back(s->mem.get());
+    e = hrt::largest_index(b.idx, 3 * ntris, b.meta, hs);
+    if (e == hipSuccess) e = back.read(0, b.meta, 1, hs);
+    if (e == hipSuccess) e = hipStreamSynchronize(hs);
+    in_range = e != hipSuccess || back.words()[0] < nVert;
+  }
+  if (e == hipSuccess && in_range) e = hrt::blas_build(b, hs);
+  if (raw) {
+    (void)hipStreamSynchronize(hs);
+    s->mem->free(raw);
+  }
   if (e != hipSuccess) {
     hrt::blas_free(b);
     return fail_hip(e, "LBVH build");
+  }
+  if (!in_range) {
+    hrt::blas_free(b);
+    return fail(HRT_ERR_INVALID_ARG, "index out of range");
   }
   if (b.max_run > 127) {
     hrt::blas_free(b);
@@ -493,10 +537,10 @@ hrt_status hrt_update_triangles(hrt_scene* s, uint32_t geomId, const float* vpos
     for (size_t i = 0; i < 3 * ntris; i++)
       if (idx[i] >= nVert) return fail(HRT_ERR_INVALID_ARG, "index out of range");
   }
-  const std::vector<float> v4 = repack_vertices(vpos, nVert, vStrideBytes);
   hipError_t e = hipSetDevice(s->ctx->device);
   if (e != hipSuccess) return fail_hip(e, "hipSetDevice");
   hipStream_t hs = s->ctx->stream;
+  void* raw = nullptr;
   s->committed = false;
   free_tlas(s);
   if (quality == HRT_BUILD_REFIT) {
@@ -510,9 +554,11 @@ hrt_status hrt_update_triangles(hrt_scene* s, uint32_t geomId, const float* vpos
         if (x >= nVert) return fail(HRT_ERR_INVALID_ARG, "kept indices reach past the new vertex count");
     }
     b.nverts = uint32_t(nVert);
-    e = hipMemcpyAsync(b.verts, v4.data(), 16 * nVert, hipMemcpyHostToDevice, hs);
+    e = upload_vertices(s->ctx, vpos, nVert, vStrideBytes, b.verts, &raw);
     if (e == hipSuccess && idx) e = hipMemcpyAsync(b.idx, idx, 12 * ntris, hipMemcpyHostToDevice, hs);
     if (e == hipSuccess) e = hrt::blas_refit(b, hs);
+    if (e != hipSuccess) (void)hipStreamSynchronize(hs);
+    s->mem->free(raw);
     if (e != hipSuccess) return fail_hip(e, "refit");
     return HRT_OK;
   }
@@ -527,10 +573,12 @@ hrt_status hrt_update_triangles(hrt_scene* s, uint32_t geomId, const float* vpos
     idx = kept.data();
   }
   hrt::Blas nb;
-  if ((e = hrt::blas_alloc(nb, uint32_t(nVert), uint32_t(ntris), s->keep_debug)) == hipSuccess) {
-    e = hipMemcpyAsync(nb.verts, v4.data(), 16 * nVert, hipMemcpyHostToDevice, hs);
+  if ((e = hrt::blas_alloc(nb, s->mem.get(), uint32_t(nVert), uint32_t(ntris), s->keep_debug)) == hipSuccess) {
+    e = upload_vertices(s->ctx, vpos, nVert, vStrideBytes, nb.verts, &raw);
     if (e == hipSuccess) e = hipMemcpyAsync(nb.idx, idx, 12 * ntris, hipMemcpyHostToDevice, hs);
     if (e == hipSuccess) e = hrt::blas_build(nb, hs);
+    if (e != hipSuccess) (void)hipStreamSynchronize(hs);
+    s->mem->free(raw);
   }
   if (e != hipSuccess) {
     hrt::blas_free(nb);
@@ -1178,7 +1226,7 @@ const char* check_tree_record(const uint32_t head[8], const TreeSpans& t, bool a
 // Reads one tree record into b (allocated here).  The record is checked on
 // the host before anything is uploaded.  Returns HRT_OK or an error status
 // with the message set.
-hrt_status read_tree(SnapReader& r, hrt::Blas& b, int depth) {
+hrt_status read_tree(SnapReader& r, hrt_ctx* ctx, hrt::Blas& b, int depth) {
   uint32_t head[8];
   float box[8], zs[4];
   if (!r.val(head) || !r.val(box) || !r.val(zs)) return fail(HRT_ERR_INVALID_ARG, "snapshot is truncated");
@@ -1217,15 +1265,15 @@ hrt_status read_tree(SnapReader& r, hrt::Blas& b, int depth) {
                         reinterpret_cast<const hrt::Quad16*>(at[11])};
   if (const char* bad = check_tree_record(head, spans, depth > 0))
     return fail(HRT_ERR_INVALID_ARG, std::string("snapshot holds an invalid tree record: ") + bad);
-  hipError_t e = hrt::blas_alloc(b, nverts, ntris, false);
+  hipError_t e = hrt::blas_alloc(b, ctx->mem.get(), nverts, ntris, false);
   if (e != hipSuccess) return fail_hip(e, "snapshot allocation");
   b.leaves = head[2];
   b.max_run = head[3];
   b.clustered = head[6] != 0;
   std::memcpy(b.box, box, sizeof(b.box));
   std::memcpy(b.zscale, zs, sizeof(b.zscale));
-  if (nq && ((e = hipMalloc(&b.quads32, sizeof(hrt::Quad32) * nq)) != hipSuccess ||
-             (e = hipMalloc(&b.quads16, sizeof(hrt::Quad16) * nq)) != hipSuccess))
+  if (nq && ((e = ctx->mem->alloc(&b.quads32, sizeof(hrt::Quad32) * nq)) != hipSuccess ||
+             (e = ctx->mem->alloc(&b.quads16, sizeof(hrt::Quad16) * nq)) != hipSuccess))
     return fail_hip(e, "snapshot allocation");
   b.nquads = head[4];
   void* dst[kArrays] = {b.verts, b.idx,         b.pairs,      b.tris, b.perm,    b.parent,
@@ -1237,7 +1285,7 @@ hrt_status read_tree(SnapReader& r, hrt::Blas& b, int depth) {
   if (head[7]) {
     b.any_tree = new (std::nothrow) hrt::Blas();
     if (!b.any_tree) return fail(HRT_ERR_OUT_OF_MEMORY, "host allocation failed");
-    return read_tree(r, *b.any_tree, depth + 1);
+    return read_tree(r, ctx, *b.any_tree, depth + 1);
   }
   return HRT_OK;
 }
@@ -1298,7 +1346,7 @@ hrt_status hrt_scene_deserialize(hrt_ctx* ctx, const void* data, size_t size, hr
   }
   for (uint32_t g = 0; st == HRT_OK && g < ngeom; g++) {
     s->geoms.emplace_back();
-    st = read_tree(r, s->geoms.back(), 0);
+    st = read_tree(r, ctx, s->geoms.back(), 0);
   }
   for (uint32_t i = 0; st == HRT_OK && i < ninst; i++) {
     uint32_t geom = 0;

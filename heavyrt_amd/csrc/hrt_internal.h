@@ -5,17 +5,89 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <map>
+#include <memory>
+#include <mutex>
 #include <string>
 #include <type_traits>
+#include <unordered_map>
 #include <vector>
 
 #include "../../include/hrt.h"
 #include "hrt_device.h"
 
-// One device and one default-priority stream (hrt_init).
+namespace hrt {
+
+// Device memory of one context's trees and build scratch, kept for reuse when
+// it is given back (a 128 MB hipMalloc takes 53 us and its hipFree 265 us, and
+// a build has a dozen arrays: a million triangles loaded and committed took
+// 10.3 ms, and 2.8 with this and the geometry expanded on the device), and pinned words for small readbacks (12 us with
+// the wait, 21 us through pageable memory).  At most kMaxIdle bytes are kept
+// idle, for blocks of up to a quarter less; trim gives them all back (when an allocation fails, and at the end).
+// Safe with several threads.
+class DevCache {
+ public:
+  explicit DevCache(int device) : device_(device) {}
+  DevCache(const DevCache&) = delete;
+  DevCache& operator=(const DevCache&) = delete;
+  ~DevCache();
+  template <class T>
+  hipError_t alloc(T** p, size_t bytes) {
+    return alloc_bytes(reinterpret_cast<void**>(p), bytes);
+  }
+  // For memory that nothing on the device uses any more (null is fine).
+  void free(void* p);
+  // Waits for the whole device, whatever the caller's current one is.
+  void wait();
+  void trim();
+  // kPinnedWords words, or null when all are taken.
+  static constexpr size_t kPinnedWords = 32;
+  uint32_t* pinned_get();
+  void pinned_put(uint32_t* w);
+
+ private:
+  static constexpr size_t kMaxIdle = size_t(1) << 30;
+  static constexpr int kPinnedSlots = 16;
+  hipError_t alloc_bytes(void** p, size_t bytes);
+  bool note(void* p, size_t size);
+  const int device_;
+  std::mutex mu_;
+  std::unordered_map<void*, size_t> live_;
+  std::multimap<size_t, void*> idle_;
+  size_t idle_bytes_ = 0;
+  uint32_t* pinned_ = nullptr;
+  uint32_t pinned_taken_ = 0;  // a bit per slot
+};
+
+// Words copied back from the device into pinned memory where there is some.
+class Readback {
+ public:
+  explicit Readback(DevCache* mem) : mem_(mem), pinned_(mem->pinned_get()) {}
+  ~Readback() {
+    if (pinned_) mem_->pinned_put(pinned_);
+  }
+  Readback(const Readback&) = delete;
+  Readback& operator=(const Readback&) = delete;
+  uint32_t* words() { return pinned_ ? pinned_ : local_; }
+  // Enqueues the copy of n words to words() + at; valid after a wait.
+  hipError_t read(size_t at, const void* dev, size_t n, hipStream_t s) {
+    return hipMemcpyAsync(words() + at, dev, 4 * n, hipMemcpyDeviceToHost, s);
+  }
+
+ private:
+  DevCache* mem_;
+  uint32_t* pinned_;
+  uint32_t local_[DevCache::kPinnedWords];
+};
+
+}  // namespace hrt
+
+// One device, one default-priority stream and the memory of its trees, which
+// the scenes share (hrt_init).
 struct hrt_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
+  std::shared_ptr<hrt::DevCache> mem;
 };
 
 namespace hrt {
@@ -44,12 +116,14 @@ int scene_device(const hrt_scene* s);
 
 // Device buffers of one bottom-level structure (one geometry).
 struct Blas {
+  DevCache* mem = nullptr;    // where every array below comes from (blas_alloc)
   uint32_t ntris = 0;
   uint32_t nverts = 0;
   uint32_t leaves = 0;        // unique Morton codes (valid after build)
   uint32_t max_run = 0;       // longest run of equal codes (leaf size)
   float box[8] = {0};         // scene box over vertices: min xyzw, max xyzw
   float zscale[4] = {0};      // Morton scale
+  bool owns_mesh = true;      // verts and idx are this structure's (not an any-hit tree's geometry's)
   float4* verts = nullptr;    // float4 positions, w = 1
   uint32_t* idx = nullptr;    // input index buffer (3 * ntris)
   NodePair* pairs = nullptr;  // max(leaves - 1, 1) pairs
@@ -66,6 +140,14 @@ struct Blas {
   uint32_t nquads = 0;
   Quad32* quads32 = nullptr;
   Quad16* quads16 = nullptr;
+  // What a refit leaves of the BVH4 and watertight records: their memory and
+  // each internal node's BVH4 node (kInvalid: none), which the kept hierarchy
+  // does not change; the pointers above are null until they are remade.
+  uint32_t kept_quads = 0;
+  Quad32* kept_quads32 = nullptr;
+  Quad16* kept_quads16 = nullptr;
+  uint32_t* quad_of = nullptr;
+  TriPre* kept_wt = nullptr;
   // two levels per internal node for nearest-hit walks (made on demand by
   // blas_build_wide); the word after the last node is not zero where a walk on
   // them could differ from one on the pairs
@@ -89,15 +171,16 @@ struct Blas {
   Blas* any_tree = nullptr;
 };
 
-// Scratch for one build, sized for up to `cap` triangles; reused across builds.
-struct BuildScratch {
-  size_t cap = 0;
-  size_t bytes = 0;
-  void* base = nullptr;
-};
-
-hipError_t blas_alloc(Blas& b, uint32_t nverts, uint32_t ntris, bool keep_debug);
+// Allocates b's arrays from mem (with_mesh: vertices and indices too; an
+// any-hit tree shares its geometry's).
+hipError_t blas_alloc(Blas& b, DevCache* mem, uint32_t nverts, uint32_t ntris, bool keep_debug, bool with_mesh = true);
+// Gives b's arrays back, after waiting for the device (a trace on any stream
+// may still read them).
 void blas_free(Blas& b);
+// float4 vertices (w = 1) from nverts records of `stride` floats on the device.
+hipError_t expand_vertices(const float* raw, uint32_t stride, uint32_t nverts, float4* out, hipStream_t stream);
+// The largest of n indices on the device into *out (device).
+hipError_t largest_index(const uint32_t* idx, uint64_t n, uint32_t* out, hipStream_t stream);
 // Builds the LBVH of b.verts / b.idx (already on the device) on `stream`;
 // synchronises the stream before returning (leaves/max_run/box are host
 // values afterwards).

@@ -432,10 +432,12 @@ __global__ __launch_bounds__(kBlock) void k_leaves(Src src, const uint32_t* __re
 // ---------------------------------------------------------------------------
 // BVH4 collapse
 // ---------------------------------------------------------------------------
-// flag[k] = 1 when internal node k has even depth (it becomes a BVH4 node)
+// flag[k] = 1 when internal node k has even depth (it becomes a BVH4 node);
+// flag[ninternal] = 0
 __global__ __launch_bounds__(kBlock) void k_even_depth(const uint32_t* __restrict__ parent_int, uint32_t ninternal,
                                                        uint32_t* __restrict__ flag) {
   const uint32_t k = blockIdx.x * kBlock + threadIdx.x;
+  if (k == ninternal) flag[k] = 0u;
   if (k >= ninternal) return;
   uint32_t d = 0, p = k;
   while (p != 0) {  // at most 30 steps: the tree has at most 30 internal levels
@@ -443,6 +445,13 @@ __global__ __launch_bounds__(kBlock) void k_even_depth(const uint32_t* __restric
     d++;
   }
   flag[k] = (d & 1u) ? 0u : 1u;
+}
+
+// Scanned flags -> the BVH4 node of each internal node, kInvalid for none.
+__global__ __launch_bounds__(kBlock) void k_quad_index(const uint32_t* __restrict__ flag, uint32_t ninternal,
+                                                       uint32_t* __restrict__ index) {
+  const uint32_t k = blockIdx.x * kBlock + threadIdx.x;
+  if (k < ninternal && !flag[k]) index[k] = kInvalid;
 }
 
 struct Child {
@@ -463,12 +472,11 @@ __device__ inline Child pair_child(const NodePair* pairs, uint32_t k, uint32_t s
 // child replaced by its two children, left to right
 // (cbvh_core.cpp:263-352); internal references become quad indices.
 __global__ __launch_bounds__(kBlock) void k_collapse4(const NodePair* __restrict__ pairs,
-                                                      const uint32_t* __restrict__ flag,
                                                       const uint32_t* __restrict__ qidx, uint32_t ninternal,
                                                       Quad32* __restrict__ q32, Quad16* __restrict__ q16) {
   const uint32_t k = blockIdx.x * kBlock + threadIdx.x;
   const bool single = (ninternal == 0);  // the root is a leaf: one node from pair 0
-  if (single ? k != 0 : (k >= ninternal || !flag[k])) return;
+  if (single ? k != 0 : (k >= ninternal || qidx[k] == kInvalid)) return;
   Child c[4];
   int n = 0;
   for (uint32_t side = 0; side < 2; side++) {
@@ -505,6 +513,25 @@ __global__ __launch_bounds__(kBlock) void k_collapse4(const NodePair* __restrict
                         round_to_pos(c[i].hi.y) | (round_to_pos(c[i].hi.z) << 16), ref[i]);
   }
   q16[q] = h;
+}
+
+// float4 copies (w = 1) of vertices `stride` floats apart
+// (BVH2CommonRT_host.cpp:79-84).
+__global__ __launch_bounds__(kBlock) void k_expand_vertices(const float* __restrict__ raw, uint32_t stride, uint32_t n,
+                                                            float4* __restrict__ out) {
+  const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+  if (i >= n) return;
+  const float* p = raw + size_t(i) * stride;
+  out[i] = make_float4(p[0], p[1], p[2], 1.0f);
+}
+
+__global__ __launch_bounds__(kBlock) void k_largest_index(const uint32_t* __restrict__ idx, uint64_t n,
+                                                          uint32_t* __restrict__ out) {
+  uint32_t m = 0;
+  for (uint64_t i = uint64_t(blockIdx.x) * kBlock + threadIdx.x; i < n; i += uint64_t(gridDim.x) * kBlock)
+    m = max(m, idx[i]);
+  for (int o = 32; o > 0; o >>= 1) m = max(m, uint32_t(__shfl_xor(m, o)));
+  if ((threadIdx.x & 63) == 0) atomicMax(out, m);
 }
 
 // One WideNode per internal node (a one-leaf tree's pair 0 counts as one):
@@ -567,28 +594,137 @@ inline uint32_t blocks_for(uint64_t n) { return uint32_t((n + kBlock - 1) / kBlo
 
 }  // namespace
 
-hipError_t blas_alloc(Blas& b, uint32_t nverts, uint32_t ntris, bool keep_debug) {
+DevCache::~DevCache() {
+  trim();
+  if (pinned_) (void)hipHostFree(pinned_);
+}
+
+void DevCache::wait() {
+  int current = device_;
+  (void)hipGetDevice(&current);
+  if (current != device_) (void)hipSetDevice(device_);
+  (void)hipDeviceSynchronize();
+  if (current != device_) (void)hipSetDevice(current);
+}
+
+void DevCache::trim() {
+  std::multimap<size_t, void*> idle;
+  {
+    std::lock_guard<std::mutex> lock(mu_);
+    idle.swap(idle_);
+    idle_bytes_ = 0;
+  }
+  for (auto& x : idle) (void)hipFree(x.second);
+}
+
+hipError_t DevCache::alloc_bytes(void** p, size_t bytes) {
+  // sizes in steps, so that a slightly different geometry finds its memory
+  const size_t step = bytes < (size_t(1) << 16) ? size_t(1) << 12 : bytes < (size_t(1) << 20) ? size_t(1) << 16 : size_t(1) << 21;
+  const size_t size = (std::max<size_t>(bytes, 1) + step - 1) / step * step;
+  {
+    std::lock_guard<std::mutex> lock(mu_);
+    auto it = idle_.lower_bound(size);
+    if (it != idle_.end() && it->first <= size + size / 4) {
+      if (!note(it->second, it->first)) return hipErrorOutOfMemory;
+      *p = it->second;
+      idle_bytes_ -= it->first;
+      idle_.erase(it);
+      return hipSuccess;
+    }
+  }
+  hipError_t e = hipMalloc(p, size);
+  if (e == hipErrorOutOfMemory) {
+    (void)hipGetLastError();
+    trim();
+    e = hipMalloc(p, size);
+  }
+  if (e != hipSuccess) {
+    *p = nullptr;
+    return e;
+  }
+  std::lock_guard<std::mutex> lock(mu_);
+  if (note(*p, size)) return hipSuccess;
+  (void)hipFree(*p);
+  *p = nullptr;
+  return hipErrorOutOfMemory;
+}
+
+// mu_ held; false: no host memory
+bool DevCache::note(void* p, size_t size) {
+  try {
+    live_[p] = size;
+  } catch (const std::bad_alloc&) {
+    return false;
+  }
+  return true;
+}
+
+void DevCache::free(void* p) {
+  if (!p) return;
+  {
+    std::lock_guard<std::mutex> lock(mu_);
+    const auto it = live_.find(p);
+    if (it == live_.end()) return;
+    const size_t size = it->second;
+    live_.erase(it);
+    try {
+      if (idle_bytes_ + size <= kMaxIdle) {
+        idle_.emplace(size, p);
+        idle_bytes_ += size;
+        return;
+      }
+    } catch (const std::bad_alloc&) {  // given back below
+    }
+  }
+  (void)hipFree(p);
+}
+
+uint32_t* DevCache::pinned_get() {
+  std::lock_guard<std::mutex> lock(mu_);
+  if (!pinned_ && hipHostMalloc(reinterpret_cast<void**>(&pinned_), 4 * kPinnedWords * kPinnedSlots, hipHostMallocDefault) != hipSuccess) {
+    (void)hipGetLastError();
+    pinned_ = nullptr;
+    return nullptr;
+  }
+  for (int k = 0; k < kPinnedSlots; k++) {
+    if (pinned_taken_ & (1u << k)) continue;
+    pinned_taken_ |= 1u << k;
+    return pinned_ + k * kPinnedWords;
+  }
+  return nullptr;
+}
+
+void DevCache::pinned_put(uint32_t* w) {
+  std::lock_guard<std::mutex> lock(mu_);
+  pinned_taken_ &= ~(1u << (size_t(w - pinned_) / kPinnedWords));
+}
+
+hipError_t blas_alloc(Blas& b, DevCache* mem, uint32_t nverts, uint32_t ntris, bool keep_debug, bool with_mesh) {
+  b.mem = mem;
   b.nverts = nverts;
   b.ntris = ntris;
   b.keep_debug = keep_debug;
   const size_t npairs = std::max<size_t>(ntris > 1 ? ntris - 1 : 1, 1);
-  HRT_CHECK(hipMalloc(&b.verts, sizeof(float4) * std::max<size_t>(nverts, 1)));
-  HRT_CHECK(hipMalloc(&b.idx, sizeof(uint32_t) * 3 * size_t(ntris)));
-  HRT_CHECK(hipMalloc(&b.pairs, sizeof(NodePair) * npairs));
-  HRT_CHECK(hipMalloc(&b.tris, sizeof(TriPre) * size_t(ntris)));
-  HRT_CHECK(hipMalloc(&b.perm, sizeof(uint32_t) * size_t(ntris)));
-  HRT_CHECK(hipMalloc(&b.parent, sizeof(uint32_t) * npairs));
-  HRT_CHECK(hipMalloc(&b.leaf_run, sizeof(uint32_t) * size_t(ntris)));
-  HRT_CHECK(hipMalloc(&b.parent_leaf, sizeof(uint32_t) * size_t(ntris)));
-  HRT_CHECK(hipMalloc(&b.node_range, sizeof(uint2) * npairs));
-  HRT_CHECK(hipMalloc(&b.meta, sizeof(uint32_t) * 64));
+  if (with_mesh) {
+    HRT_CHECK(mem->alloc(&b.verts, sizeof(float4) * std::max<size_t>(nverts, 1)));
+    HRT_CHECK(mem->alloc(&b.idx, sizeof(uint32_t) * 3 * size_t(ntris)));
+  }
+  b.owns_mesh = with_mesh;
+  HRT_CHECK(mem->alloc(&b.pairs, sizeof(NodePair) * npairs));
+  HRT_CHECK(mem->alloc(&b.tris, sizeof(TriPre) * size_t(ntris)));
+  HRT_CHECK(mem->alloc(&b.perm, sizeof(uint32_t) * size_t(ntris)));
+  HRT_CHECK(mem->alloc(&b.parent, sizeof(uint32_t) * npairs));
+  HRT_CHECK(mem->alloc(&b.leaf_run, sizeof(uint32_t) * size_t(ntris)));
+  HRT_CHECK(mem->alloc(&b.parent_leaf, sizeof(uint32_t) * size_t(ntris)));
+  HRT_CHECK(mem->alloc(&b.node_range, sizeof(uint2) * npairs));
+  HRT_CHECK(mem->alloc(&b.meta, sizeof(uint32_t) * 64));
   if (keep_debug) {
-    HRT_CHECK(hipMalloc(&b.codes_in, sizeof(uint32_t) * size_t(ntris)));
-    HRT_CHECK(hipMalloc(&b.codes_sorted, sizeof(uint32_t) * size_t(ntris)));
-    HRT_CHECK(hipMalloc(&b.ids_sorted, sizeof(uint32_t) * size_t(ntris)));
-    HRT_CHECK(hipMalloc(&b.run_start, sizeof(uint32_t) * size_t(ntris)));
-    HRT_CHECK(hipMalloc(&b.ucodes, sizeof(uint32_t) * size_t(ntris)));
-    HRT_CHECK(hipMalloc(&b.karras_lr, sizeof(uint32_t) * 2 * npairs));
+    HRT_CHECK(mem->alloc(&b.codes_in, sizeof(uint32_t) * size_t(ntris)));
+    HRT_CHECK(mem->alloc(&b.codes_sorted, sizeof(uint32_t) * size_t(ntris)));
+    HRT_CHECK(mem->alloc(&b.ids_sorted, sizeof(uint32_t) * size_t(ntris)));
+    HRT_CHECK(mem->alloc(&b.run_start, sizeof(uint32_t) * size_t(ntris)));
+    HRT_CHECK(mem->alloc(&b.ucodes, sizeof(uint32_t) * size_t(ntris)));
+    HRT_CHECK(mem->alloc(&b.karras_lr, sizeof(uint32_t) * 2 * npairs));
   }
   return hipSuccess;
 }
@@ -599,12 +735,17 @@ void blas_free(Blas& b) {
     delete b.any_tree;
     b.any_tree = nullptr;
   }
-  void* ptrs[] = {b.leaf_run,   b.parent_leaf, b.node_range, b.meta,       b.tris_wt, b.wide,
-                  b.verts,      b.idx,        b.pairs,      b.tris,      b.perm,   b.parent,
-                  b.quads32,    b.quads16,    b.codes_in,   b.codes_sorted, b.ids_sorted,
-                  b.run_start,  b.ucodes,     b.karras_lr};
-  for (void* p : ptrs)
-    if (p) (void)hipFree(p);
+  if (b.mem) {
+    b.mem->wait();
+    if (b.quads32 != b.kept_quads32) b.mem->free(b.kept_quads32);
+    if (b.quads16 != b.kept_quads16) b.mem->free(b.kept_quads16);
+    if (b.tris_wt != b.kept_wt) b.mem->free(b.kept_wt);
+    void* ptrs[] = {b.leaf_run, b.parent_leaf, b.node_range, b.meta,     b.tris_wt,  b.wide,
+                    b.pairs,    b.tris,        b.perm,       b.parent,   b.quads32,  b.quads16,
+                    b.quad_of,  b.codes_in,    b.codes_sorted, b.ids_sorted, b.run_start, b.ucodes,
+                    b.karras_lr, b.owns_mesh ? b.verts : nullptr, b.owns_mesh ? b.idx : nullptr};
+    for (void* p : ptrs) b.mem->free(p);
+  }
   b = Blas();
 }
 
@@ -637,7 +778,8 @@ hipError_t lbvh_build(Blas& b, const Src& src, uint32_t box_items, hipStream_t s
   const size_t o_tops = take(tops_cap);
   const size_t o_part = take(size_t(box_parts) * 8), o_box = take(16);
   uint32_t* base = nullptr;
-  HRT_CHECK(hipMallocAsync(reinterpret_cast<void**>(&base), words * 4, s));
+  HRT_CHECK(b.mem->alloc(&base, words * 4));
+  Readback back(b.mem);
   uint32_t *ka = base + o_ka, *va = base + o_va, *kb = base + o_kb, *vb = base + o_vb;
   uint32_t *sort_tmp = base + o_sort, *stmp = base + o_scan;
   uint32_t *flags = base + o_flags, *pos = base + o_pos, *uc = base + o_uc, *arrive = base + o_arr;
@@ -683,10 +825,10 @@ hipError_t lbvh_build(Blas& b, const Src& src, uint32_t box_items, hipStream_t s
       if ((err = hipMemcpyAsync(b.run_start, rs, 4 * N, hipMemcpyDeviceToDevice, s)) != hipSuccess) break;
       if ((err = hipMemcpyAsync(b.ucodes, uc, 4 * N, hipMemcpyDeviceToDevice, s)) != hipSuccess) break;
     }
-    uint32_t hmeta[5];
-    float hbox[12];
-    if ((err = hipMemcpyAsync(hmeta, meta, sizeof(hmeta), hipMemcpyDeviceToHost, s)) != hipSuccess) break;
-    if ((err = hipMemcpyAsync(hbox, box, sizeof(hbox), hipMemcpyDeviceToHost, s)) != hipSuccess) break;
+    const uint32_t* hmeta = back.words();
+    const uint32_t* hbox = back.words() + 8;
+    if ((err = back.read(0, meta, 5, s)) != hipSuccess) break;
+    if ((err = back.read(8, box, 12, s)) != hipSuccess) break;
     if ((err = hipStreamSynchronize(s)) != hipSuccess) break;
     if (hmeta[3] != 0u || hmeta[4] != 0u) {  // a device-side check failed: the tree is incomplete
       err = hipErrorIllegalState;
@@ -697,9 +839,8 @@ hipError_t lbvh_build(Blas& b, const Src& src, uint32_t box_items, hipStream_t s
     std::memcpy(b.box, hbox, sizeof(b.box));
     std::memcpy(b.zscale, hbox + 8, sizeof(b.zscale));
   } while (false);
-  hipError_t ferr = hipFreeAsync(base, s);
-  if (err == hipSuccess) err = ferr;
-  if (err == hipSuccess) err = hipStreamSynchronize(s);
+  if (err != hipSuccess) (void)hipStreamSynchronize(s);  // the scratch may still be in use
+  b.mem->free(base);
   return err;
 }
 
@@ -731,7 +872,8 @@ hipError_t blas_refit(Blas& b, hipStream_t s) {
   const uint32_t tops_cap = refit_tops_capacity(N);
   const size_t o_tops = (N + 63) & ~size_t(63);
   const size_t o_part = o_tops + ((tops_cap + 63) & ~size_t(63));
-  HRT_CHECK(hipMallocAsync(reinterpret_cast<void**>(&base), 4 * (o_part + 8 * size_t(box_parts) + 16), s));
+  HRT_CHECK(b.mem->alloc(&base, 4 * (o_part + 8 * size_t(box_parts) + 16)));
+  Readback back(b.mem);
   uint32_t* arrive = base;
   uint32_t* tops = base + o_tops;
   float4* part = reinterpret_cast<float4*>(base + o_part);
@@ -747,24 +889,26 @@ hipError_t blas_refit(Blas& b, hipStream_t s) {
   k_refit_chunks<OneTree><<<uint32_t((N + kRefitChunk - 1) / kRefitChunk), kRefitThreads, 0, s>>>(
       tree, b.pairs, b.parent, b.parent_leaf, b.node_range, tops, b.meta + 2, b.meta + 3);
   k_refit_tops<OneTree><<<1, kRefitTopsThreads, 0, s>>>(tree, b.pairs, b.parent, tops, b.meta + 2, arrive);
-  hipError_t err = hipGetLastError();
-  float hbox[8];
-  uint32_t hmeta[4];
-  if (err == hipSuccess) err = hipMemcpyAsync(hbox, box, sizeof(hbox), hipMemcpyDeviceToHost, s);
-  if (err == hipSuccess) err = hipMemcpyAsync(hmeta, b.meta, sizeof(hmeta), hipMemcpyDeviceToHost, s);
-  hipError_t ferr = hipFreeAsync(base, s);
-  if (err == hipSuccess) err = ferr;
-  if (err == hipSuccess) err = hipStreamSynchronize(s);
-  if (err == hipSuccess && hmeta[3] != 0u) err = hipErrorIllegalState;  // a refit list overflowed
-  if (err != hipSuccess) return err;
-  std::memcpy(b.box, hbox, sizeof(b.box));
-  // boxes changed: the BVH4 nodes, the watertight records and the any-hit
-  // tree are made again on the next commit
   b.wide_made = false;
-  if (b.tris_wt) (void)hipFree(b.tris_wt);
+  hipError_t err = b.wide ? blas_build_wide(b, s) : hipGetLastError();
+  if (err == hipSuccess) err = back.read(0, b.meta, 4, s);
+  if (err == hipSuccess) err = back.read(8, box, 8, s);
+  const hipError_t werr = hipStreamSynchronize(s);
+  b.mem->free(base);
+  if (err == hipSuccess) err = werr;
+  if (err == hipSuccess && back.words()[3] != 0u) err = hipErrorIllegalState;  // a refit list overflowed
+  if (err != hipSuccess) return err;
+  std::memcpy(b.box, back.words() + 8, sizeof(b.box));
+  if (b.quads32 || b.tris_wt) b.mem->wait();  // traces of the old records end before they are rewritten
+  // boxes changed: the BVH4 nodes, the watertight records and the any-hit
+  // tree are made again on the next commit, the first two in their old memory
+  if (b.tris_wt) b.kept_wt = b.tris_wt;
   b.tris_wt = nullptr;
-  if (b.quads32) (void)hipFree(b.quads32);
-  if (b.quads16) (void)hipFree(b.quads16);
+  if (b.quads32) {
+    b.kept_quads = b.nquads;
+    b.kept_quads32 = b.quads32;
+    b.kept_quads16 = b.quads16;
+  }
   b.quads32 = nullptr;
   b.quads16 = nullptr;
   b.nquads = 0;
@@ -780,9 +924,9 @@ hipError_t blas_build_any_tree(Blas& b, hipStream_t s) {
   if (b.any_tree) return hipSuccess;
   Blas* a = new (std::nothrow) Blas();
   if (!a) return hipErrorOutOfMemory;
-  hipError_t e = blas_alloc(*a, b.nverts, b.ntris, b.keep_debug);
-  if (e == hipSuccess) e = hipMemcpyAsync(a->verts, b.verts, 16ull * b.nverts, hipMemcpyDeviceToDevice, s);
-  if (e == hipSuccess) e = hipMemcpyAsync(a->idx, b.idx, 12ull * b.ntris, hipMemcpyDeviceToDevice, s);
+  hipError_t e = blas_alloc(*a, b.mem, b.nverts, b.ntris, b.keep_debug, false);
+  a->verts = b.verts;
+  a->idx = b.idx;
   if (e == hipSuccess) e = blas_build(*a, s, true);
   // a run longer than the 7-bit leaf count cannot be stored: keep the
   // reference tree for any-hit queries then
@@ -806,10 +950,21 @@ hipError_t tlas_build(Blas& t, const InstDev* by_id, InstDev* leaf_order, hipStr
   });
 }
 
+hipError_t expand_vertices(const float* raw, uint32_t stride, uint32_t nverts, float4* out, hipStream_t s) {
+  k_expand_vertices<<<blocks_for(nverts), kBlock, 0, s>>>(raw, stride, nverts, out);
+  return hipGetLastError();
+}
+
+hipError_t largest_index(const uint32_t* idx, uint64_t n, uint32_t* out, hipStream_t s) {
+  k_fill<<<1, kBlock, 0, s>>>(out, 1, 0u);
+  k_largest_index<<<fill_blocks(n), kBlock, 0, s>>>(idx, n, out);
+  return hipGetLastError();
+}
+
 hipError_t blas_build_wide(Blas& b, hipStream_t s) {
   if (b.wide_made) return hipSuccess;
   const uint32_t n = internal_nodes(b);
-  if (!b.wide && hipMalloc(&b.wide, sizeof(WideNode) * (size_t(n) + 1)) != hipSuccess) {
+  if (!b.wide && b.mem->alloc(&b.wide, sizeof(WideNode) * (size_t(n) + 1)) != hipSuccess) {
     (void)hipGetLastError();  // no memory: the walks stay on the pairs
     b.wide = nullptr;
     return hipSuccess;
@@ -824,7 +979,8 @@ hipError_t blas_build_wide(Blas& b, hipStream_t s) {
 
 hipError_t blas_build_wt_tris(Blas& b, hipStream_t s) {
   if (b.tris_wt) return hipSuccess;
-  HRT_CHECK(hipMalloc(&b.tris_wt, sizeof(TriPre) * size_t(b.ntris)));
+  if (!b.kept_wt) HRT_CHECK(b.mem->alloc(&b.kept_wt, sizeof(TriPre) * size_t(b.ntris)));
+  b.tris_wt = b.kept_wt;
   k_wt_tris<<<blocks_for(b.ntris), kBlock, 0, s>>>(b.verts, b.idx, b.perm, b.ntris, b.tris_wt);
   return hipGetLastError();
 }
@@ -832,41 +988,52 @@ hipError_t blas_build_wt_tris(Blas& b, hipStream_t s) {
 hipError_t blas_build_bvh4(Blas& b, hipStream_t s) {
   if (b.quads32) return hipSuccess;
   const uint32_t ninternal = b.leaves > 1 ? b.leaves - 1 : 0;
-  const size_t nflag = std::max<uint32_t>(ninternal, 1);
-  const size_t w_scan = scan_temp_words(nflag);
-  uint32_t* base = nullptr;
-  HRT_CHECK(hipMallocAsync(reinterpret_cast<void**>(&base), 4 * (2 * nflag + w_scan + 64), s));
-  uint32_t *flag = base, *qidx = base + nflag, *stmp = base + 2 * nflag;
   hipError_t err = hipSuccess;
-  do {
+  if (!b.quad_of) {  // which internal nodes are BVH4 nodes, and which ones
+    const size_t nflag = size_t(ninternal) + 1;  // one past the end: the scan's total
+    uint32_t *flag = nullptr, *index = nullptr;
     uint32_t nq = 1;
-    if (ninternal > 0) {
-      k_even_depth<<<blocks_for(ninternal), kBlock, 0, s>>>(b.parent, ninternal, flag);
-      if ((err = exclusive_scan(flag, qidx, ninternal, stmp, s)) != hipSuccess) break;
-      uint32_t last[2];
-      if ((err = hipMemcpyAsync(&last[0], qidx + ninternal - 1, 4, hipMemcpyDeviceToHost, s)) != hipSuccess) break;
-      if ((err = hipMemcpyAsync(&last[1], flag + ninternal - 1, 4, hipMemcpyDeviceToHost, s)) != hipSuccess) break;
-      if ((err = hipStreamSynchronize(s)) != hipSuccess) break;
-      nq = last[0] + last[1];
+    HRT_CHECK(b.mem->alloc(&index, 4 * nflag));
+    if ((err = b.mem->alloc(&flag, 4 * (nflag + scan_temp_words(nflag)))) == hipSuccess && ninternal > 0) {
+      Readback back(b.mem);
+      k_even_depth<<<blocks_for(nflag), kBlock, 0, s>>>(b.parent, ninternal, flag);
+      err = exclusive_scan(flag, index, nflag, flag + nflag, s);
+      if (err == hipSuccess) k_quad_index<<<blocks_for(ninternal), kBlock, 0, s>>>(flag, ninternal, index);
+      if (err == hipSuccess) err = hipGetLastError();
+      if (err == hipSuccess) err = back.read(0, index + ninternal, 1, s);
+      const hipError_t werr = hipStreamSynchronize(s);
+      if (err == hipSuccess) err = werr;
+      nq = back.words()[0];
     }
-    if ((err = hipMalloc(&b.quads32, sizeof(Quad32) * nq)) != hipSuccess) break;
-    if ((err = hipMalloc(&b.quads16, sizeof(Quad16) * nq)) != hipSuccess) break;
-    k_collapse4<<<blocks_for(std::max<uint32_t>(ninternal, 1)), kBlock, 0, s>>>(b.pairs, flag, qidx, ninternal,
-                                                                               b.quads32, b.quads16);
-    if ((err = hipGetLastError()) != hipSuccess) break;
-    b.nquads = nq;
-  } while (false);
-  hipError_t ferr = hipFreeAsync(base, s);
-  if (err == hipSuccess) err = ferr;
-  if (err == hipSuccess) err = hipStreamSynchronize(s);
-  if (err != hipSuccess) {
-    if (b.quads32) (void)hipFree(b.quads32);
-    if (b.quads16) (void)hipFree(b.quads16);
-    b.quads32 = nullptr;
-    b.quads16 = nullptr;
-    b.nquads = 0;
+    b.mem->free(flag);
+    if (b.kept_quads != nq) {  // (equal: a restored tree that was refitted)
+      b.mem->free(b.kept_quads32);
+      b.mem->free(b.kept_quads16);
+      b.kept_quads32 = nullptr;
+      b.kept_quads16 = nullptr;
+      if (err == hipSuccess) err = b.mem->alloc(&b.kept_quads32, sizeof(Quad32) * nq);
+      if (err == hipSuccess) err = b.mem->alloc(&b.kept_quads16, sizeof(Quad16) * nq);
+    }
+    if (err != hipSuccess) {
+      b.mem->free(index);
+      b.mem->free(b.kept_quads32);
+      b.mem->free(b.kept_quads16);
+      b.kept_quads32 = nullptr;
+      b.kept_quads16 = nullptr;
+      b.kept_quads = 0;
+      return err;
+    }
+    b.quad_of = index;
+    b.kept_quads = nq;
   }
-  return err;
+  k_collapse4<<<blocks_for(std::max<uint32_t>(ninternal, 1)), kBlock, 0, s>>>(b.pairs, b.quad_of, ninternal,
+                                                                             b.kept_quads32, b.kept_quads16);
+  if ((err = hipGetLastError()) == hipSuccess) err = hipStreamSynchronize(s);
+  if (err != hipSuccess) return err;
+  b.quads32 = b.kept_quads32;
+  b.quads16 = b.kept_quads16;
+  b.nquads = b.kept_quads;
+  return hipSuccess;
 }
 
 }  // namespace hrt

@@ -390,10 +390,11 @@ hipError_t blas_ploc(Blas& b, hipStream_t s, bool* replaced) {
   // the same capacities as blas_alloc's (pairs for every triangle but one),
   // so the swapped arrays can stand in for the originals everywhere
   const size_t cap = std::max<size_t>(b.ntris > 1 ? b.ntris - 1 : 1, 1);
-  hipError_t e = hipMalloc(&npairs, sizeof(NodePair) * cap);
-  if (e == hipSuccess) e = hipMalloc(&nparent, 4ull * cap);
-  if (e == hipSuccess && b.karras_lr) e = hipMalloc(&nlr, 8ull * cap);
-  if (e == hipSuccess) e = hipMallocAsync(reinterpret_cast<void**>(&base), 4 * words, s);
+  hipError_t e = b.mem->alloc(&npairs, sizeof(NodePair) * cap);
+  if (e == hipSuccess) e = b.mem->alloc(&nparent, 4ull * cap);
+  if (e == hipSuccess && b.karras_lr) e = b.mem->alloc(&nlr, 8ull * cap);
+  if (e == hipSuccess) e = b.mem->alloc(&base, 4 * words);
+  Readback back(b.mem);
   bool ok = false;
   if (e == hipSuccess) {
     Cluster* ca = reinterpret_cast<Cluster*>(base + o_ca);
@@ -412,8 +413,9 @@ hipError_t blas_ploc(Blas& b, hipStream_t s, bool* replaced) {
       k_ploc_finish<<<1, kFinishThreads, 0, s>>>(ca, cb, st + rounds, npairs, nparent, nlr);
       PlocState after;
       if ((e = hipGetLastError()) != hipSuccess) break;
-      if ((e = hipMemcpyAsync(&after, st + rounds, sizeof(after), hipMemcpyDeviceToHost, s)) != hipSuccess) break;
+      if ((e = back.read(0, st + rounds, sizeof(after) / 4, s)) != hipSuccess) break;
       if ((e = hipStreamSynchronize(s)) != hipSuccess) break;
+      std::memcpy(&after, back.words(), sizeof(after));
       // every round merges at least one pair (see the rule above), and each
       // merge takes one cluster and one id
       if (after.n == 0 || after.n >= now.n || now.n - after.n != now.next_id - after.next_id) {
@@ -427,11 +429,8 @@ hipError_t blas_ploc(Blas& b, hipStream_t s, bool* replaced) {
     // internal levels
     ok = e == hipSuccess && now.height <= uint32_t(kMaxLevels4);
   }
-  if (base) {
-    const hipError_t fe = hipFreeAsync(base, s);
-    if (e == hipSuccess) e = fe;
-  }
-  if (e == hipSuccess) e = hipStreamSynchronize(s);
+  const hipError_t werr = hipStreamSynchronize(s);  // the scratch may still be in use
+  if (e == hipSuccess) e = werr;
   if (e == hipSuccess && ok) {
     std::swap(b.pairs, npairs);
     std::swap(b.parent, nparent);
@@ -439,9 +438,10 @@ hipError_t blas_ploc(Blas& b, hipStream_t s, bool* replaced) {
     b.clustered = true;
     *replaced = true;
   }
-  if (npairs) (void)hipFree(npairs);
-  if (nparent) (void)hipFree(nparent);
-  if (nlr) (void)hipFree(nlr);
+  b.mem->free(base);
+  b.mem->free(npairs);
+  b.mem->free(nparent);
+  b.mem->free(nlr);
   return e;
 }
 
