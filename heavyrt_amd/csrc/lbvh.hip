@@ -21,6 +21,7 @@
 
 #include "hrt_internal.h"
 #include "refit.h"
+#include "small.h"
 
 namespace hrt {
 namespace {
@@ -454,20 +455,6 @@ __global__ __launch_bounds__(kBlock) void k_quad_index(const uint32_t* __restric
   if (k < ninternal && !flag[k]) index[k] = kInvalid;
 }
 
-struct Child {
-  float3 lo, hi;
-  uint32_t ref;
-};
-
-__device__ inline Child pair_child(const NodePair* pairs, uint32_t k, uint32_t side) {
-  const uint32_t* pw = reinterpret_cast<const uint32_t*>(pairs + k) + 8 * side;
-  Child c;
-  c.lo = make_float3(__uint_as_float(pw[0]), __uint_as_float(pw[1]), __uint_as_float(pw[2]));
-  c.hi = make_float3(__uint_as_float(pw[4]), __uint_as_float(pw[5]), __uint_as_float(pw[6]));
-  c.ref = pw[3];
-  return c;
-}
-
 // One BVH4 node per even-depth internal node k: k's children, each internal
 // child replaced by its two children, left to right
 // (cbvh_core.cpp:263-352); internal references become quad indices.
@@ -534,41 +521,12 @@ __global__ __launch_bounds__(kBlock) void k_largest_index(const uint32_t* __rest
   if ((threadIdx.x & 63) == 0) atomicMax(out, m);
 }
 
-// One WideNode per internal node (a one-leaf tree's pair 0 counts as one):
-// three pairs in, 128 B out.  *differ is set when a child box is not the union
-// of its own children's boxes, or one of those is inverted (a leaf of NaN
-// vertices): the walk takes a child's distances from its children's.
+// One WideNode per internal node: three pairs in, 128 B out; *differ is set when
+// the tree may not be walked on them (make_wide_node).
 __global__ __launch_bounds__(kBlock) void k_wide_nodes(const NodePair* __restrict__ pairs, uint32_t n,
                                                        WideNode* __restrict__ out, uint32_t* __restrict__ differ) {
   const uint32_t k = blockIdx.x * kBlock + threadIdx.x;
-  if (k >= n) return;
-  Child g[4];
-  uint32_t ref[2];
-  bool exact = true;
-  for (int side = 0; side < 2; side++) {
-    const Child c = pair_child(pairs, k, side);
-    Child &g0 = g[2 * side], &g1 = g[2 * side + 1];
-    ref[side] = c.ref;
-    if (c.ref & kLeafBit) {
-      g0 = g1 = c;
-      g1.ref = kInvalid;
-      continue;
-    }
-    g0 = pair_child(pairs, c.ref, 0);
-    g1 = pair_child(pairs, c.ref, 1);
-    exact = exact && g0.lo.x <= g0.hi.x && g0.lo.y <= g0.hi.y && g0.lo.z <= g0.hi.z && g1.lo.x <= g1.hi.x &&
-            g1.lo.y <= g1.hi.y && g1.lo.z <= g1.hi.z && c.lo.x == fminf(g0.lo.x, g1.lo.x) &&
-            c.lo.y == fminf(g0.lo.y, g1.lo.y) && c.lo.z == fminf(g0.lo.z, g1.lo.z) &&
-            c.hi.x == fmaxf(g0.hi.x, g1.hi.x) && c.hi.y == fmaxf(g0.hi.y, g1.hi.y) &&
-            c.hi.z == fmaxf(g0.hi.z, g1.hi.z);
-  }
-  if (!exact) *differ = 1u;
-  WideNode w;
-  for (int i = 0; i < 4; i++) {
-    w.g[2 * i] = make_float4(g[i].lo.x, g[i].lo.y, g[i].lo.z, __uint_as_float(g[i].ref));
-    w.g[2 * i + 1] = make_float4(g[i].hi.x, g[i].hi.y, g[i].hi.z, __uint_as_float(ref[i >> 1]));
-  }
-  out[k] = w;
+  if (k < n && !make_wide_node(pairs, k, out + k)) *differ = 1u;
 }
 
 // Leaf-order triangle j with its absolute vertices for the watertight test:
@@ -759,6 +717,14 @@ __global__ __launch_bounds__(kBlock) void k_fill(uint32_t* __restrict__ p, uint6
 
 inline uint32_t fill_blocks(uint64_t n) { return uint32_t(std::min<uint64_t>(1024, std::max<uint64_t>(1, (n + kBlock - 1) / kBlock))); }
 
+template <class Src, uint32_t kThreads, uint32_t kItems>
+__global__ __launch_bounds__(kThreads) void k_small_build(Src src, uint32_t n, int cubic, SmallTree out) {
+  __shared__ SmallLds<kThreads, kItems> lds;
+  if (threadIdx.x < 8) out.leaves[threadIdx.x] = 0u;  // the meta words
+  __syncthreads();
+  small_build(src, n, cubic, out, lds);
+}
+
 // The LBVH pipeline over any primitive source.  `finish(ids_sorted)` enqueues
 // the leaf-order pass; the stream is synchronised before returning and the
 // leaf count, longest run and scene box are host values afterwards.
@@ -766,6 +732,27 @@ template <class Src, class Finish>
 hipError_t lbvh_build(Blas& b, const Src& src, uint32_t box_items, hipStream_t s, Finish&& finish, int cubic = 0) {
   const uint64_t N = b.ntris;
   if (N == 0) return hipErrorInvalidValue;
+  if (N <= kSmallMax && box_items <= kSmallVerts) {
+    // one launch (small.h): adding 4,096 triangles takes 114 us, the 4,097th
+    // and with it the staged build 196
+    const SmallTree out{b.pairs,      b.tris,         b.perm,       b.parent,    b.parent_leaf, b.leaf_run,
+                        b.node_range, b.meta,         b.meta + 1,   reinterpret_cast<float*>(b.meta + 8),
+                        b.codes_in,   b.codes_sorted, b.ids_sorted, b.run_start, b.ucodes,      b.karras_lr,
+                        nullptr,      nullptr};
+    if (N <= 1024) k_small_build<Src, 512, 2><<<1, 512, 0, s>>>(src, uint32_t(N), cubic, out);
+    else k_small_build<Src, 1024, 4><<<1, 1024, 0, s>>>(src, uint32_t(N), cubic, out);
+    HRT_CHECK(hipGetLastError());
+    finish(b.perm);
+    HRT_CHECK(hipGetLastError());
+    Readback back(b.mem);
+    HRT_CHECK(back.read(0, b.meta, 20, s));
+    HRT_CHECK(hipStreamSynchronize(s));
+    b.leaves = back.words()[0];
+    b.max_run = back.words()[1];
+    std::memcpy(b.box, back.words() + 8, sizeof(b.box));
+    std::memcpy(b.zscale, back.words() + 16, sizeof(b.zscale));
+    return hipSuccess;
+  }
   const int box_parts = int(std::min<uint64_t>(1024, std::max<uint64_t>(1, (box_items + kBlock - 1) / kBlock)));
   // scratch layout (u32 words)
   const size_t w_codes = N, w_sort = radix_sort_scratch_words(N, 4), w_scan = scan_temp_words(N);
@@ -844,10 +831,10 @@ hipError_t lbvh_build(Blas& b, const Src& src, uint32_t box_items, hipStream_t s
   return err;
 }
 
-// Instance records in leaf order.
+// Instance records in leaf order (perm may be ids_sorted).
 __global__ __launch_bounds__(kBlock) void k_inst_order(const InstDev* __restrict__ by_id,
-                                                       const uint32_t* __restrict__ ids_sorted, uint32_t n,
-                                                       InstDev* __restrict__ leaf_order, uint32_t* __restrict__ perm) {
+                                                       const uint32_t* ids_sorted, uint32_t n,
+                                                       InstDev* __restrict__ leaf_order, uint32_t* perm) {
   const uint32_t j = blockIdx.x * kBlock + threadIdx.x;
   if (j >= n) return;
   const uint32_t t = ids_sorted[j];

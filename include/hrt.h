@@ -362,7 +362,9 @@ hrt_status hrt_batch_build(hrt_batch* batch, void* stream);
 hrt_status hrt_batch_trace(hrt_batch* batch, void* stream);
 /* Trace-kernel candidates: waves per workgroup, LDS stack entries per lane
  * (0 = one ray per lane without refill), the refill threshold (idle lanes)
- * and the number of ray indices a wave claims from the queue at once. */
+ * and the number of ray indices a wave claims from the queue at once.  A batch
+ * of at most 65,536 rays over scenes of at most 4,096 triangles is traced by a
+ * kernel of its own, whatever candidate is set. */
 int hrt_batch_candidate_count(void);
 hrt_status hrt_batch_candidate_info(int i, int* wavesPerGroup, int* ldsStackEntries, int* refillAt, int* claim);
 hrt_status hrt_batch_set_candidate(hrt_batch* batch, int i);

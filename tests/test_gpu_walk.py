@@ -8,7 +8,7 @@ from gpu_util import make_scene, say, trace
 from heavyrt_amd import workloads as W
 from oracle import oracle as O
 from test_gpu_bvh4 import oracle_any_tree
-from test_gpu_parity import rays_for
+from test_gpu_parity import check_build, rays_for
 
 pytestmark = pytest.mark.gpu
 
@@ -201,3 +201,61 @@ def test_commit_is_whole_for_a_trace_on_another_stream(gpu_ctx, layout):
         torch.cuda.synchronize()
         np.testing.assert_array_equal(out[0].cpu().numpy(), out[1].cpu().numpy())
     s.close()
+
+
+SMALL = [1, 2, 3, 64, 65, 255, 256, 512, 1023, 1024, 1025, 4095, 4096, 4097]
+
+
+@pytest.mark.parametrize("n", SMALL)
+def test_small_build_equals_the_oracle(gpu_ctx, n):
+    """Trees of one workgroup, up to and past the last size, with triangles that share a code; then their refit."""
+    v, f = W.soup(n, stream=W.STREAM_TEST)
+    if n >= 256:
+        f = f.copy()
+        f[5::7] = f[5]  # one code many times over
+        f[6::64] = f[6]
+        f = np.concatenate([f[:n - n // 8], f[:n // 8]]) if n // 7 < 127 else W.soup(n, stream=W.STREAM_TEST)[1]
+    say(f"small build {n}")
+    ob = O.OracleBVH(v, f)
+    s = make_scene(gpu_ctx, v, f)
+    check_build(s, ob)
+    rays = rays_for(v, 500, 8600)
+    g = trace(s, rays, "full")
+    t, prim = ob.trace(rays)[:2]
+    np.testing.assert_array_equal(g["t"].view(np.uint32), t.view(np.uint32))
+    np.testing.assert_array_equal(g["prim"], prim)
+    pairs = s.dump(0, H.DUMP_PAIRS)
+    s.update_triangles(0, (v * np.float32(2)).astype(np.float32), quality=3)
+    s.update_triangles(0, v, quality=3)
+    np.testing.assert_array_equal(s.dump(0, H.DUMP_PAIRS), pairs)  # through the parents and ranges
+    s.close()
+
+
+@pytest.mark.parametrize("sizes,rays", [([1, 2, 3, 256, 1000, 1024], 37), (SMALL[:-1], 700), (SMALL[:-1], 9000),
+                                        (SMALL, 37)],
+                         ids=["1024", "4096", "4096_many_rays", "4097"])
+def test_small_batch_equals_solo_scenes(gpu_ctx, sizes, rays):
+    import torch
+    from test_gpu_batch import make_batch
+    scenes = []
+    for k, n in enumerate(sizes):
+        v, f = W.soup(n, stream=2000 + k)
+        scenes.append((v, f, W.incoherent_rays(0 if k == 1 else rays + k, stream=3000 + k)))
+    scenes[2][0][scenes[2][1][0]] = np.nan  # one scene is walked on its pairs
+    b = make_batch(gpu_ctx, scenes)
+    stream = torch.cuda.current_stream().cuda_stream
+    for run in (b.run, b.run, b.trace):
+        run(stream)
+        torch.cuda.synchronize()
+        hits = b.hits()
+        for k, (v, f, r) in enumerate(scenes):
+            s = make_scene(gpu_ctx, v, f, keep=False)
+            np.testing.assert_array_equal(b.dump(k, H.DUMP_SIZES)[:4], s.dump(0, H.DUMP_SIZES)[:4])
+            np.testing.assert_array_equal(b.dump(k, H.DUMP_PAIRS), s.dump(0, H.DUMP_PAIRS))
+            np.testing.assert_array_equal(b.dump(k, H.DUMP_PERM), s.dump(0, H.DUMP_PERM))
+            if r.shape[0]:
+                c = trace(s, r, "compact")
+                np.testing.assert_array_equal(hits[b.ray_off[k]:b.ray_off[k + 1], 0], c["t"].view(np.uint32))
+                np.testing.assert_array_equal(hits[b.ray_off[k]:b.ray_off[k + 1], 1], c["prim"])
+            s.close()
+    b.close()
