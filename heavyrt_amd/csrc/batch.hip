@@ -706,16 +706,18 @@ __global__ __launch_bounds__(64 * kWaves) void k_b_trace(const NodePair* __restr
   }
 }
 
-// One ray per lane, no refill (kBlk threads per workgroup, full LDS stack).
+// One ray per lane, no refill (kBlk threads per workgroup, full LDS stack), one
+// fetch a step.  us, with a pair and leaf loop and now: 64 scenes of 200,000
+// triangles and 8.3 M rays 10,135 and 7,824, 8 of 4,000 and 128,000 94 and 71.
 template <int kBlk>
 __global__ __launch_bounds__(kBlk) void k_b_trace_simple(const NodePair* __restrict__ pairs_all,
                                                          const TriPre* __restrict__ tris_all, SceneOffsets off,
                                                          const Ray* __restrict__ rays, uint32_t R,
                                                          uint2* __restrict__ hits) {
-  __shared__ uint32_t stack_mem[kStackDepth * kBlk];
+  __shared__ uint32_t stack_mem[kWalkDepth * kBlk];
   const uint32_t i = blockIdx.x * kBlk + threadIdx.x;
   if (i >= R) return;
-  uint32_t* stack = stack_mem + threadIdx.x;
+  const LdsStack<kBlk> stk(stack_mem + threadIdx.x);
   const uint32_t sc = seg_of_wave(off.ray, off.S, i);
   const NodePair* P = pairs_all + off.pair[sc];
   const TriPre* Tr = tris_all + off.tri[sc];
@@ -725,40 +727,17 @@ __global__ __launch_bounds__(kBlk) void k_b_trace_simple(const NodePair* __restr
   const float tnear = r.pos_near.w;
   const bool any = r.dir_far.w <= 0.0f;
   const float3 inv = safe_inverse(d);
-  HitRec h;
-  h.t = any ? -r.dir_far.w : r.dir_far.w;
-  h.prim = kInvalid;
-  h.u = h.v = 0.0f;
-  int top = 0;
+  const MtTest tt(o, d);
+  HitRec h{any ? -r.dir_far.w : r.dir_far.w, kInvalid, 0.0f, 0.0f};
+  int top = 1;
   uint32_t cur = 0;
-  while (true) {
-    if ((cur & kLeafBit) == 0) {
-      const float4* pp = reinterpret_cast<const float4*>(P + cur);
-      const float4 lmin = pp[0], lmax = pp[1], rmin = pp[2], rmax = pp[3];
-      const float2 t0 = slab(o, inv, lmin.x, lmin.y, lmin.z, lmax.x, lmax.y, lmax.z);
-      const float2 t1 = slab(o, inv, rmin.x, rmin.y, rmin.z, rmax.x, rmax.y, rmax.z);
-      const bool h0 = (t0.x <= t0.y) && (t0.y >= tnear) && (t0.x <= h.t);
-      const bool h1 = (t1.x <= t1.y) && (t1.y >= tnear) && (t1.x <= h.t);
-      const uint32_t c0 = __float_as_uint(lmin.w), c1 = __float_as_uint(rmin.w);
-      if (h0 && h1) {
-        const bool left_first = t0.x <= t1.x;
-        cur = left_first ? c0 : c1;
-        stack[top * kBlk] = left_first ? c1 : c0;
-        top++;
-        continue;
-      }
-      if (h0 || h1) {
-        cur = h0 ? c0 : c1;
-        continue;
-      }
-    } else if (cur != kInvalid) {
-      const uint32_t s = leaf_start(cur), c = leaf_count(cur);
-      for (uint32_t k = s; k < s + c; k++) mt_test(o, d, tnear, Tr[k], h);
-      if (any && h.prim != kInvalid) break;
-    }
-    if (top == 0) break;
-    top--;
-    cur = stack[top * kBlk];
+  stk.put(0, kInvalid, true);
+  while (cur != kInvalid) {
+    const bool leaf_done = walk_step(P, Tr, tt, o, d, inv, tnear, h.t, stk, top, cur,
+                                     [&h](float t, float u, float v, uint32_t prim) {
+                                       if (t < h.t) h = HitRec{t, prim, u, v};
+                                     });
+    if (any && leaf_done && h.prim != kInvalid) break;
   }
   hits[i] = make_uint2(__float_as_uint(h.t), h.prim);
 }
@@ -894,6 +873,19 @@ const Candidate kCandidates[] = {
 #undef HRT_S
 constexpr int kNumCandidates = int(sizeof(kCandidates) / sizeof(kCandidates[0]));
 constexpr int kDefaultCandidate = 1;
+constexpr int kLaneCandidate = 11, kStreamCandidate = 14;
+
+// The candidate of a batch for which none was set or tuned: one ray per lane,
+// unless many rays walk large trees, where a wave that waits for its longest
+// ray loses more than refilling costs.  us, with candidates 1 (all of them
+// before), 11 and 14: 64 scenes of 1,000 triangles and 1 M rays 443 171 406,
+// 200 of 4,000 and 12.8 M 3,423 3,335 3,313, 8 of 80,000 and 128,000 430 235
+// 335, 64 of 80,000 and 1 M 1,129 1,023 1,030, with 4 M 3,086 2,974 2,764,
+// 200 of 20,000 and 12.8 M 5,960 6,518 5,694.
+constexpr uint64_t kStreamRays = 1u << 20;
+inline int candidate_for(uint64_t rays, bool small_scenes) {
+  return rays > kStreamRays && !small_scenes ? kStreamCandidate : kLaneCandidate;
+}
 
 int resident_blocks(const void* fn, int threads) {
   int dev = 0, cus = 0, per_cu = 0;
@@ -943,6 +935,7 @@ struct hrt_batch {
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
   int candidate = hrt::kDefaultCandidate;
+  bool chosen = false;  // the candidate was set or tuned
   std::vector<uint32_t> grid;  // per candidate, fixed at creation (no queries during capture)
   std::vector<float> tuning_ms;
   bool built = false;
@@ -1048,7 +1041,8 @@ hipError_t enqueue_candidate(hrt_batch* b, int cand, hipStream_t s) {
 
 hipError_t enqueue_trace(hrt_batch* b, hipStream_t s) {
   using namespace hrt;
-  if (!b->quads) return enqueue_candidate(b, b->candidate, s);
+  if (!b->quads)
+    return enqueue_candidate(b, b->chosen ? b->candidate : candidate_for(b->R, b->small != 0), s);
   k_b_trace_quad<<<uint32_t((b->R + kQuadRaysB - 1) / kQuadRaysB), 256, 0, s>>>(
       b->pairs, b->wide, b->differ, b->tris, offsets(b), b->rays, uint32_t(b->R), b->hits);
   return hipGetLastError();
@@ -1313,8 +1307,9 @@ hrt_status hrt_batch_candidate_info(int i, int* wavesPerGroup, int* ldsStackEntr
 hrt_status hrt_batch_set_candidate(hrt_batch* b, int i) {
   if (!b) return fail(HRT_ERR_INVALID_ARG, "batch is null");
   if (i < 0 || i >= hrt::kNumCandidates) return fail(HRT_ERR_INVALID_ARG, "no such candidate");
-  if (i != b->candidate) {
+  if (i != b->candidate || !b->chosen) {
     b->candidate = i;
+    b->chosen = true;
     drop_graph(b);
   }
   return HRT_OK;

@@ -259,3 +259,25 @@ def test_small_batch_equals_solo_scenes(gpu_ctx, sizes, rays):
                 np.testing.assert_array_equal(hits[b.ray_off[k]:b.ray_off[k + 1], 1], c["prim"])
             s.close()
     b.close()
+
+
+@pytest.mark.parametrize("sizes,rays", [([700, 3000], 40_000), ([700, 5000], 40_000), ([700, 5000], 600_000)],
+                         ids=["small", "lane", "stream"])
+def test_batch_default_kernel_equals_the_candidates(gpu_ctx, sizes, rays):
+    import torch
+    from test_gpu_batch import make_batch
+    scenes = [(*W.soup(n, stream=2100 + k), W.incoherent_rays(rays + k, stream=3100 + k)) for k, n in enumerate(sizes)]
+    for _, _, r in scenes:
+        r[1::3, 7] = -0.5  # any-hit queries among them
+    b = make_batch(gpu_ctx, scenes)
+    stream = torch.cuda.current_stream().cuda_stream
+    b.run(stream)
+    torch.cuda.synchronize()
+    ref = b.hits()
+    assert b.candidate == 1
+    for c in (1, 11, 12, 14):
+        b.set_candidate(c)
+        b.run(stream)
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(b.hits(), ref)
+    b.close()
