@@ -46,6 +46,11 @@ namespace hrt {
 namespace {
 
 constexpr int kB = 256;
+constexpr uint32_t kClimbChunk = 4096;  // leaves per workgroup in k_b_climb_chunks
+
+// Capacity of a scene's top-entry list for at most n leaves.
+inline uint32_t climb_tops_capacity(uint64_t n) { return uint32_t(kTopsPerEdge * (n / kClimbChunk + 2)); }
+
 constexpr uint32_t kBoxChunk = 4096;   // vertices per box-reduction workgroup
 
 inline uint32_t blocks(uint64_t n) { return uint32_t(std::max<uint64_t>(1, (n + kB - 1) / kB)); }
@@ -245,7 +250,7 @@ __global__ __launch_bounds__(kB) void k_b_run_compact(const uint32_t* __restrict
 // workgroup's range is arrived at only by that workgroup.
 //   k_b_leaves        kB leaves per workgroup: the leaf halves, then every
 //                     node inside the block, halves and codes in LDS
-//   k_b_climb_chunks  kRefitChunk leaves per workgroup, from the events of
+//   k_b_climb_chunks  kClimbChunk leaves per workgroup, from the events of
 //                     its blocks (arrivals that left a block), LDS exchange
 //                     of the child's far end
 //   k_b_climb_tops    one workgroup per scene, from the arrivals that left a
@@ -319,6 +324,15 @@ __device__ inline void push_top(const ManyTrees& trees, uint32_t s, uint32_t e, 
 // One thread per global leaf m: its half (box, leaf ref, far end m) starts the
 // block's climb, its triangles go into leaf order with scene-local ids, and
 // its run length into the scene's longest run.
+//
+// What bounded it were the texture addresser (98 % busy on 256 scenes of 1,000
+// to 200,000 triangles, 9.6 M together: 1,080 us), where a lane's 16-byte store
+// to a line of its own takes a cycle as its loads do, and lines fetched into
+// all eight L2s.  The triangles are therefore staged in LDS and stored in
+// order, and a node's pair, which lies in LDS as its split's two halves, by
+// four lanes together, and a triangle's indices are one load (930 us); and an
+// XCD takes consecutive blocks, so that a scene's vertices and indices, which
+// its leaves read in no order of theirs, come into one L2 (575 us).
 __global__ __launch_bounds__(kB) void k_b_leaves(const float4* __restrict__ v, const uint32_t* __restrict__ idx,
                                                  const uint32_t* __restrict__ ids_sorted,
                                                  const uint32_t* __restrict__ run_start_all,
@@ -327,110 +341,132 @@ __global__ __launch_bounds__(kB) void k_b_leaves(const float4* __restrict__ v, c
                                                  NodePair* __restrict__ pairs_all, uint4* __restrict__ slots,
                                                  uint4* __restrict__ ev, uint32_t* __restrict__ evn,
                                                  TriPre* __restrict__ tris, uint32_t* __restrict__ perm,
-                                                 uint32_t* __restrict__ max_run, uint32_t* __restrict__ err) {
-  __shared__ Half bh[kB][2];         // halves of the block's splits, one per side
+                                                 uint32_t* __restrict__ max_run, uint32_t* __restrict__ err,
+                                                 uint32_t nblk) {
+  const uint32_t blk = (blockIdx.x % kXcds) * ((nblk + kXcds - 1) / kXcds) + blockIdx.x / kXcds;
+  if (blk >= nblk) return;
+  __shared__ union {
+    Half bh[kB][2];    // halves of the block's splits, one per side
+    float4 tri[3 * kB];  // before: the block's triangles
+  } sh;
   __shared__ uint32_t bother[kB];    // exchange words, as in k_b_climb_chunks
+  __shared__ uint32_t bpair[kB];     // the pair formed at a split, kInvalid for none
   __shared__ uint32_t bcode[kB + 2];  // codes of leaves blo - 1 .. bhi + 1
-  __shared__ uint32_t nev;
+  __shared__ uint32_t nev, first, past;  // triangles [first, past) of the sorted order
   const uint32_t total = leaf_off[off.S];
-  const uint32_t blo = blockIdx.x * kB;
+  const uint32_t blo = blk * kB;
   const uint32_t bhi = min(blo + kB, max(total, blo + 1u)) - 1u;  // last leaf of the block (when it has any)
   bother[threadIdx.x] = 0u;
+  bpair[threadIdx.x] = kInvalid;
   for (uint32_t k = threadIdx.x; k < kB + 2; k += kB) {
     const uint32_t q = blo + k - 1u;  // wraps for blo = 0, k = 0: not read
     bcode[k] = (k > 0 || blo > 0) && q < total ? ucodes[q] : 0u;
   }
-  if (threadIdx.x == 0) nev = 0u;
+  if (threadIdx.x == 0) nev = first = past = 0u;
   __syncthreads();
-  const uint32_t m = blockIdx.x * kB + threadIdx.x;
+  const uint32_t m = blk * kB + threadIdx.x;
   const bool valid = m < total;
-  uint32_t s = 0, run = 0;
-  // this leaf's half, and its scene's leaves [lb, lb + L) (L > 1: it climbs)
-  Half own{};
-  bool two = false;
-  uint32_t lb = 0, L = 0;
+  uint32_t s = 0, run = 0, tb = 0, st = 0, n = 0, nv = 0;
+  uint32_t lb = 0, L = 0;  // the scene's leaves are [lb, lb + L)
+  const float4* vs = v;
   if (valid) {
     s = seg_of_wave(leaf_off, off.S, m);
     lb = leaf_off[s];
     L = leaf_off[s + 1] - lb;
-    const uint32_t tb = off.tri[s];
-    const uint32_t n = off.tri[s + 1] - tb;
-    const float4* vs = v + off.vert[s];
-    const uint32_t nv = off.vert[s + 1] - off.vert[s];
-    const uint32_t st = run_start_all[m];
-    const uint32_t e = (m - lb + 1 < L) ? run_start_all[m + 1] : n;
-    run = e - st;
+    tb = off.tri[s];
+    n = off.tri[s + 1] - tb;
+    vs = v + off.vert[s];
+    nv = off.vert[s + 1] - off.vert[s];
+    st = run_start_all[m];
+    run = ((m - lb + 1 < L) ? run_start_all[m + 1] : n) - st;
+    if (m == blo) first = tb + st;
+    if (m == bhi) past = tb + st + run;
+  }
+  __syncthreads();
+  const bool staged = past - first <= kB;  // else long runs: each lane stores its own
+  Half own{};
+  if (valid) {
     float3 lo = make_float3(kLbvhInf, kLbvhInf, kLbvhInf);
     float3 hi = make_float3(-kLbvhInf, -kLbvhInf, -kLbvhInf);
-    for (uint32_t jj = st; jj < e; jj++) {
-      const uint32_t t = ids_sorted[tb + jj];
-      const float4 a = vs[corner(idx, t, 0, nv)], b = vs[corner(idx, t, 1, nv)], c = vs[corner(idx, t, 2, nv)];
+    for (uint32_t j = tb + st; j < tb + st + run; j++) {
+      const uint32_t t = ids_sorted[j];
+      const uint3 c3 = *reinterpret_cast<const uint3*>(idx + 3 * size_t(t));
+      const float4 a = vs[min(c3.x, nv - 1)], b = vs[min(c3.y, nv - 1)], c = vs[min(c3.z, nv - 1)];
       TriPre r;
       r.a = make_float4(a.x, a.y, a.z, __uint_as_float(t - tb));
       r.e1 = make_float4(b.x - a.x, b.y - a.y, b.z - a.z, 0.0f);
       r.e2 = make_float4(c.x - a.x, c.y - a.y, c.z - a.z, 0.0f);
-      tris[tb + jj] = r;
-      perm[tb + jj] = t - tb;
+      if (staged) {
+        sh.tri[3 * (j - first)] = r.a;
+        sh.tri[3 * (j - first) + 1] = r.e1;
+        sh.tri[3 * (j - first) + 2] = r.e2;
+      } else {
+        tris[j] = r;
+      }
+      perm[j] = t - tb;
       lo = make_float3(fminf(lo.x, fminf(a.x, fminf(b.x, c.x))), fminf(lo.y, fminf(a.y, fminf(b.y, c.y))),
                        fminf(lo.z, fminf(a.z, fminf(b.z, c.z))));
       hi = make_float3(fmaxf(hi.x, fmaxf(a.x, fmaxf(b.x, c.x))), fmaxf(hi.y, fmaxf(a.y, fmaxf(b.y, c.y))),
                        fmaxf(hi.z, fmaxf(a.z, fmaxf(b.z, c.z))));
     }
-    NodePair* pairs = pairs_all + off.pair[s];
     if (L == 1) {
       // root is a leaf: pair 0 = (root leaf, empty dummy), as in lbvh.hip
+      NodePair* pairs = pairs_all + off.pair[s];
       store_box(pairs, 0, 0, lo, hi);
       store_box(pairs, 0, 1, make_float3(0.f, 0.f, 0.f), make_float3(0.f, 0.f, 0.f));
       uint32_t* pw = reinterpret_cast<uint32_t*>(pairs);
-      pw[3] = pack_leaf(st, e - st);
+      pw[3] = pack_leaf(st, run);
       pw[7] = 0u;
       pw[11] = 0x80000000u;
       pw[15] = 0u;
     } else {
-      two = true;
-      own = Half{make_uint4(__float_as_uint(lo.x), __float_as_uint(lo.y), __float_as_uint(lo.z), pack_leaf(st, e - st)),
+      own = Half{make_uint4(__float_as_uint(lo.x), __float_as_uint(lo.y), __float_as_uint(lo.z), pack_leaf(st, run)),
                  make_uint4(__float_as_uint(hi.x), __float_as_uint(hi.y), __float_as_uint(hi.z), m)};
     }
   }
+  __syncthreads();
+  if (staged) {
+    float4* t4 = reinterpret_cast<float4*>(tris + first);
+    for (uint32_t k = threadIdx.x; k < 3 * (past - first); k += kB) t4[k] = sh.tri[k];
+  }
+  __syncthreads();  // the triangles' LDS is the halves' from here on
   // Climb inside the block: nodes whose leaves all lie in [blo, bhi] are
   // formed here, with the halves in LDS.  An arrival at a split on the
   // block's edge, and a split left with one arrival, store the half in its
   // slot and become an event for k_b_climb_chunks.
-  if (two) {
-    const uint32_t le = lb + L;
-    NodePair* pairs = pairs_all + off.pair[s];
+  if (valid && L > 1) {
+    const uint32_t le = lb + L, pb = off.pair[s];
     auto side_left = [&](uint32_t l, uint32_t r) {  // b_is_left on the block's codes
       if (l == lb) return true;
       if (r + 1 == le) return false;
       return (bcode[r + 1 - blo] ^ bcode[r + 2 - blo]) < (bcode[l - blo] ^ bcode[l + 1 - blo]);
     };
-    uint32_t l = m, r = m;
-    bool leaf = true;
+    uint32_t l = m, r = m, split = kInvalid;  // the split of a formed node
     Half h0{}, h1{};
     for (;;) {
-      if (!leaf && l == lb && r + 1 == le) {
-        put_pair(pairs, 0, h0, h1);
+      if (split != kInvalid && l == lb && r + 1 == le) {
+        bpair[split - blo] = pb;
         break;
       }
       const bool left = side_left(l, r);
       const uint32_t g = left ? r : l - 1, side = left ? 0u : 1u, far = left ? l : r;
-      if (!leaf) {
+      if (split != kInvalid) {
         const uint32_t k = (left ? r : l) - lb;
-        put_pair(pairs, k, h0, h1);
+        bpair[split - blo] = pb + k;
         own = union_half(h0, h1, k, far);
       }
       if (g < blo || g >= bhi) {
         store_half(slots, 2 * g + side, own);
         const uint32_t i = atomicAdd(&nev, 1u);
-        if (i < kEventCap) ev[size_t(blockIdx.x) * kEventCap + i] = make_uint4(g, (far << 1) | side, s, 0u);
+        if (i < kEventCap) ev[size_t(blk) * kEventCap + i] = make_uint4(g, (far << 1) | side, s, 0u);
         break;
       }
-      bh[g - blo][side] = own;
+      sh.bh[g - blo][side] = own;
       const uint32_t old = __hip_atomic_exchange(&bother[g - blo], (far + 1u) | (side << 31), __ATOMIC_ACQ_REL,
                                                  __HIP_MEMORY_SCOPE_WORKGROUP);
       if (old == 0u) break;
       bother[g - blo] = kClimbDone;
-      const Half sib = bh[g - blo][side ^ 1u];
+      const Half sib = sh.bh[g - blo][side ^ 1u];
       if (left) {
         r = (old & 0x7FFFFFFFu) - 1u;
         h0 = own;
@@ -440,23 +476,31 @@ __global__ __launch_bounds__(kB) void k_b_leaves(const float4* __restrict__ v, c
         h0 = sib;
         h1 = own;
       }
-      leaf = false;
+      split = g;
     }
   }
   __syncthreads();
+  // the pairs formed here (range ends dropped)
+  for (uint32_t k = threadIdx.x; k < 4 * kB; k += kB) {
+    const uint32_t p = bpair[k >> 2];
+    if (p == kInvalid) continue;
+    uint4 w = reinterpret_cast<const uint4*>(sh.bh[k >> 2])[k & 3u];
+    if (k & 1u) w.w = 0u;
+    reinterpret_cast<uint4*>(pairs_all + p)[k & 3u] = w;
+  }
   // splits left with one arrival (the other child crosses the block's edge)
   if (blo < total && threadIdx.x < bhi - blo) {
     const uint32_t v = bother[threadIdx.x];
     if (v != 0u && v != kClimbDone) {
       const uint32_t g = blo + threadIdx.x, side = v >> 31, far = (v & 0x7FFFFFFFu) - 1u;
-      store_half(slots, 2 * g + side, bh[threadIdx.x][side]);
+      store_half(slots, 2 * g + side, sh.bh[threadIdx.x][side]);
       const uint32_t i = atomicAdd(&nev, 1u);
-      if (i < kEventCap) ev[size_t(blockIdx.x) * kEventCap + i] = make_uint4(g, (far << 1) | side, s, 0u);
+      if (i < kEventCap) ev[size_t(blk) * kEventCap + i] = make_uint4(g, (far << 1) | side, s, 0u);
     }
   }
   __syncthreads();
   if (threadIdx.x == 0) {
-    evn[blockIdx.x] = min(nev, kEventCap);
+    evn[blk] = min(nev, kEventCap);
     if (nev > kEventCap) __hip_atomic_store(err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
   // Longest run per scene.  A wave's leaves span one or a few scenes: the
@@ -468,17 +512,16 @@ __global__ __launch_bounds__(kB) void k_b_leaves(const float4* __restrict__ v, c
     const uint32_t ls = __shfl(s, leader);
     const bool mine = valid && s == ls;
     uint32_t mv = mine ? run : 0u;
-    for (int o = 32; o > 0; o >>= 1) mv = max(mv, __shfl_xor(mv, o));
-    if (int(threadIdx.x & 63) == leader) atomicMax(&max_run[ls], mv);
+    raise_max(&max_run[ls], mv);
     todo &= ~__ballot(mine);
   }
 }
 
-// Chunk pass: one workgroup per kRefitChunk leaves, from the events of the
+// Chunk pass: one workgroup per kClimbChunk leaves, from the events of the
 // chunk's leaf-pass blocks.  other[k]: 0 before any arrival at split
 // chunk_lo + k, then the first child's (far end + 1) | side << 31, then
 // kClimbDone.
-constexpr uint32_t kBlocksPerChunk = kRefitChunk / kB;
+constexpr uint32_t kBlocksPerChunk = kClimbChunk / kB;
 
 __global__ __launch_bounds__(kRefitThreads) void k_b_climb_chunks(ManyTrees trees, const uint32_t* __restrict__ ucodes,
                                                                  uint4* __restrict__ slots, NodePair* pairs_all,
@@ -487,13 +530,13 @@ __global__ __launch_bounds__(kRefitThreads) void k_b_climb_chunks(ManyTrees tree
                                                                  uint32_t* __restrict__ tops,
                                                                  uint32_t* __restrict__ ntops,
                                                                  uint32_t* __restrict__ err) {
-  __shared__ uint32_t other[kRefitChunk];
+  __shared__ uint32_t other[kClimbChunk];
   __shared__ uint32_t base[kBlocksPerChunk + 1];
-  for (uint32_t k = threadIdx.x; k < kRefitChunk; k += kRefitThreads) other[k] = 0u;
+  for (uint32_t k = threadIdx.x; k < kClimbChunk; k += kRefitThreads) other[k] = 0u;
   const uint32_t total = trees.leaves();
-  const uint32_t chunk_lo = blockIdx.x * kRefitChunk;
+  const uint32_t chunk_lo = blockIdx.x * kClimbChunk;
   if (chunk_lo >= total) return;  // the whole workgroup
-  const uint32_t chunk_hi = min(chunk_lo + kRefitChunk, total) - 1u;
+  const uint32_t chunk_hi = min(chunk_lo + kClimbChunk, total) - 1u;
   const uint32_t b0 = chunk_lo / kB, nb = chunk_hi / kB - b0 + 1u;
   if (threadIdx.x == 0) {
     uint32_t a = 0;
@@ -1011,10 +1054,12 @@ hipError_t enqueue_build(hrt_batch* b, hipStream_t s) {
   k_b_run_flags<<<blocks(T), kB, 0, s>>>(kin, off, T, b->flags);
   if ((e = scan_exclusive(b->flags, b->pos, T, b->scan_tmp, s)) != hipSuccess) return e;
   k_b_run_compact<<<blocks(T), kB, 0, s>>>(kin, b->flags, b->pos, off, T, b->run_start, b->ucodes, b->leaf_off);
-  k_b_leaves<<<blocks(T), kB, 0, s>>>(b->verts, b->idx, vin, b->run_start, b->leaf_off, off, b->ucodes, b->pairs,
-                                      b->slots, b->ev, b->evn, b->tris, b->perm, b->max_run, b->refit_err);
+  const uint32_t nblk = blocks(T);
+  k_b_leaves<<<(nblk + kXcds - 1) / kXcds * kXcds, kB, 0, s>>>(
+      b->verts, b->idx, vin, b->run_start, b->leaf_off, off, b->ucodes, b->pairs, b->slots, b->ev, b->evn, b->tris,
+      b->perm, b->max_run, b->refit_err, nblk);
   const ManyTrees trees{b->leaf_off, off.pair, off.tops, b->S};
-  k_b_climb_chunks<<<uint32_t((T + kRefitChunk - 1) / kRefitChunk), kRefitThreads, 0, s>>>(
+  k_b_climb_chunks<<<uint32_t((T + kClimbChunk - 1) / kClimbChunk), kRefitThreads, 0, s>>>(
       trees, b->ucodes, b->slots, b->pairs, b->ev, b->evn, b->tops, b->ntops, b->refit_err);
   k_b_climb_tops<<<b->S, kRefitTopsThreads, 0, s>>>(trees, b->ucodes, b->slots, b->pairs, b->tops, b->ntops,
                                                     b->arrive);
@@ -1142,7 +1187,7 @@ hrt_status hrt_batch_create(hrt_ctx* ctx, uint32_t nScenes, const uint32_t* nVer
     T += nTris[s];
     R += nRays[s];
     P += std::max<uint32_t>(nTris[s] > 1 ? nTris[s] - 1 : 1, 1);
-    TOPS += refit_tops_capacity(nTris[s]);
+    TOPS += climb_tops_capacity(nTris[s]);
     most = std::max(most, nTris[s]);
     all_small = all_small && nTris[s] <= kSmallMax && nVerts[s] <= kSmallVerts;
   }

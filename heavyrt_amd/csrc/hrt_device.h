@@ -637,6 +637,15 @@ __device__ inline int kdelta(const uint32_t* __restrict__ c, int L, int i, int j
   return x == 0 ? 32 : int(__builtin_clz(x));
 }
 
+// Raises *word to the largest v of the wave (all lanes call it).  Most waves
+// find it that large already and leave out the atomic: one address takes an
+// atomic every 7 to 12 ns, whoever sends it.
+__device__ inline void raise_max(uint32_t* word, uint32_t v) {
+  for (int o = 32; o > 0; o >>= 1) v = max(v, uint32_t(__shfl_xor(v, o)));
+  if ((threadIdx.x & 63u) == 0 && v > __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+    atomicMax(word, v);
+}
+
 // Writes one child box of node pair p (side 0 = left, 1 = right).
 __device__ inline void store_box(NodePair* pairs, uint32_t p, uint32_t side, float3 lo, float3 hi) {
   uint32_t* pw = reinterpret_cast<uint32_t*>(pairs + p) + side * 8;

@@ -65,12 +65,14 @@ struct TriSource {
                        (fminf(v1.z, fminf(v2.z, v3.z)) + fmaxf(v1.z, fmaxf(v2.z, v3.z))) * 0.5f);
   }
   __device__ void corners(uint32_t t, float4& a, float4& b, float4& c) const {
-    a = v[idx[3 * t + 0]];
-    b = v[idx[3 * t + 1]];
-    c = v[idx[3 * t + 2]];
+    const uint3 k = *reinterpret_cast<const uint3*>(idx + 3 * size_t(t));  // one load
+    a = v[k.x];
+    b = v[k.y];
+    c = v[k.z];
   }
   __device__ void prim_box(uint32_t t, float3& lo, float3& hi) const {
-    const float4 a = v[idx[3 * t + 0]], b = v[idx[3 * t + 1]], c = v[idx[3 * t + 2]];
+    float4 a, b, c;
+    corners(t, a, b, c);
     lo = make_float3(fminf(a.x, fminf(b.x, c.x)), fminf(a.y, fminf(b.y, c.y)), fminf(a.z, fminf(b.z, c.z)));
     hi = make_float3(fmaxf(a.x, fmaxf(b.x, c.x)), fmaxf(a.y, fmaxf(b.y, c.y)), fmaxf(a.z, fmaxf(b.z, c.z)));
   }
@@ -379,6 +381,10 @@ __global__ __launch_bounds__(kBlock) void k_karras(const uint32_t* __restrict__ 
 // {A, origId}, {B - A}, {C - A} (BVH2CommonRT_host.cpp:45-64,
 // BVH2CommonRT.cpp:26-27) and the permutation (perm may be null: a refit
 // keeps it).  meta[1] gets the longest run.
+// An atomic per wave on that one word took 128 us with 1.07 M triangles (16,700
+// waves) and 790 with 4.2 M; without it and laid out as the batched build's
+// leaf pass (k_b_leaves: an XCD takes consecutive leaves, the records are
+// staged in LDS and stored in order) 54 and 290.
 template <class Src>
 __global__ __launch_bounds__(kBlock) void k_leaves(Src src, const uint32_t* __restrict__ ids_sorted,
                                                    const uint32_t* __restrict__ run_start,
@@ -386,11 +392,26 @@ __global__ __launch_bounds__(kBlock) void k_leaves(Src src, const uint32_t* __re
                                                    NodePair* __restrict__ pairs,
                                                    const uint32_t* __restrict__ parent_leaf,
                                                    TriPre* __restrict__ tris, uint32_t* __restrict__ perm) {
+  __shared__ float4 staged[Src::kTris ? 3 * kBlock : 1];
   const uint32_t L = meta[0];
-  const uint32_t m = blockIdx.x * kBlock + threadIdx.x;
-  if (m >= L) return;
-  const uint32_t s = run_start[m];
-  const uint32_t e = (m + 1 < L) ? run_start[m + 1] : ntris;
+  const uint32_t blk = (blockIdx.x % kXcds) * (gridDim.x / kXcds) + blockIdx.x / kXcds;
+  const uint32_t m = blk * kBlock + threadIdx.x;
+  const bool valid = m < L;
+  uint32_t s = 0, e = 0, first = 0, past = 0;
+  bool stage = false;
+  if (valid) {
+    s = run_start[m];
+    e = (m + 1 < L) ? run_start[m + 1] : ntris;
+  }
+  if constexpr (Src::kTris) {
+    // the block's triangles: [first, past) of the sorted order
+    const uint32_t ml = blk * kBlock;
+    if (ml < L) {
+      first = run_start[ml];
+      past = ml + kBlock < L ? run_start[ml + kBlock] : ntris;
+      stage = past - first <= uint32_t(kBlock);  // else long runs: each lane stores its own
+    }
+  }
   float3 lo = make_float3(kLbvhInf, kLbvhInf, kLbvhInf);
   float3 hi = make_float3(-kLbvhInf, -kLbvhInf, -kLbvhInf);
   for (uint32_t j = s; j < e; j++) {
@@ -403,7 +424,13 @@ __global__ __launch_bounds__(kBlock) void k_leaves(Src src, const uint32_t* __re
       r.a = make_float4(va.x, va.y, va.z, __uint_as_float(t));
       r.e1 = make_float4(vb.x - va.x, vb.y - va.y, vb.z - va.z, 0.0f);
       r.e2 = make_float4(vc.x - va.x, vc.y - va.y, vc.z - va.z, 0.0f);
-      tris[j] = r;
+      if (stage) {
+        staged[3 * (j - first)] = r.a;
+        staged[3 * (j - first) + 1] = r.e1;
+        staged[3 * (j - first) + 2] = r.e2;
+      } else {
+        tris[j] = r;
+      }
       if (perm) perm[j] = t;
       a = make_float3(fminf(va.x, fminf(vb.x, vc.x)), fminf(va.y, fminf(vb.y, vc.y)), fminf(va.z, fminf(vb.z, vc.z)));
       b = make_float3(fmaxf(va.x, fmaxf(vb.x, vc.x)), fmaxf(va.y, fmaxf(vb.y, vc.y)), fmaxf(va.z, fmaxf(vb.z, vc.z)));
@@ -413,7 +440,15 @@ __global__ __launch_bounds__(kBlock) void k_leaves(Src src, const uint32_t* __re
     lo = make_float3(fminf(lo.x, a.x), fminf(lo.y, a.y), fminf(lo.z, a.z));
     hi = make_float3(fmaxf(hi.x, b.x), fmaxf(hi.y, b.y), fmaxf(hi.z, b.z));
   }
-  atomicMax(&meta[1], e - s);  // one address: combined across the wave
+  if constexpr (Src::kTris) {
+    __syncthreads();
+    if (stage) {
+      float4* t4 = reinterpret_cast<float4*>(tris + first);
+      for (uint32_t k = threadIdx.x; k < 3 * (past - first); k += kBlock) t4[k] = staged[k];
+    }
+  }
+  raise_max(&meta[1], e - s);
+  if (!valid) return;
   if (L == 1) {
     // Root is a leaf: pair 0 = (root leaf, empty dummy), as the reference's
     // peach layout stores it (lbvh.cpp:497-504, cbvh.h:28-36).
@@ -512,13 +547,25 @@ __global__ __launch_bounds__(kBlock) void k_expand_vertices(const float* __restr
   out[i] = make_float4(p[0], p[1], p[2], 1.0f);
 }
 
+// The largest of n words (16-byte aligned) into *out, which starts at 0; an
+// atomic per workgroup (per wave they took 50 us with 4,096 waves).
 __global__ __launch_bounds__(kBlock) void k_largest_index(const uint32_t* __restrict__ idx, uint64_t n,
                                                           uint32_t* __restrict__ out) {
+  __shared__ uint32_t part[kBlock / 64];
+  const uint64_t n4 = n / 4, i0 = uint64_t(blockIdx.x) * kBlock + threadIdx.x, step = uint64_t(gridDim.x) * kBlock;
   uint32_t m = 0;
-  for (uint64_t i = uint64_t(blockIdx.x) * kBlock + threadIdx.x; i < n; i += uint64_t(gridDim.x) * kBlock)
-    m = max(m, idx[i]);
+  for (uint64_t i = i0; i < n4; i += step) {
+    const uint4 w = reinterpret_cast<const uint4*>(idx)[i];
+    m = max(m, max(max(w.x, w.y), max(w.z, w.w)));
+  }
+  if (i0 < n - 4 * n4) m = max(m, idx[4 * n4 + i0]);
   for (int o = 32; o > 0; o >>= 1) m = max(m, uint32_t(__shfl_xor(m, o)));
-  if ((threadIdx.x & 63) == 0) atomicMax(out, m);
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = m;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < kBlock / 64; w++) m = max(m, part[w]);
+    atomicMax(out, m);
+  }
 }
 
 // One WideNode per internal node: three pairs in, 128 B out; *differ is set when
@@ -549,6 +596,8 @@ __global__ __launch_bounds__(kBlock) void k_wt_tris(const float4* __restrict__ v
 }
 
 inline uint32_t blocks_for(uint64_t n) { return uint32_t((n + kBlock - 1) / kBlock); }
+// a multiple of kXcds (k_leaves)
+inline uint32_t leaf_blocks(uint64_t n) { return (blocks_for(n) + kXcds - 1) / kXcds * kXcds; }
 
 }  // namespace
 
@@ -760,9 +809,9 @@ hipError_t lbvh_build(Blas& b, const Src& src, uint32_t box_items, hipStream_t s
   auto take = [&](size_t n) { size_t o = words; words += (n + 63) & ~size_t(63); return o; };
   const size_t o_ka = take(w_codes), o_va = take(w_codes), o_kb = take(w_codes), o_vb = take(w_codes);
   const size_t o_sort = take(w_sort), o_scan = take(w_scan);
-  const size_t o_flags = take(N), o_pos = take(N), o_uc = take(N), o_arr = take(N);
-  const uint32_t tops_cap = refit_tops_capacity(N);
-  const size_t o_tops = take(tops_cap);
+  const size_t w_arr = N + refit_groups(N) + 1;  // the refit's arrival counters and list counts
+  const size_t o_flags = take(N), o_pos = take(N), o_uc = take(N), o_arr = take(w_arr);
+  const size_t o_tops = take(refit_list_words(N));
   const size_t o_part = take(size_t(box_parts) * 8), o_box = take(16);
   uint32_t* base = nullptr;
   HRT_CHECK(b.mem->alloc(&base, words * 4));
@@ -779,8 +828,7 @@ hipError_t lbvh_build(Blas& b, const Src& src, uint32_t box_items, hipStream_t s
 
   hipError_t err = hipSuccess;
   do {
-    // meta: [0] leaves, [1] longest run, [2] refit top entries, [3] refit
-    // overflow, [4] sort look-back timeout; flags stay zero unless a check fails
+    // meta: [0] leaves, [1] longest run, [3] refit overflow, [4] sort look-back timeout; flags stay zero unless a check fails
     k_fill<<<1, kBlock, 0, s>>>(meta, 64, 0u);
     k_box_partial<Src><<<box_parts, kBlock, 0, s>>>(src, part);
     k_box_final<<<1, kBlock, 0, s>>>(part, box_parts, box, box + 8, cubic);
@@ -794,16 +842,14 @@ hipError_t lbvh_build(Blas& b, const Src& src, uint32_t box_items, hipStream_t s
     k_run_flags<<<blocks_for(N), kBlock, 0, s>>>(kin, uint32_t(N), flags);
     if ((err = exclusive_scan(flags, pos, N, stmp, s)) != hipSuccess) break;
     k_run_compact<<<blocks_for(N), kBlock, 0, s>>>(kin, flags, pos, uint32_t(N), rs, uc, meta);
-    k_fill<<<fill_blocks(N), kBlock, 0, s>>>(arrive, N, 0u);
+    k_fill<<<fill_blocks(w_arr), kBlock, 0, s>>>(arrive, w_arr, 0u);
     k_karras<<<blocks_for(N), kBlock, 0, s>>>(uc, rs, meta, uint32_t(N), b.pairs, b.parent, pleaf, range,
                                               b.karras_lr);
-    k_leaves<Src><<<blocks_for(N), kBlock, 0, s>>>(src, vin, rs, meta, uint32_t(N), b.pairs, pleaf, b.tris,
+    k_leaves<Src><<<leaf_blocks(N), kBlock, 0, s>>>(src, vin, rs, meta, uint32_t(N), b.pairs, pleaf, b.tris,
                                                    b.perm);
-    // meta[2] counts the refit's top entries, meta[3] flags an overflow (both zeroed above)
-    const OneTree tree{meta, tops_cap};
-    k_refit_chunks<OneTree><<<uint32_t((N + kRefitChunk - 1) / kRefitChunk), kRefitThreads, 0, s>>>(
-        tree, b.pairs, b.parent, pleaf, range, tops, meta + 2, meta + 3);
-    k_refit_tops<OneTree><<<1, kRefitTopsThreads, 0, s>>>(tree, b.pairs, b.parent, tops, meta + 2, arrive);
+    // meta[3] flags an overflow of the refit's lists (zeroed above)
+    if ((err = refit_boxes(meta, N, b.pairs, b.parent, pleaf, range, tops, arrive + N, arrive, meta + 3, s)) != hipSuccess)
+      break;
     finish(vin);
     if ((err = hipGetLastError()) != hipSuccess) break;
     if (b.keep_debug) {
@@ -856,9 +902,9 @@ hipError_t blas_refit(Blas& b, hipStream_t s) {
   const TriSource src{b.verts, b.idx, b.nverts};
   const int box_parts = int(std::min<uint64_t>(1024, std::max<uint64_t>(1, (b.nverts + kBlock - 1) / kBlock)));
   uint32_t* base = nullptr;
-  const uint32_t tops_cap = refit_tops_capacity(N);
-  const size_t o_tops = (N + 63) & ~size_t(63);
-  const size_t o_part = o_tops + ((tops_cap + 63) & ~size_t(63));
+  const size_t w_arr = N + refit_groups(N) + 1;
+  const size_t o_tops = (w_arr + 63) & ~size_t(63);
+  const size_t o_part = o_tops + ((refit_list_words(N) + 63) & ~size_t(63));
   HRT_CHECK(b.mem->alloc(&base, 4 * (o_part + 8 * size_t(box_parts) + 16)));
   Readback back(b.mem);
   uint32_t* arrive = base;
@@ -867,17 +913,15 @@ hipError_t blas_refit(Blas& b, hipStream_t s) {
   float* box = reinterpret_cast<float*>(base + o_part + 8 * size_t(box_parts));
   k_box_partial<TriSource><<<box_parts, kBlock, 0, s>>>(src, part);
   k_box_final<<<1, kBlock, 0, s>>>(part, box_parts, box, box + 8, 0);
-  k_fill<<<fill_blocks(N), kBlock, 0, s>>>(arrive, N, 0u);
-  k_fill<<<1, kBlock, 0, s>>>(b.meta + 2, 2, 0u);  // top-entry count, overflow flag
+  k_fill<<<fill_blocks(w_arr), kBlock, 0, s>>>(arrive, w_arr, 0u);
+  k_fill<<<1, kBlock, 0, s>>>(b.meta + 2, 2, 0u);  // the overflow flag
   // the kept permutation gives the leaf order; it is not rewritten
-  k_leaves<TriSource><<<blocks_for(N), kBlock, 0, s>>>(src, b.perm, b.leaf_run, b.meta, uint32_t(N), b.pairs,
+  k_leaves<TriSource><<<leaf_blocks(N), kBlock, 0, s>>>(src, b.perm, b.leaf_run, b.meta, uint32_t(N), b.pairs,
                                                        b.parent_leaf, b.tris, nullptr);
-  const OneTree tree{b.meta, tops_cap};
-  k_refit_chunks<OneTree><<<uint32_t((N + kRefitChunk - 1) / kRefitChunk), kRefitThreads, 0, s>>>(
-      tree, b.pairs, b.parent, b.parent_leaf, b.node_range, tops, b.meta + 2, b.meta + 3);
-  k_refit_tops<OneTree><<<1, kRefitTopsThreads, 0, s>>>(tree, b.pairs, b.parent, tops, b.meta + 2, arrive);
+  hipError_t err = refit_boxes(b.meta, N, b.pairs, b.parent, b.parent_leaf, b.node_range, tops, arrive + N, arrive,
+                               b.meta + 3, s);
   b.wide_made = false;
-  hipError_t err = b.wide ? blas_build_wide(b, s) : hipGetLastError();
+  if (err == hipSuccess && b.wide) err = blas_build_wide(b, s);
   if (err == hipSuccess) err = back.read(0, b.meta, 4, s);
   if (err == hipSuccess) err = back.read(8, box, 8, s);
   const hipError_t werr = hipStreamSynchronize(s);
@@ -944,7 +988,7 @@ hipError_t expand_vertices(const float* raw, uint32_t stride, uint32_t nverts, f
 
 hipError_t largest_index(const uint32_t* idx, uint64_t n, uint32_t* out, hipStream_t s) {
   k_fill<<<1, kBlock, 0, s>>>(out, 1, 0u);
-  k_largest_index<<<fill_blocks(n), kBlock, 0, s>>>(idx, n, out);
+  k_largest_index<<<std::min<uint32_t>(512, blocks_for((n + 3) / 4)), kBlock, 0, s>>>(idx, n, out);
   return hipGetLastError();
 }
 

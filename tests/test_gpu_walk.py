@@ -281,3 +281,27 @@ def test_batch_default_kernel_equals_the_candidates(gpu_ctx, sizes, rays):
         torch.cuda.synchronize()
         np.testing.assert_array_equal(b.hits(), ref)
     b.close()
+
+
+@pytest.mark.parametrize("n,dup", [(4097, 1), (16384, 1), (16385, 130), (33_000, 200), (70_000, 1)])
+def test_leaf_pass_and_refit_at_group_edges(gpu_ctx, n, dup):
+    """Trees over one or several of the refit's groups, with runs longer than the leaf pass stages."""
+    v, f = W.soup(n, stream=W.STREAM_TEST)
+    f = f.copy()
+    for k in range(0, dup - 1):  # a run of up to 127 and many of two and three
+        f[(k * 71) % n if k < 100 else (k * 37) % n] = f[n // 2 if k < 100 else n // 3]
+    ob = O.OracleBVH(v, f)
+    s = make_scene(gpu_ctx, v, f)
+    check_build(s, ob)
+    pairs, perm = s.dump(0, H.DUMP_PAIRS), s.dump(0, H.DUMP_PERM)
+    rays = rays_for(v, 2000, 8700)
+    g = trace(s, rays, "full")
+    t, prim = ob.trace(rays)[:2]
+    np.testing.assert_array_equal(g["t"].view(np.uint32), t.view(np.uint32))
+    np.testing.assert_array_equal(g["prim"], prim)
+    s.update_triangles(0, (v * np.float32(2)).astype(np.float32), quality=3)
+    assert (s.dump(0, H.DUMP_PAIRS) != pairs).any()
+    s.update_triangles(0, v, quality=3)
+    np.testing.assert_array_equal(s.dump(0, H.DUMP_PAIRS), pairs)
+    np.testing.assert_array_equal(s.dump(0, H.DUMP_PERM), perm)
+    s.close()
