@@ -31,9 +31,16 @@ constexpr int kWave = 64;
 constexpr int kBlock4 = 64;
 constexpr int kRefillAt4 = 40;
 // LDS stack entries per lane of the one-ray-per-lane kernels (the rest spill
-// to global memory).  Deep, incoherent nearest-hit walks push often and
-// measured slower with spills, so BVH4 keeps its whole stack in LDS.
-constexpr int kSimpleLds4 = 48;
+// to global memory).  48 keep most walks in LDS but only 13 waves on a CU,
+// which hide too little of a node's fetch; 24 keep 26.  ms a call with 48 / 32
+// / 24 / 16: 4,194,304 random rays sorted on FP16 nodes of a 4,194,304-triangle
+// soup 8.8 7.1 6.4 7.0; 1,000,000 on 1,000,000 triangles 1.55 1.34 1.20 1.29;
+// 1,000,000 bounced rays over 500,000 triangles, FP16 0.77 0.67 0.61 0.58.
+constexpr int kSimpleLds4 = 24;
+constexpr int kStatsLds4 = 48;  // the counting variant, whose spill area grows with the rays
+// Rays a launch: the spill area of a larger one is the size of this one's (650
+// MB), and where that cannot be had, of smaller ones' down to the least.
+constexpr uint64_t kLaunchRays = 1u << 22, kLaunchRaysMin = 1u << 16;
 // Nearest-hit batches of at least this many rays on a tree (nodes and
 // triangles) of at least this many bytes are sorted into coherent waves before
 // they are traced.  A tree well inside the 256 MB MALL gains nothing that pays
@@ -184,9 +191,7 @@ __device__ inline void trace4_one(const void* __restrict__ quads, const TriPre* 
       uint32_t ch[4];
       visit_quad<kFp16, kForceAny && kFp16>(quads, cur, o, inv, oi, fz, tt, tnear, h.t, tm, ch);
       if (kStats) nvisits++;
-      if (tm[3] < kMaxFloat) stk.push(top, ch[3]);
-      if (tm[2] < kMaxFloat) stk.push(top, ch[2]);
-      if (tm[1] < kMaxFloat) stk.push(top, ch[1]);
+      stk.push_masked3(top, tm[3] < kMaxFloat, ch[3], tm[2] < kMaxFloat, ch[2], tm[1] < kMaxFloat, ch[1]);
       if (tm[0] < kMaxFloat) cur = ch[0];
       else pop = true;
     }
@@ -217,10 +222,11 @@ __global__ __launch_bounds__(kBlock4) void k_trace4_simple(const void* __restric
                                                            const Ray* __restrict__ rays, uint64_t n, void* out,
                                                            int format, uint2 ids, uint32_t* __restrict__ stats,
                                                            uint32_t* __restrict__ spill) {
-  __shared__ uint32_t stack_mem[kSimpleLds4 * kBlock4];
+  constexpr int kLds = kStats ? kStatsLds4 : kSimpleLds4;
+  __shared__ uint32_t stack_mem[kLds * kBlock4];
   const uint64_t i = uint64_t(blockIdx.x) * kBlock4 + threadIdx.x;
   if (i >= n) return;
-  const ShortStack<kSimpleLds4, kBlock4> stk{stack_mem + threadIdx.x, spill + i, gridDim.x * kBlock4};
+  const ShortStack<kLds, kBlock4> stk{stack_mem + threadIdx.x, spill + i, gridDim.x * kBlock4};
   trace4_one<kForceAny, kFp16, kStats, Tri>(quads, tris, rays, i, out, format, ids, stats, stk);
 }
 
@@ -232,11 +238,11 @@ __global__ __launch_bounds__(kBlock4) void k_trace4_simple(const void* __restric
 // take unequal time (camera rays: a region of the screen each).
 template <bool kFp16, class Tri>
 __global__ __launch_bounds__(kBlock4) void k_trace4_sorted(const void* __restrict__ quads,
-                                                           const TriPre* __restrict__ tris,
-                                                           const Ray* __restrict__ rays, uint64_t n, void* out,
-                                                           int format, uint2 ids, uint32_t* __restrict__ spill,
-                                                           const uint32_t* const* __restrict__ order_slot,
-                                                           uint32_t* __restrict__ queue) {
+                                                         const TriPre* __restrict__ tris,
+                                                         const Ray* __restrict__ rays, uint64_t n, void* out,
+                                                         int format, uint2 ids, uint32_t* __restrict__ spill,
+                                                         const uint32_t* const* __restrict__ order_slot,
+                                                         uint32_t* __restrict__ queue) {
   __shared__ uint32_t stack_mem[kSimpleLds4 * kBlock4];
   const uint32_t* __restrict__ order = *order_slot;
   const ShortStack<kSimpleLds4, kBlock4> stk{stack_mem + threadIdx.x, spill + blockIdx.x * kBlock4 + threadIdx.x,
@@ -262,8 +268,6 @@ __global__ __launch_bounds__(kBlock4) void k_trace4_sorted(const void* __restric
 // from a wave-local ray pool (the BVH2 kernel in trace.hip describes the
 // scheme): a lane parks the first leaf it finds and keeps descending until
 // the wave tests leaves together; the answer does not depend on the order.
-// (Nearest hits stay on k_trace4_simple: on deep, heavily overlapping trees
-// its 48-entry LDS stack beats a short LDS stack with global spill.)
 // Src gives ray i: StoredRays reads it from HBM, AoRays makes AO sample i
 // from its pixel's frame; both trace every ray in the launch's tree and
 // write answer i at out[i].  ServeRays (kSegments) belongs to the server:
@@ -689,35 +693,40 @@ hipError_t launch_simple4(const Blas& b, const TraceArgs& a, hipStream_t stream)
         make_uint2(a.inst_id, a.geom_id));
     return hipGetLastError();
   }
-  const uint32_t blocks = uint32_t((a.n + kBlock4 - 1) / kBlock4);
   const void* q = kFp16 ? static_cast<const void*>(b.quads16) : static_cast<const void*>(b.quads32);
-  // stack entries beyond the LDS part, per lane (none while LDS holds them all)
-  uint32_t* spill = nullptr;
-  hipError_t e = hipSuccess;
-  if (kSimpleLds4 < kStackDepth4 &&
-      (e = hipMallocAsync(reinterpret_cast<void**>(&spill),
-                          sizeof(uint32_t) * size_t(blocks) * kBlock4 * (kStackDepth4 - kSimpleLds4), stream)) !=
-          hipSuccess)
-    return e;
   const uint2 ids = make_uint2(a.inst_id, a.geom_id);
   const TriPre* tris = tri_records<Tri>(b);
-  if (a.anyhit) {
-    if (a.stats)
-      k_trace4_simple<true, kFp16, true, Tri><<<blocks, kBlock4, 0, stream>>>(q, tris, a.rays, a.n, a.out, a.format,
-                                                                             ids, a.stats, spill);
-    else
-      k_trace4_simple<true, kFp16, false, Tri><<<blocks, kBlock4, 0, stream>>>(q, tris, a.rays, a.n, a.out, a.format,
-                                                                              ids, nullptr, spill);
-  } else {
-    if (a.stats)
-      k_trace4_simple<false, kFp16, true, Tri><<<blocks, kBlock4, 0, stream>>>(q, tris, a.rays, a.n, a.out, a.format,
-                                                                              ids, a.stats, spill);
-    else
-      k_trace4_simple<false, kFp16, false, Tri><<<blocks, kBlock4, 0, stream>>>(q, tris, a.rays, a.n, a.out,
-                                                                               a.format, ids, nullptr, spill);
+  // stack entries beyond the LDS part, per lane; launches of kLaunchRays bound them, smaller ones with less memory
+  const size_t lane_words = kStackDepth4 - (a.stats ? kStatsLds4 : kSimpleLds4);
+  uint64_t share = a.stats ? a.n : std::min(a.n, kLaunchRays);
+  uint32_t* spill = nullptr;
+  hipError_t e;
+  while (true) {
+    const uint64_t lanes = (share + kBlock4 - 1) / kBlock4 * kBlock4;
+    e = hipMallocAsync(reinterpret_cast<void**>(&spill), sizeof(uint32_t) * lanes * lane_words, stream);
+    if (e != hipErrorOutOfMemory || a.stats || share <= kLaunchRaysMin) break;
+    (void)hipGetLastError();
+    share = std::max(share / 4, kLaunchRaysMin);
   }
-  e = hipGetLastError();
-  const hipError_t f = spill ? hipFreeAsync(spill, stream) : hipSuccess;
+  if (e != hipSuccess) return e;
+  for (uint64_t at = 0; at < a.n && e == hipSuccess; at += share) {
+    const uint64_t n = std::min(a.n - at, share);
+    const uint32_t blocks = uint32_t((n + kBlock4 - 1) / kBlock4);
+    const Ray* rays = a.rays + at;
+    if (a.anyhit) {  // (without counters: launch_any4)
+      k_trace4_simple<true, kFp16, true, Tri><<<blocks, kBlock4, 0, stream>>>(q, tris, rays, n, a.out, a.format, ids,
+                                                                             a.stats, spill);
+    } else if (a.stats) {
+      k_trace4_simple<false, kFp16, true, Tri><<<blocks, kBlock4, 0, stream>>>(q, tris, rays, n, a.out, a.format, ids,
+                                                                              a.stats, spill);
+    } else {
+      char* out = static_cast<char*>(a.out) + at * (a.format == kHitCompact ? sizeof(uint2) : sizeof(HitOutFull));
+      k_trace4_simple<false, kFp16, false, Tri><<<blocks, kBlock4, 0, stream>>>(q, tris, rays, n, out, a.format, ids,
+                                                                               nullptr, spill);
+    }
+    e = hipGetLastError();
+  }
+  const hipError_t f = hipFreeAsync(spill, stream);
   return e != hipSuccess ? e : f;
 }
 

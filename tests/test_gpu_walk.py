@@ -305,3 +305,29 @@ def test_leaf_pass_and_refit_at_group_edges(gpu_ctx, n, dup):
     np.testing.assert_array_equal(s.dump(0, H.DUMP_PAIRS), pairs)
     np.testing.assert_array_equal(s.dump(0, H.DUMP_PERM), perm)
     s.close()
+
+
+@pytest.mark.parametrize("full", [False, True], ids=["compact", "full"])
+def test_bvh4_launches_of_a_large_batch_join(gpu_ctx, full):
+    """More rays than one launch takes: the seam's records are those of the same rays traced by themselves."""
+    import torch
+    v, f = W.soup(3000, stream=W.STREAM_TEST)
+    s = H.Scene(gpu_ctx)
+    s.add_instance(s.add_triangles(v, f))
+    s.commit(layout=H.LAYOUT_BVH4_FP16)
+    n, seam = (1 << 22) + 65, 1 << 22
+    rays = torch.from_numpy(np.tile(rays_for(v, 4096, 8800), (n // 4096 + 1, 1))[:n]).cuda()
+    rays[:, 0] += torch.arange(n, device="cuda") * 1e-8
+    words, fmt = (8, H.HIT_FULL) if full else (2, H.HIT_COMPACT)
+    out = torch.full((n, words), -7, dtype=torch.int32, device="cuda")
+    part = torch.zeros((300_000, words), dtype=torch.int32, device="cuda")
+    stream = torch.cuda.current_stream().cuda_stream
+    s.trace_nearest(rays, n, out, fmt, stream=stream)
+    lo = n - 300_000
+    s.trace_nearest(rays[lo:].contiguous(), 300_000, part, fmt, stream=stream)
+    torch.cuda.synchronize()
+    assert lo < seam < n and torch.equal(out[lo:], part)
+    s.trace_nearest(rays[:300_000].contiguous(), 300_000, part, fmt, stream=stream)
+    torch.cuda.synchronize()
+    assert torch.equal(out[:300_000], part)
+    s.close()
