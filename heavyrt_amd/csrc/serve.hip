@@ -94,7 +94,7 @@ __global__ __launch_bounds__(kWaveS) void k_serve(const uint8_t* __restrict__ ta
   h.u = h.v = 0.f;
   int top = 0;
   uint32_t cur = kInvalid;
-  RayPool pool;
+  RayPool pool(blockIdx.x, gridDim.x, R);
   while (true) {
     const uint64_t idle = __ballot(!active);
     const uint32_t nidle = __popcll(idle);

@@ -43,6 +43,7 @@ namespace {
 constexpr int kWave = 64;
 constexpr int kWavesPerBlock = 1;
 constexpr int kTraceBlock = kWave * kWavesPerBlock;
+static_assert(kWavesPerBlock == 1, "RayPool counts workgroups");
 constexpr int kRefillAt = 16;  // refill when at least this many lanes are idle
 constexpr uint32_t kClaim = 128;  // ray indices a wave claims from the queue at once
 // One-ray-per-lane kernel: stack entries per lane in LDS.  With 16 (16 KB
@@ -224,7 +225,7 @@ __global__ __launch_bounds__(kTraceBlock) void k_trace_persistent(const NodePair
   int top = 0;          // entries on the stack
   uint32_t cur = kInvalid;   // node pair to test next, a leaf, or kInvalid
   uint32_t leaf = 0;    // parked leaf (speculative any-hit), 0 = none
-  RayPool pool;  // ray indices claimed by this wave
+  RayPool pool(blockIdx.x, gridDim.x, n);  // ray indices claimed by this wave
 
   while (true) {
     // ---- refill idle lanes from the global queue -------------------------

@@ -340,7 +340,7 @@ __global__ __launch_bounds__(kBlock4, 8) void k_trace4_any_persistent(const void
   int top = 0;
   uint32_t cur = kInvalid;
   uint32_t leaf = 0, leaf2 = 0;  // parked leaves (leaf2 only while leaf is held)
-  RayPool pool;  // ray indices claimed by this wave (one queue: per-XCD queues measured 3 % slower here)
+  RayPool pool(blockIdx.x, gridDim.x, n);  // ray indices claimed by this wave (one queue: per-XCD queues measured 3 % slower here)
   // the tree and answer buffer of this lane's ray (a per-request source);
   // a launch-wide source keeps the kernel arguments
   const void* lane_quads = quads;

@@ -79,7 +79,7 @@ __global__ __launch_bounds__(kBlock) void k_trace_two_level(const NodePair* __re
   uint32_t cur_inst = 0, cur_geom = 0;
   uint32_t cur = kInvalid;
   uint32_t npairs = 0, ntests = 0;
-  RayPool pool;  // ray indices claimed by this wave
+  RayPool pool(blockIdx.x, gridDim.x, n);  // ray indices claimed by this wave
 
   auto enter = [&](uint32_t slot) {
     const InstDev* I = inst + slot;
