@@ -75,7 +75,7 @@ INVALID = 0xFFFFFFFF
 WORKLOADS = ("rtao", "eye", "precision", "batched", "serving")
 # kernels whose HBM bytes the counter child measures, by workload (substrings
 # of the demangled names rocprofv3 reports)
-COUNTER_KERNELS = {"rtao": ("AoRays",), "eye": ("k_trace_simple",), "precision": ("k_trace4_simple",),
+COUNTER_KERNELS = {"rtao": ("AoRays",), "eye": ("k_trace_simple",), "precision": ("k_trace4_simple", "k_trace4_sorted"),
                    "batched": ("k_b_trace",), "serving": ("k_serve", "ServeRays")}
 # workloads whose counters are summed over every matching dispatch of one
 # replayed request stream (the others: mean of the last three launches)
