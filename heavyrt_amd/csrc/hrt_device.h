@@ -607,6 +607,36 @@ __device__ inline float2 slab_fused(float3 oi, float3 inv, uint4 w, uint3 sel) {
   return make_float2(fmaxf(fmaxf(nx, ny), nz), fminf(fminf(fx, fy), fz));
 }
 
+// b - o for the FP16 bound b in the low or high half of w: one instruction, as
+// the widening is exact and fma(b, 1, -o) rounds like the subtraction.  (In asm
+// because the compiler turns that fma back into a conversion and a subtraction.)
+__device__ inline float h2f_sub_lo(uint32_t w, float o) {
+  float r;
+  asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(w), "v"(o));
+  return r;
+}
+__device__ inline float h2f_sub_hi(uint32_t w, float o) {
+  float r;
+  asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(w), "v"(o));
+  return r;
+}
+
+// slab on an FP16 child with each axis's near and far plane picked by the
+// ray's direction (near_far_selectors) instead of by min and max: rounding is
+// monotonic, so for lo <= hi the distances are the same.  17 instructions
+// instead of 26: 4,194,304 sorted random rays in a 4,194,304-triangle soup, a
+// walk bound by its VALU instructions, 6.25 ms a call before and 6.11 now.  An
+// inverted box (an unused slot) is empty in this form.
+__device__ inline float2 slab_half(float3 o, float3 inv, uint4 w, uint3 sel) {
+  const uint32_t bx = __builtin_amdgcn_perm(w.y, w.x, sel.x);
+  const uint32_t by = __builtin_amdgcn_perm(w.z, w.x, sel.y);
+  const uint32_t bz = __builtin_amdgcn_perm(w.z, w.y, sel.z);
+  const float nx = inv.x * h2f_sub_lo(bx, o.x), fx = inv.x * h2f_sub_hi(bx, o.x);
+  const float ny = inv.y * h2f_sub_lo(by, o.y), fy = inv.y * h2f_sub_hi(by, o.y);
+  const float nz = inv.z * h2f_sub_lo(bz, o.z), fz = inv.z * h2f_sub_hi(bz, o.z);
+  return make_float2(fmaxf(fmaxf(nx, ny), nz), fminf(fminf(fx, fy), fz));
+}
+
 // FP32 -> FP16 bits, round to nearest even (v_cvt_f16_f32 in the default mode).
 __device__ inline uint32_t f2h_rne(float f) { return __builtin_bit_cast(uint16_t, _Float16(f)); }
 

@@ -46,10 +46,10 @@ constexpr uint64_t kLaunchRays = 1u << 22, kLaunchRaysMin = 1u << 16;
 // they are traced.  A tree well inside the 256 MB MALL gains nothing that pays
 // for the sort: ms a call on FP16 nodes of the clustered tree, in the rays' own
 // order and sorted, random rays / camera rays: 1,048,576 rays in a
-// 1,000,000-triangle soup (70 MB) 1.55 and 1.52 / 0.82 and 1.06, over
-// 1,000,000 triangles of hills 0.64 and 0.81 / 0.29 and 0.63; 4,194,304 rays in
-// a 4,194,304-triangle soup (290 MB) 13.2 and 9.4 / 4.6 and 5.5, in a
-// 2,000,000-triangle soup (140 MB) 7.9 and 6.5 / 3.2 and 4.1.
+// 1,000,000-triangle soup (70 MB) 1.24 and 1.16 / 0.84 and 1.07, over
+// 1,000,000 triangles of hills 0.44 and 0.74 / 0.38 and 0.73; 4,194,304 rays in
+// a 4,194,304-triangle soup (290 MB) 11.6 and 6.4 / 2.9 and 3.2, in a
+// 2,000,000-triangle soup (140 MB) 6.4 and 4.3 / 2.1 and 2.4.
 constexpr uint64_t kSortRaysMin4 = 1u << 20;
 constexpr uint64_t kSortTreeMin4 = 128u << 20;
 // The speculative any-hit kernels leave the node loop for the leaf phase once
@@ -70,11 +70,13 @@ __global__ void k_reset_counter4(uint32_t* c) { *c = 0u; }
 // triangle-test policy tt: bt[k] = the child's (entry, exit) distances,
 // ch[k] its reference.  kFused (FP16 nodes of any-hit traversals under the
 // reference's test only): slab_fused with oi = -(o * inv) for a lane whose
-// fz = fused_ok(oi), slab otherwise.
-template <bool kFp16, bool kFused, class Tri>
+// fz = fused_ok(oi), slab otherwise.  kNearFar (FP16 nodes of nearest hits under
+// that test): slab_half, which leaves out a child without a finite triangle,
+// whose box is inverted; the counting variant counts its visit and keeps slab.
+template <bool kFp16, bool kFused, class Tri, bool kNearFar = false>
 __device__ inline void quad_boxes(const void* __restrict__ quads, uint32_t q, float3 o, float3 inv, float3 oi,
                                   bool fz, const Tri& tt, float2 bt[4], uint32_t ch[4]) {
-  static_assert(kFp16 || !kFused, "the fused box test is for FP16 nodes");
+  static_assert(kFp16 || !(kFused || kNearFar), "these box tests are for FP16 nodes");
   if (kFp16) {
     // per child {minx | miny << 16, minz | maxx << 16, maxy | maxz << 16, ref};
     // the FP16 values are widened inside each branch, so the fused one feeds
@@ -90,6 +92,10 @@ __device__ inline void quad_boxes(const void* __restrict__ quads, uint32_t q, fl
       const uint3 sel = near_far_selectors(inv);
 #pragma unroll
       for (int k = 0; k < 4; k++) bt[k] = slab_fused(oi, inv, w[k], sel);
+    } else if (kNearFar && !Tri::kRobustBoxes) {
+      const uint3 sel = near_far_selectors(inv);
+#pragma unroll
+      for (int k = 0; k < 4; k++) bt[k] = slab_half(o, inv, w[k], sel);
     } else {
 #pragma unroll
       for (int k = 0; k < 4; k++)
@@ -123,11 +129,11 @@ __device__ inline bool child_hit(float2 t, uint32_t c, float tnear, float tcull)
 
 // quad_boxes, then the entry distances (kMaxFloat for a miss) sorted
 // ascending with their references, as the reference orders a node's children.
-template <bool kFp16, bool kFused, class Tri>
+template <bool kFp16, bool kFused, class Tri, bool kNearFar>
 __device__ inline void visit_quad(const void* __restrict__ quads, uint32_t q, float3 o, float3 inv, float3 oi,
                                   bool fz, const Tri& tt, float tnear, float tcull, float tm[4], uint32_t ch[4]) {
   float2 bt[4];
-  quad_boxes<kFp16, kFused>(quads, q, o, inv, oi, fz, tt, bt, ch);
+  quad_boxes<kFp16, kFused, Tri, kNearFar>(quads, q, o, inv, oi, fz, tt, bt, ch);
 #pragma unroll
   for (int k = 0; k < 4; k++) tm[k] = child_hit(bt[k], ch[k], tnear, tcull) ? bt[k].x : kMaxFloat;
   // five-comparator network, BVH4HalfRT.cpp:121-180 (swap when strictly less)
@@ -189,7 +195,8 @@ __device__ inline void trace4_one(const void* __restrict__ quads, const TriPre* 
     if ((cur & kLeafBit) == 0) {
       float tm[4];
       uint32_t ch[4];
-      visit_quad<kFp16, kForceAny && kFp16>(quads, cur, o, inv, oi, fz, tt, tnear, h.t, tm, ch);
+      visit_quad<kFp16, kForceAny && kFp16, Tri, kFp16 && !kForceAny && !kStats>(quads, cur, o, inv, oi, fz, tt, tnear,
+                                                                                h.t, tm, ch);
       if (kStats) nvisits++;
       stk.push_masked3(top, tm[3] < kMaxFloat, ch[3], tm[2] < kMaxFloat, ch[2], tm[1] < kMaxFloat, ch[1]);
       if (tm[0] < kMaxFloat) cur = ch[0];
@@ -459,6 +466,7 @@ __device__ inline float2 child_box(const void* __restrict__ quads, uint32_t q, u
     const uint4 w = static_cast<const Quad16*>(quads)[q].c[l];
     ref = w.w;
     if (kFused && !Tri::kRobustBoxes && fz) return slab_fused(oi, inv, w, near_far_selectors(inv));
+    if (!kFused && !Tri::kRobustBoxes) return slab_half(o, inv, w, near_far_selectors(inv));
     return tt.box(o, inv, h2f_lo(w.x), h2f_hi(w.x), h2f_lo(w.y), h2f_hi(w.y), h2f_lo(w.z), h2f_hi(w.z));
   }
   const float* f = reinterpret_cast<const float*>(static_cast<const Quad32*>(quads) + q) + l;

@@ -331,3 +331,22 @@ def test_bvh4_launches_of_a_large_batch_join(gpu_ctx, full):
     torch.cuda.synchronize()
     assert torch.equal(out[:300_000], part)
     s.close()
+
+
+@pytest.mark.parametrize("n", [700, 70_000], ids=["four_lanes", "one_lane"])
+def test_fp16_planes_picked_by_direction(gpu_ctx, n):
+    """Zero, negative-zero and signed direction components, origins on box planes, triangles without finite corners:
+    the hits of the FP16 walk are the counting variant's, which takes minimum and maximum."""
+    v, f = W.soup(5000, stream=W.STREAM_TEST)
+    v = v.copy()
+    v[f[::61].reshape(-1)] = np.nan
+    s = H.Scene(gpu_ctx)
+    s.add_instance(s.add_triangles(v, f))
+    s.commit(layout=H.LAYOUT_BVH4_FP16)
+    rays = rays_for(np.nan_to_num(v), n, 8900)
+    rays[1::5, 4] = 0.0
+    rays[2::5, 5] = -0.0
+    rays[3::5, 4:7] = [0.0, 0.0, -1.0]
+    rays[4::5, 0:3] = v[f[1 + (np.arange(len(rays[4::5])) % 60), 0]].astype(np.float16)  # on FP16 planes
+    same(trace(s, rays, "full"), trace(s, rays, "full", stats=True))
+    s.close()
