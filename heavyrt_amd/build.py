@@ -23,8 +23,8 @@ INCLUDE = os.path.join(ROOT, "include")
 LIB_HRT = os.path.join(HERE, "libhrt.so")
 LIB_SCENE = os.path.join(HERE, "libhrt_scene.so")
 
-HIP_SOURCES = ["sort.hip", "lbvh.hip", "ploc.hip", "trace.hip", "trace4.hip", "trace_tlas.hip", "batch.hip", "serve.hip",
-               "rtao.hip", "eye.hip", "capi.hip", "noalloc.hip", "probe.hip"]
+HIP_SOURCES = ["devmem.cpp", "sort.hip", "lbvh.hip", "ploc.hip", "trace.hip", "trace4.hip", "trace_tlas.hip",
+               "batch.hip", "serve.hip", "rtao.hip", "eye.hip", "capi.hip", "noalloc.hip", "probe.hip"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
 HIP_FLAGS = [
@@ -52,7 +52,7 @@ def build_hrt(verbose: bool = True) -> str:
     objdir = os.path.join(HERE, "_build")
     os.makedirs(objdir, exist_ok=True)
     for src in HIP_SOURCES:
-        obj = os.path.join(objdir, src.replace(".hip", ".o"))
+        obj = os.path.join(objdir, os.path.splitext(src)[0] + ".o")
         _run([HIPCC, *HIP_FLAGS, "-I", INCLUDE, "-I", CSRC, "-c", os.path.join(CSRC, src), "-o", obj])
         objs.append(obj)
     tmp = LIB_HRT + ".tmp"

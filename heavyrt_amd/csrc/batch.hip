@@ -1210,7 +1210,7 @@ hrt_status hrt_batch_create(hrt_ctx* ctx, uint32_t nScenes, const uint32_t* nVer
 
   hipError_t e = hipSetDevice(ctx->device);
   auto al = [&](auto** p, size_t bytes) {
-    if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void**>(p), std::max<size_t>(bytes, 16));
+    if (e == hipSuccess) e = device_malloc(p, std::max<size_t>(bytes, 16));
   };
   al(&b->d_off, 4 * 5 * size_t(S + 1));
   al(&b->d_chunks, sizeof(uint4) * chunks.size());
@@ -1244,7 +1244,7 @@ hrt_status hrt_batch_create(hrt_ctx* ctx, uint32_t nScenes, const uint32_t* nVer
   b->quads = b->small && R > 0 &&
              2 * ((R + kQuadRaysB - 1) / kQuadRaysB) <=
                  resident_grid(reinterpret_cast<const void*>(&k_b_trace_quad), 256);
-  if (e == hipSuccess && b->quads && hipMalloc(&b->scratch, 4 * (words + words_wide)) != hipSuccess) {
+  if (e == hipSuccess && b->quads && device_malloc(&b->scratch, 4 * (words + words_wide)) != hipSuccess) {
     (void)hipGetLastError();
     b->scratch = nullptr;
     b->quads = false;

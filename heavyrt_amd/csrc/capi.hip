@@ -718,7 +718,7 @@ hrt_status host_batch(hrt_scene* s, const float* rays, size_t n, void* out, size
     if (s->host_dev) (void)hipFree(s->host_dev);
     s->host_dev = nullptr;
     s->host_dev_bytes = 0;
-    e = hipMalloc(&s->host_dev, need);
+    e = hrt::device_malloc(&s->host_dev, need);
     if (e == hipSuccess) s->host_dev_bytes = need;
   }
   if (e != hipSuccess) return fail_hip(e, "host batch staging");
@@ -852,7 +852,7 @@ hipError_t rtao_pass(hrt_scene* s, const hrt::Blas* b, uint32_t inst, const hrt:
   hipError_t e = hipSuccess;
   if (lay == HRT_LAYOUT_BVH2) {
     void* rays = nullptr;
-    if ((e = hipMallocAsync(&rays, sizeof(hrt::Ray) * n, hs)) != hipSuccess) return e;
+    if ((e = hrt::stream_malloc(&rays, sizeof(hrt::Ray) * n, hs)) != hipSuccess) return e;
     hrt::TraceArgs a;
     a.rays = static_cast<const hrt::Ray*>(rays);
     a.n = n;
@@ -873,7 +873,7 @@ hipError_t rtao_pass(hrt_scene* s, const hrt::Blas* b, uint32_t inst, const hrt:
   const bool fp16 = lay == HRT_LAYOUT_BVH4_FP16 || auto16 || lay == HRT_LAYOUT_PLOC_FP16;
   // the frames (32 B per pixel), then the samples' direction order (2 B each)
   void* frames = nullptr;
-  if ((e = hipMallocAsync(&frames, 32ull * npix + 2ull * n, hs)) != hipSuccess) return e;
+  if ((e = hrt::stream_malloc(&frames, 32ull * npix + 2ull * n, hs)) != hipSuccess) return e;
   hrt::AoFrame* f = static_cast<hrt::AoFrame*>(frames);
   uint16_t* order = reinterpret_cast<uint16_t*>(static_cast<char*>(frames) + 32ull * npix);
   e = hrt::rtao_frames(*b, prim, hits, npix, f, hs);
@@ -964,7 +964,7 @@ hrt_status hrt_eye_render(hrt_scene* s, const float projInvColMajor16[16], const
   }
   // other trees: rays to HBM, traced as a batch, coloured from the hits
   void* buf = nullptr;
-  if ((e = hipMallocAsync(&buf, 40 * n, hs)) != hipSuccess) return fail_hip(e, "eye render buffers");
+  if ((e = hrt::stream_malloc(&buf, 40 * n, hs)) != hipSuccess) return fail_hip(e, "eye render buffers");
   float* rays = static_cast<float*>(buf);
   uint32_t* hits = reinterpret_cast<uint32_t*>(static_cast<char*>(buf) + 32 * n);
   // XCD stripes: the image is all this call owes, and stripes trace fastest
@@ -996,7 +996,7 @@ hrt_status hrt_rtao_render(hrt_scene* s, const float projInvColMajor16[16], cons
   if (e != hipSuccess) return fail_hip(e, "hipSetDevice");
   // eye rays (32 B), compact hits (8 B) and AO bytes (raysPerHit) per pixel
   void* buf = nullptr;
-  if ((e = hipMallocAsync(&buf, (40 + size_t(raysPerHit)) * n, hs)) != hipSuccess)
+  if ((e = hrt::stream_malloc(&buf, (40 + size_t(raysPerHit)) * n, hs)) != hipSuccess)
     return fail_hip(e, "rtao render buffers");
   float* rays = static_cast<float*>(buf);
   uint32_t* hits = reinterpret_cast<uint32_t*>(static_cast<char*>(buf) + 32 * n);

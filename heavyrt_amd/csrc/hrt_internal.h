@@ -5,59 +5,16 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-#include <map>
 #include <memory>
-#include <mutex>
 #include <string>
 #include <type_traits>
-#include <unordered_map>
 #include <vector>
 
 #include "../../include/hrt.h"
+#include "devmem.h"
 #include "hrt_device.h"
 
 namespace hrt {
-
-// Device memory of one context's trees and build scratch, kept for reuse when
-// it is given back (a 128 MB hipMalloc takes 53 us and its hipFree 265 us, and
-// a build has a dozen arrays: a million triangles loaded and committed took
-// 10.3 ms, and 2.8 with this and the geometry expanded on the device), and pinned words for small readbacks (12 us with
-// the wait, 21 us through pageable memory).  At most kMaxIdle bytes are kept
-// idle, for blocks of up to a quarter less; trim gives them all back (when an allocation fails, and at the end).
-// Safe with several threads.
-class DevCache {
- public:
-  explicit DevCache(int device) : device_(device) {}
-  DevCache(const DevCache&) = delete;
-  DevCache& operator=(const DevCache&) = delete;
-  ~DevCache();
-  template <class T>
-  hipError_t alloc(T** p, size_t bytes) {
-    return alloc_bytes(reinterpret_cast<void**>(p), bytes);
-  }
-  // For memory that nothing on the device uses any more (null is fine).
-  void free(void* p);
-  // Waits for the whole device, whatever the caller's current one is.
-  void wait();
-  void trim();
-  // kPinnedWords words, or null when all are taken.
-  static constexpr size_t kPinnedWords = 32;
-  uint32_t* pinned_get();
-  void pinned_put(uint32_t* w);
-
- private:
-  static constexpr size_t kMaxIdle = size_t(1) << 30;
-  static constexpr int kPinnedSlots = 16;
-  hipError_t alloc_bytes(void** p, size_t bytes);
-  bool note(void* p, size_t size);
-  const int device_;
-  std::mutex mu_;
-  std::unordered_map<void*, size_t> live_;
-  std::multimap<size_t, void*> idle_;
-  size_t idle_bytes_ = 0;
-  uint32_t* pinned_ = nullptr;
-  uint32_t pinned_taken_ = 0;  // a bit per slot
-};
 
 // Words copied back from the device into pinned memory where there is some.
 class Readback {

@@ -601,111 +601,6 @@ inline uint32_t leaf_blocks(uint64_t n) { return (blocks_for(n) + kXcds - 1) / k
 
 }  // namespace
 
-DevCache::~DevCache() {
-  trim();
-  if (pinned_) (void)hipHostFree(pinned_);
-}
-
-void DevCache::wait() {
-  int current = device_;
-  (void)hipGetDevice(&current);
-  if (current != device_) (void)hipSetDevice(device_);
-  (void)hipDeviceSynchronize();
-  if (current != device_) (void)hipSetDevice(current);
-}
-
-void DevCache::trim() {
-  std::multimap<size_t, void*> idle;
-  {
-    std::lock_guard<std::mutex> lock(mu_);
-    idle.swap(idle_);
-    idle_bytes_ = 0;
-  }
-  for (auto& x : idle) (void)hipFree(x.second);
-}
-
-hipError_t DevCache::alloc_bytes(void** p, size_t bytes) {
-  // sizes in steps, so that a slightly different geometry finds its memory
-  const size_t step = bytes < (size_t(1) << 16) ? size_t(1) << 12 : bytes < (size_t(1) << 20) ? size_t(1) << 16 : size_t(1) << 21;
-  const size_t size = (std::max<size_t>(bytes, 1) + step - 1) / step * step;
-  {
-    std::lock_guard<std::mutex> lock(mu_);
-    auto it = idle_.lower_bound(size);
-    if (it != idle_.end() && it->first <= size + size / 4) {
-      if (!note(it->second, it->first)) return hipErrorOutOfMemory;
-      *p = it->second;
-      idle_bytes_ -= it->first;
-      idle_.erase(it);
-      return hipSuccess;
-    }
-  }
-  hipError_t e = hipMalloc(p, size);
-  if (e == hipErrorOutOfMemory) {
-    (void)hipGetLastError();
-    trim();
-    e = hipMalloc(p, size);
-  }
-  if (e != hipSuccess) {
-    *p = nullptr;
-    return e;
-  }
-  std::lock_guard<std::mutex> lock(mu_);
-  if (note(*p, size)) return hipSuccess;
-  (void)hipFree(*p);
-  *p = nullptr;
-  return hipErrorOutOfMemory;
-}
-
-// mu_ held; false: no host memory
-bool DevCache::note(void* p, size_t size) {
-  try {
-    live_[p] = size;
-  } catch (const std::bad_alloc&) {
-    return false;
-  }
-  return true;
-}
-
-void DevCache::free(void* p) {
-  if (!p) return;
-  {
-    std::lock_guard<std::mutex> lock(mu_);
-    const auto it = live_.find(p);
-    if (it == live_.end()) return;
-    const size_t size = it->second;
-    live_.erase(it);
-    try {
-      if (idle_bytes_ + size <= kMaxIdle) {
-        idle_.emplace(size, p);
-        idle_bytes_ += size;
-        return;
-      }
-    } catch (const std::bad_alloc&) {  // given back below
-    }
-  }
-  (void)hipFree(p);
-}
-
-uint32_t* DevCache::pinned_get() {
-  std::lock_guard<std::mutex> lock(mu_);
-  if (!pinned_ && hipHostMalloc(reinterpret_cast<void**>(&pinned_), 4 * kPinnedWords * kPinnedSlots, hipHostMallocDefault) != hipSuccess) {
-    (void)hipGetLastError();
-    pinned_ = nullptr;
-    return nullptr;
-  }
-  for (int k = 0; k < kPinnedSlots; k++) {
-    if (pinned_taken_ & (1u << k)) continue;
-    pinned_taken_ |= 1u << k;
-    return pinned_ + k * kPinnedWords;
-  }
-  return nullptr;
-}
-
-void DevCache::pinned_put(uint32_t* w) {
-  std::lock_guard<std::mutex> lock(mu_);
-  pinned_taken_ &= ~(1u << (size_t(w - pinned_) / kPinnedWords));
-}
-
 hipError_t blas_alloc(Blas& b, DevCache* mem, uint32_t nverts, uint32_t ntris, bool keep_debug, bool with_mesh) {
   b.mem = mem;
   b.nverts = nverts;

@@ -34,7 +34,7 @@ extern "C" hrt_status hrt_issue_probe(hrt_ctx* ctx, void* stream) {
   // 4 SIMDs per CU, 8 waves per SIMD, one wave per workgroup
   const uint32_t blocks = uint32_t(cus) * 32u;
   float* sink = nullptr;
-  if ((e = hipMallocAsync(reinterpret_cast<void**>(&sink), sizeof(float) * blocks, hs)) != hipSuccess)
+  if ((e = hrt::stream_malloc(&sink, sizeof(float) * blocks, hs)) != hipSuccess)
     return hrt::fail_hip(e, "issue probe");
   k_issue_probe<<<blocks, 64, 0, hs>>>(sink, 100000, 0.999f, 0.001f);
   e = hipGetLastError();

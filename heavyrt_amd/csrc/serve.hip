@@ -472,7 +472,7 @@ hrt_status hrt_server_create(hrt_ctx* ctx, uint64_t budgetBytes, uint32_t stepsI
   sv->ctx = ctx;
   sv->budget = align_up(budgetBytes, 256);
   hipError_t e = hipSetDevice(ctx->device);
-  if (e == hipSuccess) e = hipMalloc(&sv->arena_dev, sv->budget);
+  if (e == hipSuccess) e = device_malloc(&sv->arena_dev, sv->budget);
   // steps in flight share the chip: each gets its share of the resident waves
   const uint32_t resident[kKinds] = {resident_grid(reinterpret_cast<const void*>(&k_serve), kWaveS),
                                      serve_any4_resident_grid(true), serve_any4_resident_grid(false)};
@@ -489,8 +489,8 @@ hrt_status hrt_server_create(hrt_ctx* ctx, uint64_t budgetBytes, uint32_t stepsI
     if (e == hipSuccess) e = hipEventCreateWithFlags(&st.done, hipEventDisableTiming);
     if (e == hipSuccess)
       e = hipHostMalloc(reinterpret_cast<void**>(&st.tab_host), kKinds * kTabBytes, hipHostMallocDefault);
-    if (e == hipSuccess) e = hipMalloc(&st.tab_dev, kKinds * kTabBytes);
-    if (e == hipSuccess) e = hipMalloc(&st.spill, 4 * sv->spill_words);
+    if (e == hipSuccess) e = device_malloc(&st.tab_dev, kKinds * kTabBytes);
+    if (e == hipSuccess) e = device_malloc(&st.spill, 4 * sv->spill_words);
   }
   if (e != hipSuccess) {
     destroy_server(sv);

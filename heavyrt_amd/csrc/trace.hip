@@ -361,9 +361,7 @@ hipError_t launch_persistent(const Blas& b, const TraceArgs& a, hipStream_t stre
   const size_t spill_words = size_t(grid) * kTraceBlock * kLaneWords;
   uint32_t* buf = a.workspace;
   hipError_t e = hipSuccess;
-  if (!buf && (e = hipMallocAsync(reinterpret_cast<void**>(&buf), sizeof(uint32_t) * (64 + spill_words), stream)) !=
-                  hipSuccess)
-    return e;
+  if (!buf && (e = stream_malloc(&buf, sizeof(uint32_t) * (64 + spill_words), stream)) != hipSuccess) return e;
   k_reset_counter<<<1, 1, 0, stream>>>(buf);
   k_trace_persistent<kAny, kSpec, Tri><<<grid, kTraceBlock, 0, stream>>>(
       b.pairs, tri_records<Tri>(b), a.rays, a.n, a.out, a.format, make_uint2(a.inst_id, a.geom_id), buf, buf + 64);
@@ -399,8 +397,7 @@ hipError_t trace_nearest(const Blas& b, const Io& io, uint64_t n, hipStream_t st
     return hipGetLastError();
   }
   uint32_t* spill = nullptr;
-  hipError_t e = hipMallocAsync(reinterpret_cast<void**>(&spill),
-                                sizeof(uint32_t) * size_t(blocks) * 256 * (kWalkDepth - kSimpleLds), stream);
+  hipError_t e = stream_malloc(&spill, sizeof(uint32_t) * size_t(blocks) * 256 * (kWalkDepth - kSimpleLds), stream);
   if (e != hipSuccess) return e;
   k_trace_simple<false, false, kSimpleLds, Tri, Io><<<blocks, 256, 0, stream>>>(b.pairs, tris, io, n, nullptr, spill);
   e = hipGetLastError();

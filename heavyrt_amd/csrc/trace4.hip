@@ -623,9 +623,7 @@ hipError_t launch_any4(const Blas& b, Src src, uint64_t n, uint8_t* out, hipStre
   const size_t spill_words = size_t(grid) * kBlock4 * kLaneWords;
   uint32_t* buf = workspace;
   hipError_t e = hipSuccess;
-  if (!buf && (e = hipMallocAsync(reinterpret_cast<void**>(&buf), sizeof(uint32_t) * (64 + spill_words), stream)) !=
-                  hipSuccess)
-    return e;
+  if (!buf && (e = stream_malloc(&buf, sizeof(uint32_t) * (64 + spill_words), stream)) != hipSuccess) return e;
   k_reset_counter4<<<1, 1, 0, stream>>>(buf);
   k_trace4_any_persistent<kFp16, Src, Tri><<<grid, kBlock4, 0, stream>>>(q, tri_records<Tri>(b), src, n, out, buf,
                                                                           buf + 64);
@@ -708,14 +706,7 @@ hipError_t launch_simple4(const Blas& b, const TraceArgs& a, hipStream_t stream)
   const size_t lane_words = kStackDepth4 - (a.stats ? kStatsLds4 : kSimpleLds4);
   uint64_t share = a.stats ? a.n : std::min(a.n, kLaunchRays);
   uint32_t* spill = nullptr;
-  hipError_t e;
-  while (true) {
-    const uint64_t lanes = (share + kBlock4 - 1) / kBlock4 * kBlock4;
-    e = hipMallocAsync(reinterpret_cast<void**>(&spill), sizeof(uint32_t) * lanes * lane_words, stream);
-    if (e != hipErrorOutOfMemory || a.stats || share <= kLaunchRaysMin) break;
-    (void)hipGetLastError();
-    share = std::max(share / 4, kLaunchRaysMin);
-  }
+  hipError_t e = lane_malloc(&spill, &share, a.stats ? a.n : kLaunchRaysMin, kBlock4, lane_words, stream);
   if (e != hipSuccess) return e;
   for (uint64_t at = 0; at < a.n && e == hipSuccess; at += share) {
     const uint64_t n = std::min(a.n - at, share);
@@ -754,7 +745,7 @@ hipError_t launch_nearest4_sorted(const Blas& b, const TraceArgs& a, hipStream_t
   const size_t spill_words = size_t(grid) * kBlock4 * (kStackDepth4 - kSimpleLds4);
   const size_t words = 64 + kXcdQueueWords + 4 * n + sort_words + spill_words;
   uint32_t* base = nullptr;
-  hipError_t e = hipMallocAsync(reinterpret_cast<void**>(&base), sizeof(uint32_t) * words, stream);
+  hipError_t e = stream_malloc(&base, sizeof(uint32_t) * words, stream);
   if (e != hipSuccess) return e;
   // base[0..1]: the order slot (8-byte aligned), base[2]: the sort's error word
   const uint32_t** slot = reinterpret_cast<const uint32_t**>(base);

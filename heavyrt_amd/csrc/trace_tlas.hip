@@ -230,7 +230,7 @@ hipError_t launch(const Blas& tlas, const InstDev* inst, const TraceArgs& a, hip
   const int grid = int(std::min<uint64_t>(want, uint64_t(resident_grid(kfn, kBlock))));
   const size_t spill_words = size_t(grid) * kBlock * (kTwoLevelDepth - kShortStack);
   uint32_t* buf = nullptr;
-  hipError_t e = hipMallocAsync(reinterpret_cast<void**>(&buf), sizeof(uint32_t) * (64 + spill_words), stream);
+  hipError_t e = stream_malloc(&buf, sizeof(uint32_t) * (64 + spill_words), stream);
   if (e != hipSuccess) return e;
   k_reset_counter<<<1, 1, 0, stream>>>(buf);
   k_trace_two_level<kAny, kStats><<<grid, kBlock, 0, stream>>>(tlas.pairs, inst, a.rays, a.n, a.out, a.format,

@@ -1,0 +1,134 @@
+"""One scenario of test_gpu_memory.py in a process of its own: `gpu_memory_worker.py SHIM SCENARIO`."""
+import ctypes as C
+import os
+import sys
+
+shim = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)  # before libhrt.so, whose calls then find it
+sys.path.insert(0, os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
+
+import numpy as np  # noqa: E402
+
+import heavyrt_amd as H  # noqa: E402
+from heavyrt_amd import workloads as W  # noqa: E402
+
+MB = 1 << 20
+for fn in (shim.shim_used, shim.shim_calls, shim.shim_refused):
+    fn.restype = C.c_uint64
+shim.shim_limit.argtypes = [C.c_size_t]
+shim.shim_names.restype = C.c_char_p
+
+
+def kernels():
+    """Names launched since the last call."""
+    n = shim.shim_names().decode().split()
+    shim.shim_clear_names()
+    return n
+
+
+def limited(room):
+    """From here on the device has `room` bytes more than are allocated."""
+    shim.shim_limit(shim.shim_used() + room)
+
+
+def unlimited():
+    shim.shim_limit(C.c_size_t(-1).value)
+
+
+def committed(ctx, v, f, layout=H.LAYOUT_BVH2):
+    s = H.Scene(ctx)
+    s.add_instance(s.add_triangles(v, f))
+    s.commit(layout=layout)
+    return s
+
+
+def leave_idle(ctx):
+    """Memory that the engine keeps for its next trees: more than 200 MB."""
+    unlimited()
+    v, f = W.soup(600_000, stream=W.STREAM_TEST)
+    s = committed(ctx, v, f, H.LAYOUT_AUTO_FP16)
+    before = shim.shim_used()
+    s.close()
+    assert before > 300 * MB and shim.shim_used() > 200 * MB, (before, shim.shim_used())
+
+
+def refused(fn):
+    try:
+        fn()
+    except H.HrtError as e:
+        assert e.status == 3, e.status  # out of memory
+        return True
+    return False
+
+
+def idle_memory():
+    """What a call of the engine needs beside its trees, it takes from their idle memory."""
+    ctx = H.Context(0)
+    v, f = W.soup(100_000, stream=W.STREAM_TEST)
+    rays = W.incoherent_rays(700_000, stream=W.STREAM_TEST)
+
+    def batch():
+        b = H.Batch(ctx, [v.shape[0]], [f.shape[0]], [1000])
+        b.upload([(v, f, rays[:1000])])
+        b.run()
+        b.hits()
+        b.close()
+
+    def server():
+        H.Server(ctx, 20 * MB).close()
+
+    def trace(layout, any_hit=False):
+        s = committed(ctx, v, f, layout)
+        run = s.trace_any_host if any_hit else s.trace_nearest_host
+        want = run(rays)  # (and the staging of the next call: that one needs stacks alone)
+
+        def call():
+            assert np.asarray(run(rays)).tobytes() == np.asarray(want).tobytes()
+            s.close()
+        return call
+
+    calls = [("batch", lambda: batch), ("server", lambda: server)]
+    calls += [(f"trace {lay}", lambda lay=lay: trace(lay)) for lay in (H.LAYOUT_BVH2, H.LAYOUT_BVH4)]
+    calls += [("any", lambda: trace(H.LAYOUT_AUTO_FP16, True))]
+    for name, make in calls:
+        call = make()
+        print("idle memory for", name, flush=True)
+        leave_idle(ctx)
+        limited(MB)
+        n = shim.shim_refused()
+        call()
+        assert shim.shim_refused() > n, "the device was not full"
+    unlimited()
+    ctx.close()
+
+
+def smaller_launches():
+    """BVH4 nearest hits without memory for every lane's stack: several launches, the same records."""
+    ctx = H.Context(0)
+    v, f = W.soup(50_000, stream=W.STREAM_TEST)
+    s = committed(ctx, v, f, H.LAYOUT_BVH4)
+    rays = W.incoherent_rays(300_001, stream=W.STREAM_TEST)
+    rays[::3, 7] = -1.0
+    kernels()
+    want = s.trace_nearest_host(rays)
+    assert len([k for k in kernels() if "k_trace4_simple" in k]) == 1
+    limited(0)
+    assert refused(lambda: s.trace_nearest_host(rays))  # (nothing is idle after that)
+    kernels()
+    for share, launches in ((75_000, 5), (65_536, 5)):  # a quarter of the rays, and the least
+        lanes = (share + 63) // 64 * 64
+        limited(156 * lanes)
+        got = s.trace_nearest_host(rays)
+        assert len([k for k in kernels() if "k_trace4_simple" in k]) == launches
+        assert np.asarray(got).tobytes() == np.asarray(want).tobytes()
+    limited(156 * 65_536 - 1)
+    assert refused(lambda: s.trace_nearest_host(rays))
+    unlimited()
+    assert np.asarray(s.trace_nearest_host(rays)).tobytes() == np.asarray(want).tobytes()
+    s.close()
+    ctx.close()
+
+
+if __name__ == "__main__":
+    globals()[sys.argv[2]]()
+    assert shim.shim_calls() > 0, "the engine's calls did not reach the shim"
+    print("done", sys.argv[2], flush=True)
