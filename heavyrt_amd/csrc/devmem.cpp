@@ -51,13 +51,14 @@ void DevCache::wait() {
 }
 
 bool DevCache::trim() {
-  std::multimap<size_t, void*> idle;
+  IdleMap idle;
   {
     std::lock_guard<std::mutex> lock(mu_);
     idle.swap(idle_);
+    oldest_.clear();
     idle_bytes_ = 0;
   }
-  for (auto& x : idle) (void)hipFree(x.second);
+  for (auto& x : idle) (void)hipFree(x.second.p);
   return !idle.empty();
 }
 
@@ -79,10 +80,8 @@ hipError_t DevCache::alloc_bytes(void** p, size_t bytes) {
     std::lock_guard<std::mutex> lock(mu_);
     auto it = idle_.lower_bound(size);
     if (it != idle_.end() && it->first <= size + size / 4) {
-      if (!note(it->second, it->first)) return hipErrorOutOfMemory;
-      *p = it->second;
-      idle_bytes_ -= it->first;
-      idle_.erase(it);
+      if (!note(it->second.p, it->first)) return hipErrorOutOfMemory;
+      *p = take(it);
       return hipSuccess;
     }
   }
@@ -108,22 +107,47 @@ bool DevCache::note(void* p, size_t size) {
   return true;
 }
 
+// mu_ held: the block, no longer idle
+void* DevCache::take(IdleMap::iterator it) {
+  void* p = it->second.p;
+  idle_bytes_ -= it->first;
+  oldest_.erase(it->second.since);
+  idle_.erase(it);
+  return p;
+}
+
 void DevCache::free(void* p) {
   if (!p) return;
+  size_t size = 0;
   {
     std::lock_guard<std::mutex> lock(mu_);
     const auto it = live_.find(p);
     if (it == live_.end()) return;
-    const size_t size = it->second;
+    size = it->second;
     live_.erase(it);
-    try {
-      if (idle_bytes_ + size <= kMaxIdle) {
-        idle_.emplace(size, p);
+  }
+  // The oldest idle blocks make room: a program whose sizes have changed finds
+  // its new ones.  One at a time, as hipFree waits and must not hold the lock.
+  while (size <= kMaxIdle) {
+    void* old = nullptr;
+    {
+      std::lock_guard<std::mutex> lock(mu_);
+      if (idle_bytes_ + size > kMaxIdle) {
+        old = take(oldest_.begin()->second);
+      } else {
+        auto it = idle_.end();
+        try {
+          it = idle_.emplace(size, Idle{p, clock_});
+          oldest_.emplace(clock_++, it);
+        } catch (const std::bad_alloc&) {  // no host memory: given back below
+          if (it != idle_.end()) idle_.erase(it);
+          break;
+        }
         idle_bytes_ += size;
         return;
       }
-    } catch (const std::bad_alloc&) {  // given back below
     }
+    (void)hipFree(old);
   }
   (void)hipFree(p);
 }

@@ -17,8 +17,8 @@ namespace hrt {
 // a build has a dozen arrays: a million triangles loaded and committed took
 // 10.3 ms, and 2.8 with this and the geometry expanded on the device), and
 // pinned words for small readbacks (12 us with the wait, 21 us through pageable
-// memory).  At most kMaxIdle bytes are kept idle, for blocks of up to a quarter
-// less.  They go back to the device when any allocation of the engine on it
+// memory).  At most kMaxIdle bytes are kept idle, the latest ones, for blocks of
+// up to a quarter less.  They go back to the device when any allocation of the engine on it
 // fails (here, device_malloc, stream_malloc), whichever context kept them, and
 // at the end.  Safe with several threads.
 class DevCache {
@@ -53,7 +53,15 @@ class DevCache {
   const int device_;
   std::mutex mu_;
   std::unordered_map<void*, size_t> live_;
-  std::multimap<size_t, void*> idle_;
+  struct Idle {
+    void* p;
+    uint64_t since;
+  };
+  using IdleMap = std::multimap<size_t, Idle>;  // by size
+  void* take(IdleMap::iterator it);
+  IdleMap idle_;
+  std::map<uint64_t, IdleMap::iterator> oldest_;  // the same blocks by `since`
+  uint64_t clock_ = 0;
   size_t idle_bytes_ = 0;
   uint32_t* pinned_ = nullptr;
   uint32_t pinned_taken_ = 0;  // a bit per slot

@@ -88,6 +88,26 @@ void reuse() {
   check(dev.mallocs == before + 1, "a larger one is not");
 }
 
+// A full list gives its oldest blocks back for the new ones.
+void reuse_after_the_sizes_change() {
+  DevCache mem(0);
+  leave_idle(mem, 10 * kMB, 110);
+  check(dev.used <= DevCache::kMaxIdle, "no more than the bound stays");
+  leave_idle(mem, 50 * kMB, 4);
+  check(dev.used <= DevCache::kMaxIdle, "nor then");
+  int before = dev.mallocs;
+  leave_idle(mem, 50 * kMB, 4);
+  check(dev.mallocs == before, "the new size is taken again");
+  before = dev.mallocs;
+  leave_idle(mem, 10 * kMB, 70);
+  check(dev.mallocs == before, "and what is left of the old one");
+  leave_idle(mem, DevCache::kMaxIdle + kMB, 1);
+  check(dev.mallocs == before + 1, "a block beyond the bound is not kept");
+  leave_idle(mem, 10 * kMB, 70);
+  check(dev.mallocs == before + 1, "nor does it cost the others");
+  check(dev.bad_frees == 0, "every block given back once");
+}
+
 // Allocations outside the cache get its idle memory, other contexts' too.
 void others_get_the_idle_memory() {
   DevCache mem(0), second(0);
@@ -184,6 +204,7 @@ int main(int, char** argv) {
     const char* name;
     void (*fn)();
   } all[] = {{"reuse", reuse},
+             {"reuse_after_the_sizes_change", reuse_after_the_sizes_change},
              {"others_get_the_idle_memory", others_get_the_idle_memory},
              {"not_another_devices", not_another_devices},
              {"not_under_capture", not_under_capture},

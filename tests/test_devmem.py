@@ -20,8 +20,8 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("scenario", ["reuse", "others_get_the_idle_memory", "not_another_devices",
-                                      "not_under_capture", "fewer_lanes_without_memory", "threads",
+@pytest.mark.parametrize("scenario", ["reuse", "reuse_after_the_sizes_change", "others_get_the_idle_memory",
+                                      "not_another_devices", "not_under_capture", "fewer_lanes_without_memory", "threads",
                                       "given_back_at_the_end"])
 def test_scenario(program, scenario):
     r = subprocess.run([program, scenario], capture_output=True, text=True, timeout=60)
