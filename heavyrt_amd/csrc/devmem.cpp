@@ -111,7 +111,7 @@ bool DevCache::note(void* p, size_t size) {
 void* DevCache::take(IdleMap::iterator it) {
   void* p = it->second.p;
   idle_bytes_ -= it->first;
-  oldest_.erase(it->second.since);
+  oldest_.erase(it->second.order);
   idle_.erase(it);
   return p;
 }
@@ -125,20 +125,18 @@ void DevCache::free(void* p) {
     if (it == live_.end()) return;
     size = it->second;
     live_.erase(it);
+    given_back_ += size;
   }
-  // The oldest idle blocks make room: a program whose sizes have changed finds
-  // its new ones.  One at a time, as hipFree waits and must not hold the lock.
+  // One block at a time: hipFree waits and must not hold the lock.
   while (size <= kMaxIdle) {
     void* old = nullptr;
     {
       std::lock_guard<std::mutex> lock(mu_);
-      if (idle_bytes_ + size > kMaxIdle) {
-        old = take(oldest_.begin()->second);
-      } else {
+      if (idle_bytes_ + size <= kMaxIdle) {
         auto it = idle_.end();
         try {
-          it = idle_.emplace(size, Idle{p, clock_});
-          oldest_.emplace(clock_++, it);
+          it = idle_.emplace(size, Idle{p, ++order_, given_back_});
+          oldest_.emplace(order_, it);
         } catch (const std::bad_alloc&) {  // no host memory: given back below
           if (it != idle_.end()) idle_.erase(it);
           break;
@@ -146,6 +144,9 @@ void DevCache::free(void* p) {
         idle_bytes_ += size;
         return;
       }
+      const auto it = oldest_.begin()->second;
+      if (given_back_ - it->second.since <= kStale) break;
+      old = take(it);
     }
     (void)hipFree(old);
   }
