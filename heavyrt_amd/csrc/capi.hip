@@ -553,8 +553,8 @@ hrt_status hrt_update_triangles(hrt_scene* s, uint32_t geomId, const float* vpos
       for (uint32_t x : old)
         if (x >= nVert) return fail(HRT_ERR_INVALID_ARG, "kept indices reach past the new vertex count");
     }
-    b.nverts = uint32_t(nVert);
     e = upload_vertices(s->ctx, vpos, nVert, vStrideBytes, b.verts, &raw);
+    if (e == hipSuccess) b.nverts = uint32_t(nVert);  // (without memory for the upload the geometry stays as it is)
     if (e == hipSuccess && idx) e = hipMemcpyAsync(b.idx, idx, 12 * ntris, hipMemcpyHostToDevice, hs);
     if (e == hipSuccess) e = hrt::blas_refit(b, hs);
     if (e != hipSuccess) (void)hipStreamSynchronize(hs);

@@ -128,6 +128,30 @@ def smaller_launches():
     ctx.close()
 
 
+def refused_refit():
+    """A refit that could not upload its vertices leaves the geometry as it was, its vertex count too."""
+    ctx = H.Context(0)
+    v, f = W.soup(200_000, stream=W.STREAM_TEST)
+    v = np.concatenate([v, v[:1]])  # a vertex that no triangle uses
+    rays = W.incoherent_rays(1000, stream=W.STREAM_TEST)
+    s = committed(ctx, v, f)
+    want = s.trace_nearest_host(rays)
+    other = H.Scene(ctx)
+    limited(0)
+    assert refused(lambda: other.add_triangles(*W.soup(500_000)))  # nothing is idle after that
+    limited(0)
+    assert refused(lambda: s.update_triangles(0, v[:-1], quality=3))
+    unlimited()
+    s.commit()
+    assert s.trace_nearest_host(rays).tobytes() == want.tobytes()
+    s.update_triangles(0, 2 * v, quality=3)
+    s.update_triangles(0, v, quality=3)
+    s.commit()
+    assert s.trace_nearest_host(rays).tobytes() == want.tobytes()
+    s.close()
+    ctx.close()
+
+
 if __name__ == "__main__":
     globals()[sys.argv[2]]()
     assert shim.shim_calls() > 0, "the engine's calls did not reach the shim"
