@@ -651,24 +651,23 @@ hrt_status hrt_commit(hrt_scene* s, int quality, int layout) {
       }
     }
   }
-  // nearest hits on the BVH2 trees walk two levels a fetch; the records are
-  // whole before this returns, as a trace may follow on any stream
-  if (!single || layout == HRT_LAYOUT_BVH2 || layout == HRT_LAYOUT_AUTO || layout == HRT_LAYOUT_AUTO_FP16) {
-    bool made = false;
-    for (const Instance& in : s->instances) {
-      hrt::Blas& b = s->geoms[in.geom];
-      made |= !b.wide_made;
-      if ((e = hrt::blas_build_wide(b, s->ctx->stream)) != hipSuccess) return fail_hip(e, "nearest-hit nodes");
-    }
-    if (made && (e = hipStreamSynchronize(s->ctx->stream)) != hipSuccess) return fail_hip(e, "nearest-hit nodes");
+  // Small launches of nearest hits on a single BVH2 walk two levels a fetch
+  // (instanced scenes and BVH4 layouts never do).  All records are whole before
+  // this returns, as a trace may follow on any stream.
+  bool made = false;
+  if (single && (layout == HRT_LAYOUT_BVH2 || layout == HRT_LAYOUT_AUTO || layout == HRT_LAYOUT_AUTO_FP16)) {
+    hrt::Blas& b = s->geoms[s->instances[0].geom];
+    made = !b.wide_made;
+    if ((e = hrt::blas_build_wide(b, s->ctx->stream)) != hipSuccess) return fail_hip(e, "nearest-hit nodes");
   }
   if (wt) {
     hrt::Blas& b = s->geoms[s->instances[0].geom];
+    made = true;
     if ((e = hrt::blas_build_wt_tris(b, s->ctx->stream)) != hipSuccess ||
-        (b.any_tree && (e = hrt::blas_build_wt_tris(*b.any_tree, s->ctx->stream)) != hipSuccess) ||
-        (e = hipStreamSynchronize(s->ctx->stream)) != hipSuccess)
+        (b.any_tree && (e = hrt::blas_build_wt_tris(*b.any_tree, s->ctx->stream)) != hipSuccess))
       return fail_hip(e, "watertight triangle records");
   }
+  if (made && (e = hipStreamSynchronize(s->ctx->stream)) != hipSuccess) return fail_hip(e, "commit");
   s->layout = layout;
   s->committed_tri_test = s->tri_test;
   s->committed = true;

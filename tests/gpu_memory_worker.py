@@ -152,6 +152,41 @@ def refused_refit():
     ctx.close()
 
 
+def wide_nodes():
+    """The nodes of two levels are made for the scenes that walk them, by the commit, and again after a refit."""
+    ctx = H.Context(0)
+    v, f = W.soup(50_000, stream=W.STREAM_TEST)
+    rays = W.incoherent_rays(1000, stream=W.STREAM_TEST)
+
+    def made():
+        return len([k for k in kernels() if "k_wide_nodes" in k])
+
+    s = H.Scene(ctx)
+    g = s.add_triangles(v, f)
+    for k in range(2):
+        s.add_instance(g, np.array([1, 0, 0, 0, 0, 1, 0, 0, 0, 0, 1, 0, 2 * k, 0, 0, 1], np.float32))
+    kernels()
+    s.commit()
+    two = s.trace_nearest_host(rays)
+    s.update_triangles(g, v, quality=3)
+    s.commit()
+    assert made() == 0, "an instanced scene"
+    assert s.trace_nearest_host(rays).tobytes() == two.tobytes()
+    for layout, n in ((H.LAYOUT_BVH4, 0), (H.LAYOUT_BVH2, 1), (H.LAYOUT_AUTO, 1), (H.LAYOUT_PLOC, 0)):
+        s.clear_instances()
+        s.add_instance(g)
+        s.update_triangles(g, 2 * v, quality=3)
+        s.update_triangles(g, v, quality=3)
+        assert made() == 0, "a refit"
+        s.commit(layout=layout)
+        s.commit(layout=layout)
+        assert made() == n, layout
+        assert s.trace_nearest_host(rays).shape == (1000, 8)
+        assert len([k for k in kernels() if "k_trace_quad" in k]) == n
+    s.close()
+    ctx.close()
+
+
 if __name__ == "__main__":
     globals()[sys.argv[2]]()
     assert shim.shim_calls() > 0, "the engine's calls did not reach the shim"
