@@ -651,14 +651,17 @@ hrt_status hrt_commit(hrt_scene* s, int quality, int layout) {
       }
     }
   }
-  // Small launches of nearest hits on a single BVH2 walk two levels a fetch
-  // (instanced scenes and BVH4 layouts never do).  All records are whole before
-  // this returns, as a trace may follow on any stream.
+  // Small launches of nearest hits on a single BVH2 walk two levels a fetch;
+  // instanced scenes and BVH4 layouts never do, and their refits need not keep
+  // the records up.  All records are whole before this returns, as a trace may
+  // follow on any stream.
   bool made = false;
   if (single && (layout == HRT_LAYOUT_BVH2 || layout == HRT_LAYOUT_AUTO || layout == HRT_LAYOUT_AUTO_FP16)) {
     hrt::Blas& b = s->geoms[s->instances[0].geom];
     made = !b.wide_made;
     if ((e = hrt::blas_build_wide(b, s->ctx->stream)) != hipSuccess) return fail_hip(e, "nearest-hit nodes");
+  } else {
+    for (const Instance& in : s->instances) s->geoms[in.geom].wide_made = false;
   }
   if (wt) {
     hrt::Blas& b = s->geoms[s->instances[0].geom];

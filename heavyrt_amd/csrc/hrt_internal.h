@@ -109,7 +109,7 @@ struct Blas {
   // blas_build_wide); the word after the last node is not zero where a walk on
   // them could differ from one on the pairs
   WideNode* wide = nullptr;
-  bool wide_made = false;  // blas_build_wide has run on the tree as it is now
+  bool wide_made = false;  // they are the tree's as it is now, for a layout that walks them
   // parity hooks (kept only when requested)
   uint32_t* codes_in = nullptr;    // Morton code per input triangle
   uint32_t* codes_sorted = nullptr;
@@ -173,8 +173,8 @@ inline WalkNodes walk_nodes(const Blas& b) {
   const WideNode* w = b.wide_made ? b.wide : nullptr;
   return WalkNodes{w, b.pairs, w ? reinterpret_cast<const uint32_t*>(w + internal_nodes(b)) : nullptr};
 }
-// Makes b.wide from the node pairs (idempotent; after a refit again, in the
-// same memory).  Without memory for it b.wide stays null, which is no error.
+// Makes b.wide from the node pairs (idempotent; in the same memory again after
+// a refit or another layout).  Without memory for it b.wide stays null, which is no error.
 // Asynchronous on `stream`.
 hipError_t blas_build_wide(Blas& b, hipStream_t stream);
 // Leaf-order triangles with absolute vertices for the watertight test

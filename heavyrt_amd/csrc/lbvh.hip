@@ -815,7 +815,10 @@ hipError_t blas_refit(Blas& b, hipStream_t s) {
                                                        b.parent_leaf, b.tris, nullptr);
   hipError_t err = refit_boxes(b.meta, N, b.pairs, b.parent, b.parent_leaf, b.node_range, tops, arrive + N, arrive,
                                b.meta + 3, s);
-  b.wide_made = false;  // remade in the same memory by the next commit that needs them
+  // (here, where the stream is waited for anyway: 12 us less than in the commit)
+  const bool walked = b.wide_made;
+  b.wide_made = false;
+  if (err == hipSuccess && walked) err = blas_build_wide(b, s);
   if (err == hipSuccess) err = back.read(0, b.meta, 4, s);
   if (err == hipSuccess) err = back.read(8, box, 8, s);
   const hipError_t werr = hipStreamSynchronize(s);

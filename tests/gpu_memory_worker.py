@@ -153,36 +153,44 @@ def refused_refit():
 
 
 def wide_nodes():
-    """The nodes of two levels are made for the scenes that walk them, by the commit, and again after a refit."""
+    """The nodes of two levels are made for the scenes that walk them, by the commit and then by each refit."""
     ctx = H.Context(0)
     v, f = W.soup(50_000, stream=W.STREAM_TEST)
     rays = W.incoherent_rays(1000, stream=W.STREAM_TEST)
+    s = H.Scene(ctx)
+    g = s.add_triangles(v, f)
+
+    def instanced():
+        s.clear_instances()
+        for k in range(2):
+            s.add_instance(g, np.array([1, 0, 0, 0, 0, 1, 0, 0, 0, 0, 1, 0, 2 * k, 0, 0, 1], np.float32))
+        return H.LAYOUT_BVH2
+
+    def alone(layout):
+        s.clear_instances()
+        s.add_instance(g)
+        return layout
 
     def made():
         return len([k for k in kernels() if "k_wide_nodes" in k])
 
-    s = H.Scene(ctx)
-    g = s.add_triangles(v, f)
-    for k in range(2):
-        s.add_instance(g, np.array([1, 0, 0, 0, 0, 1, 0, 0, 0, 0, 1, 0, 2 * k, 0, 0, 1], np.float32))
+    want = {}
+    walked = False  # by the layout committed last
     kernels()
-    s.commit()
-    two = s.trace_nearest_host(rays)
-    s.update_triangles(g, v, quality=3)
-    s.commit()
-    assert made() == 0, "an instanced scene"
-    assert s.trace_nearest_host(rays).tobytes() == two.tobytes()
-    for layout, n in ((H.LAYOUT_BVH4, 0), (H.LAYOUT_BVH2, 1), (H.LAYOUT_AUTO, 1), (H.LAYOUT_PLOC, 0)):
-        s.clear_instances()
-        s.add_instance(g)
+    for name in ("two", "bvh2", "two", "bvh4", "auto", "auto", "ploc", "bvh2"):
+        layout = instanced() if name == "two" else alone(getattr(H, "LAYOUT_" + name.upper()))
         s.update_triangles(g, 2 * v, quality=3)
         s.update_triangles(g, v, quality=3)
-        assert made() == 0, "a refit"
+        assert made() == (2 if walked else 0), f"refits before {name}"
         s.commit(layout=layout)
         s.commit(layout=layout)
-        assert made() == n, layout
-        assert s.trace_nearest_host(rays).shape == (1000, 8)
-        assert len([k for k in kernels() if "k_trace_quad" in k]) == n
+        walks = name in ("bvh2", "auto")
+        assert made() == (1 if walks and not walked else 0), f"commit of {name}"
+        walked = walks
+        hits = s.trace_nearest_host(rays)
+        assert len([k for k in kernels() if "k_trace_quad" in k]) == int(walks), name
+        assert hits.tobytes() == want.setdefault(name, hits).tobytes()
+        assert name == "two" or hits[:, 0].tobytes() == want.setdefault("t", hits[:, 0]).tobytes()
     s.close()
     ctx.close()
 
