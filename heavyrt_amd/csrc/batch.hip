@@ -918,7 +918,8 @@ constexpr int kNumCandidates = int(sizeof(kCandidates) / sizeof(kCandidates[0]))
 constexpr int kDefaultCandidate = 1;
 constexpr int kLaneCandidate = 11, kStreamCandidate = 14;
 
-// The candidate of a batch for which none was set or tuned: one ray per lane,
+// The candidate of a batch for which none was chosen and that is not traced by
+// k_b_trace_quad (enqueue_trace): one ray per lane,
 // unless many rays walk large trees, where a wave that waits for its longest
 // ray loses more than refilling costs.  us, with candidates 1 (all of them
 // before), 11 and 14: 64 scenes of 1,000 triangles and 1 M rays 443 171 406,
@@ -978,7 +979,7 @@ struct hrt_batch {
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
   int candidate = hrt::kDefaultCandidate;
-  bool chosen = false;  // the candidate was set or tuned
+  bool chosen = false;  // the candidate runs: it was set, or tuned and faster than the default
   std::vector<uint32_t> grid;  // per candidate, fixed at creation (no queries during capture)
   std::vector<float> tuning_ms;
   bool built = false;
@@ -1084,13 +1085,17 @@ hipError_t enqueue_candidate(hrt_batch* b, int cand, hipStream_t s) {
   return hipLaunchKernel(c.fn, dim3(b->grid[cand]), dim3(threads), args, 0, s);
 }
 
-hipError_t enqueue_trace(hrt_batch* b, hipStream_t s) {
+// The trace of a batch for which no candidate was chosen.
+hipError_t enqueue_default(hrt_batch* b, hipStream_t s) {
   using namespace hrt;
-  if (!b->quads)
-    return enqueue_candidate(b, b->chosen ? b->candidate : candidate_for(b->R, b->small != 0), s);
+  if (!b->quads) return enqueue_candidate(b, candidate_for(b->R, b->small != 0), s);
   k_b_trace_quad<<<uint32_t((b->R + kQuadRaysB - 1) / kQuadRaysB), 256, 0, s>>>(
       b->pairs, b->wide, b->differ, b->tris, offsets(b), b->rays, uint32_t(b->R), b->hits);
   return hipGetLastError();
+}
+
+hipError_t enqueue_trace(hrt_batch* b, hipStream_t s) {
+  return b->chosen ? enqueue_candidate(b, b->candidate, s) : enqueue_default(b, s);
 }
 
 // Workgroups per candidate: one ray per lane for the simple kernels; for the
@@ -1110,6 +1115,12 @@ void plan_grids(hrt_batch* b) {
     if (c.lds < kStackDepth) g = std::min<uint64_t>(g, b->spill_words / (threads * uint64_t(kStackDepth - c.lds)));
     b->grid[k] = uint32_t(std::max<uint64_t>(1, g));
   }
+}
+
+void choose(hrt_batch* b, int candidate, bool runs) {
+  if (runs != b->chosen || (runs && candidate != b->candidate)) drop_graph(b);
+  b->candidate = candidate;
+  b->chosen = runs;
 }
 
 hrt_status capture_graph(hrt_batch* b) {
@@ -1352,11 +1363,7 @@ hrt_status hrt_batch_candidate_info(int i, int* wavesPerGroup, int* ldsStackEntr
 hrt_status hrt_batch_set_candidate(hrt_batch* b, int i) {
   if (!b) return fail(HRT_ERR_INVALID_ARG, "batch is null");
   if (i < 0 || i >= hrt::kNumCandidates) return fail(HRT_ERR_INVALID_ARG, "no such candidate");
-  if (i != b->candidate || !b->chosen) {
-    b->candidate = i;
-    b->chosen = true;
-    drop_graph(b);
-  }
+  choose(b, i, true);
   return HRT_OK;
 }
 
@@ -1375,33 +1382,39 @@ hrt_status hrt_batch_autotune(hrt_batch* b, int reps, int* chosen, float* msPerC
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   if (e == hipSuccess) e = hipEventCreate(&ev0);
   if (e == hipSuccess) e = hipEventCreate(&ev1);
-  int best = b->candidate;
-  float best_ms = 0.0f;
-  b->tuning_ms.assign(hrt::kNumCandidates, 0.0f);
-  for (int c = 0; c < hrt::kNumCandidates && e == hipSuccess; c++) {
-    e = enqueue_candidate(b, c, s);  // warm-up
+  auto least_ms = [&](auto&& enqueue) {
+    e = enqueue();  // warm-up
     float ms_min = 0.0f;
     for (int r = 0; r < reps && e == hipSuccess; r++) {
       e = hipEventRecord(ev0, s);
-      if (e == hipSuccess) e = enqueue_candidate(b, c, s);
+      if (e == hipSuccess) e = enqueue();
       if (e == hipSuccess) e = hipEventRecord(ev1, s);
       if (e == hipSuccess) e = hipEventSynchronize(ev1);
       float ms = 0.0f;
       if (e == hipSuccess) e = hipEventElapsedTime(&ms, ev0, ev1);
       if (r == 0 || ms < ms_min) ms_min = ms;
     }
-    b->tuning_ms[c] = ms_min;
-    if (msPerCandidate) msPerCandidate[c] = ms_min;
-    if (c == 0 || ms_min < best_ms) {
-      best_ms = ms_min;
+    return ms_min;
+  };
+  int best = b->candidate;
+  float best_ms = 0.0f;
+  b->tuning_ms.assign(hrt::kNumCandidates, 0.0f);
+  for (int c = 0; c < hrt::kNumCandidates && e == hipSuccess; c++) {
+    const float ms = least_ms([&] { return enqueue_candidate(b, c, s); });
+    b->tuning_ms[c] = ms;
+    if (msPerCandidate) msPerCandidate[c] = ms;
+    if (c == 0 || ms < best_ms) {
+      best_ms = ms;
       best = c;
     }
   }
+  // a batch whose default is no candidate keeps it where it is faster than all of them
+  bool keep_default = false;
+  if (e == hipSuccess && b->quads) keep_default = least_ms([&] { return enqueue_default(b, s); }) <= best_ms;
   if (ev0) (void)hipEventDestroy(ev0);
   if (ev1) (void)hipEventDestroy(ev1);
   if (e != hipSuccess) return fail_hip(e, "autotune");
-  hrt_status st = hrt_batch_set_candidate(b, best);
-  if (st != HRT_OK) return st;
+  choose(b, best, !keep_default);
   if (chosen) *chosen = best;
   return HRT_OK;
 }

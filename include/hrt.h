@@ -362,16 +362,21 @@ hrt_status hrt_batch_build(hrt_batch* batch, void* stream);
 hrt_status hrt_batch_trace(hrt_batch* batch, void* stream);
 /* Trace-kernel candidates: waves per workgroup, LDS stack entries per lane
  * (0 = one ray per lane without refill), the refill threshold (idle lanes)
- * and the number of ray indices a wave claims from the queue at once.  A batch
- * of at most 65,536 rays over scenes of at most 4,096 triangles is traced by a
- * kernel of its own, whatever candidate is set. */
+ * and the number of ray indices a wave claims from the queue at once.  The
+ * candidate that was set runs.  Until one is set or tuned, the default runs: a
+ * kernel that gives a ray four lanes, and is no candidate, for a batch of at
+ * most 65,536 rays over scenes of at most 4,096 triangles, else a candidate by
+ * the numbers of rays and triangles. */
 int hrt_batch_candidate_count(void);
 hrt_status hrt_batch_candidate_info(int i, int* wavesPerGroup, int* ldsStackEntries, int* refillAt, int* claim);
 hrt_status hrt_batch_set_candidate(hrt_batch* batch, int i);
+/* The candidate set last or found fastest by hrt_batch_autotune; 1 before
+ * either, whatever the default runs. */
 int hrt_batch_get_candidate(const hrt_batch* batch);
 /* Builds if needed, times every candidate `reps` times on the batch's own
- * rays (best of reps), selects the fastest; msPerCandidate (nullable) gets
- * hrt_batch_candidate_count() timings.  Synchronous. */
+ * rays (best of reps) and selects the fastest, which runs from then on unless
+ * the default is the four-lane kernel and no slower; msPerCandidate (nullable)
+ * gets hrt_batch_candidate_count() timings.  Synchronous. */
 hrt_status hrt_batch_autotune(hrt_batch* batch, int reps, int* chosen, float* msPerCandidate);
 /* Synchronous check of the last build: HRT_OK when every scene's tree was
  * stored; HRT_ERR_LEAF_OVERFLOW (with *badScene, nullable, the first such

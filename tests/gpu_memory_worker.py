@@ -195,6 +195,46 @@ def wide_nodes():
     ctx.close()
 
 
+def candidates():
+    """The candidate that was set runs, in plain launches and in the graph; an untuned or tuned batch may keep the
+    four-lane kernel."""
+    ctx = H.Context(0)
+    for sizes, rays in (([500, 3000], 700), ([500, 5000], 700)):
+        scenes = [(*W.soup(n, stream=2200 + n), W.incoherent_rays(rays, stream=3200 + n)) for n in sizes]
+        b = H.Batch(ctx, [x[0].shape[0] for x in scenes], [x[1].shape[0] for x in scenes], [rays] * len(sizes))
+        b.upload(scenes)
+        four = sizes[1] <= 4096
+
+        def trace(run):
+            kernels()
+            run()
+            hits = b.hits().tobytes()
+            return [k for k in kernels() if "k_b_trace" in k], hits
+
+        default, hits = trace(b.run)
+        assert len(default) == 1 and ("k_b_trace_quad" in default[0]) == four, default
+        for i, c in enumerate(H.batch_candidates()):
+            b.set_candidate(i)
+            assert b.candidate == i
+            for run in (b.run, b.trace):
+                names, h = trace(run)
+                assert len(names) == 1 and h == hits
+                want = f"k_b_trace_simpleILi{64 * c[0]}E" if c[1] == 0 else f"k_b_traceILi{c[0]}ELi{c[1]}ELi{c[2]}ELj{c[3]}E"
+                assert want in names[0], (want, names)
+            assert trace(b.run)[0] == [], "the graph is recorded once"
+        chosen, ms = b.autotune(2)
+        assert b.candidate == chosen == int(np.argmin(ms))
+        kept, h = trace(b.run)
+        assert len(kept) == 1 and h == hits
+        last = kept[0]
+        assert ("k_b_trace_quad" in last and four) or f"ELj{H.batch_candidates()[chosen][3]}E" in last or "simple" in last
+        b.set_candidate(chosen)
+        names, h = trace(b.trace)
+        assert "k_b_trace_quad" not in names[0] and h == hits
+        b.close()
+    ctx.close()
+
+
 if __name__ == "__main__":
     globals()[sys.argv[2]]()
     assert shim.shim_calls() > 0, "the engine's calls did not reach the shim"

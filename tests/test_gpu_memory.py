@@ -22,7 +22,7 @@ def shim(tmp_path_factory):
     return lib
 
 
-@pytest.mark.parametrize("scenario", ["idle_memory", "smaller_launches", "refused_refit", "wide_nodes"])
+@pytest.mark.parametrize("scenario", ["idle_memory", "smaller_launches", "refused_refit", "wide_nodes", "candidates"])
 def test_scenario(gpu_ctx, shim, scenario):
     say(f"memory: {scenario}")
     r = subprocess.run([sys.executable, WORKER, shim, scenario], capture_output=True, text=True, timeout=100)
