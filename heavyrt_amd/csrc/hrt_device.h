@@ -160,10 +160,12 @@ __device__ inline uint32_t lanes_below(uint64_t m) {
 // up to 70 us, and a claim a refill would limit the whole kernel.  A claim is
 // kClaim rays, twice that while very many are left and 64 at the end, so that
 // the waves end together.  us a call with a first claim from the queue and 128
-// rays always, and now: 2 M shadow rays 739 and 637, 600,000 501 and 393, two
-// levels with 192,000 rays 469 and 317, a 1024x1024 frame with 16 AO samples
-// 3,078 and 2,620 (there 128 rays always 3,042; for 4 M rays 256 are worse than
-// 128, 1,057 and 984).
+// rays always, and now: a 1024x1024 frame with 16 AO samples 2,349 and 2,029,
+// 2 M shadow rays 676 and 594, a served burst 2,622 and 2,458, 480,000 rays over
+// 2,000 moved instances 1,562 and 1,533.  The AO frame's gain is the larger
+// claims' (of 3,078 in one sweep: 3,042 with the first rays free and claims of
+// 128, 2,620 with up to 256), the shadow rays' the free first ones' (739: 658,
+// then 637 with 64 at the end, 696 with up to 256 whatever is left).
 // Every member is wave-uniform; take() must be called by all lanes of the
 // wave together.
 struct RayPool {

@@ -476,7 +476,7 @@ __global__ __launch_bounds__(kBlock) void k_even_depth(const uint32_t* __restric
   if (k == ninternal) flag[k] = 0u;
   if (k >= ninternal) return;
   uint32_t d = 0, p = k;
-  while (p != 0) {  // at most 30 steps: the tree has at most 30 internal levels
+  while (p != 0) {  // at most 30 steps on a Karras tree, kMaxLevels4 on a clustered one
     p = parent_int[p] >> 1;
     d++;
   }

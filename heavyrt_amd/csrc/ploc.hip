@@ -24,10 +24,11 @@
 // device-side record that the round before wrote.  Above kFinish clusters a
 // round is two launches (pick and merge); from there on one workgroup does all
 // remaining rounds with the clusters in LDS.  The host enqueues as many rounds
-// as a tree of this size usually needs and looks at the result once.  On the
-// 748,422 leaves of the 1.07 M-triangle scene (59 rounds) that took 1.6 ms of
-// kernels, 590 launches and 59 waits of the host with separate neighbour, flag,
-// scan and total passes, and 0.7 ms of kernels now.
+// as a tree of this size usually needs and looks at the result once.  The
+// 564,235 leaves of 1.07 M triangles of hills with boxes (59 rounds) took 1.7 ms
+// of kernels, about 480 launches and 59 waits of the host with separate
+// neighbour, flag, scan and total passes, and take 0.7 ms of kernels in 64
+// launches now: the rounds 0.49, the last 4,096 clusters 0.18.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -195,9 +196,12 @@ __global__ __launch_bounds__(kBlock) void k_ploc_pick(const Cluster* __restrict_
   }
 }
 
-// The second half: every tile adds up the totals of the tiles before it (a few
-// hundred on a million clusters, fewer each round), ranks its own clusters and
-// writes nodes and surviving clusters.  The last tile leaves the next round's
+// The second half: every tile adds up the totals of the tiles before it, ranks
+// its own clusters and writes nodes and surviving clusters.  The sums grow with
+// the square of the tiles (on a million clusters 3,907 tiles read 16 KB each on
+// average, from the L2), but stay the smaller part up to the largest tree: a
+// commit that clusters 16 M triangles takes 14 ms, 23 with scans of the flags
+// and the host between the rounds.  The last tile leaves the next round's
 // record; a round that has nothing to do hands its own on.
 __global__ __launch_bounds__(kBlock) void k_ploc_merge(Cluster* __restrict__ c0, Cluster* __restrict__ c1,
                                                        const PlocState* __restrict__ st, uint32_t stop,
@@ -371,10 +375,9 @@ hipError_t blas_ploc(Blas& b, hipStream_t s, bool* replaced) {
   const uint32_t L = b.leaves;
   if (L < 3) return hipSuccess;  // one or two leaves: nothing to cluster
   // Rounds to enqueue before the host looks: a round leaves 75 to 87 % of the
-  // clusters (562,428 leaves of hills with boxes are down to kFinish after 26
-  // rounds, 4,177,918 of a soup after 40), and one without work costs about 4
-  // us.  The hierarchy over those 562,428 leaves took 4.1 ms with the host
-  // reading every round's totals, 1.0 ms this way.
+  // clusters (562,428 leaves of such hills are down to kFinish after 26 rounds,
+  // 4,177,918 of a soup after 40), and one without work costs about 4 us.  With
+  // its waits the hierarchy took 4.1 ms on them, 1.0 ms this way.
   uint32_t rounds = 0;
   for (double n = L; n > double(kFinish); n *= 0.85) rounds++;
   // device scratch: two cluster arrays, a byte per cluster, totals per tile,

@@ -164,9 +164,10 @@ struct SmallLds {
 // child is node r, a right child node l, the root node 0.  A box waits at its
 // node's own number: internal node m covers leaf m, whose box has been read by
 // then.  While more nodes climb than there are threads, each takes one step
-// and the formed ones are gathered (at most half remain); a thread that climbs
-// with several leaves one after the other takes as many whole climbs (49 us
-// instead of 33 on 4,096 triangles).
+// and the formed ones are gathered: at most half as many as leaves after the
+// first step, and no more after a later one (a node is formed by an arrival), so
+// they fit `nodes`.  A thread that climbs with several leaves one after the
+// other takes as many whole climbs (49 us instead of 33 on 4,096 triangles).
 template <class Src, uint32_t kThreads, uint32_t kItems>
 __device__ inline void small_build(const Src& src, uint32_t n, int cubic, const SmallTree& out,
                                    SmallLds<kThreads, kItems>& s) {

@@ -13,9 +13,10 @@
 // nodes are the even-depth nodes of a BVH2 with at most 30 internal levels:
 // 15 node levels, 3 deferred children each) and at most kStackDepth4 = 63 on
 // the clustered second tree, whose build keeps it within 42 levels.  The
-// persistent kernels keep 16 entries per lane in LDS and the one-ray-per-lane
-// kernel 48, interleaved by lane; deeper entries go to a per-lane global
-// spill area, so LDS does not limit occupancy.
+// persistent kernels keep 16 entries per lane in LDS, the one-ray-per-lane
+// kernels 24 (48 in the counting variant), interleaved by lane; deeper entries
+// go to a per-lane global spill area.  The four-lane kernels keep all of a
+// ray's in LDS.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
