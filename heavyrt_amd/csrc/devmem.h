@@ -17,14 +17,17 @@ namespace hrt {
 // a build has a dozen arrays: a million triangles loaded and committed took
 // 10.3 ms, and 2.8 with this and the geometry expanded on the device), and
 // pinned words for small readbacks (12 us with the wait, 21 us through pageable
-// memory).  At most kMaxIdle bytes are kept idle, for blocks of up to a quarter
-// less; a block that was not taken again while kStale bytes came back makes
-// room for new ones, so that a program whose sizes change finds its memory.
-// (Making room for every block costs a program that needs more than kMaxIdle
-// again and again: 16 M triangles loaded and closed 49.5 ms instead of 47.4.)
-// They go back to the device when any allocation of the engine on it
-// fails (here, device_malloc, stream_malloc), whichever context kept them, and
-// at the end.  Safe with several threads.
+// memory).  Safe with several threads.
+//
+// At most kMaxIdle bytes are kept idle, for blocks of up to a quarter less.
+// They go back to the device when any allocation of the engine on it fails
+// (here, device_malloc, stream_malloc), whichever context kept them, and at the
+// end.  On a full list a block that was not taken again while kStale bytes came
+// back makes room, so that a program whose sizes change finds its memory:
+// scenes of 1 M triangles after some of 4 M are loaded in 3.7 ms and closed in
+// none, with a list that keeps what it has in 4.3 and 2.2 for good.  Making room
+// for every block would cost a program that needs more than kMaxIdle again and
+// again: 16 M triangles loaded and closed 49.5 ms instead of 47.4.
 class DevCache {
  public:
   explicit DevCache(int device);  // may throw std::bad_alloc
